@@ -54,4 +54,24 @@ bool mx_linear_planes_ok(int64_t lda, int64_t kb);
 hipError_t mx_linear_planes_unit(const uint16_t* a, int64_t lda, const uint8_t* wq, float* c, int64_t ldc,
                                  int64_t plane, int m, int n, int k, int kb, int slices, hipStream_t st);
 hipError_t split3_rows(const float* a, int64_t lda, int64_t m, int64_t k, uint16_t* out, hipStream_t st);
+
+// The linear for few activation rows (kq_skinny.hip): one pass over the
+// weights, K split over the waves of a workgroup, no workspace.  a: bf16 or
+// fp32 rows (row stride lda elements), or E4M3 bytes (lda bytes) with E8M0
+// scales [m, k / 32]; weights and scales as kq_mx_linear takes them (k % 64
+// == 0 with 2-byte aligned scales; k % 128 == 0 needs 4-byte aligned ones,
+// as do MXFP8 rows; a and wq 16-byte aligned, lda a multiple of 16 bytes).
+struct SkinnyArgs {
+  const void* a;
+  const uint8_t* a_scale;
+  int64_t lda;
+  const uint8_t* wq;
+  const uint8_t* ws;
+  void* c;
+  int64_t ldc;
+  int m, n, k;
+};
+hipError_t mx_skinny_bf16(int fmt, bool out_f32, const SkinnyArgs& args, hipStream_t st);
+hipError_t mx_skinny_f32(int fmt, const SkinnyArgs& args, hipStream_t st);
+hipError_t mx_skinny_mx(bool out_f32, const SkinnyArgs& args, hipStream_t st);
 }  // namespace kq

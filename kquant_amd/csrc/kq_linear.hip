@@ -926,6 +926,14 @@ hipError_t split3_rows(const float* a, int64_t lda, int64_t m, int64_t k, uint16
 
 }  // namespace kq
 
+// Rows up to which the one-pass kernel of kq_skinny.hip takes the linear: a
+// 256 x 256 tile costs the same for 1 row as for 256 (N = 12288, K = 7168
+// E4M3: 137 us), the one-pass kernel 24 us at 1 row and 57 us at 64.
+constexpr int64_t SKINNY_MAX_ROWS = 64;
+static bool takes_skinny(int64_t m, int64_t k, const uint8_t* w_scale) {
+  return m <= SKINNY_MAX_ROWS && (k % 128 != 0 || !kq_misaligned(w_scale, 4));
+}
+
 extern "C" int kq_mx_linear(int w_fmt, const void* a, int64_t lda, const void* w_q,
                             const uint8_t* w_scale, int64_t m, int64_t n, int64_t k,
                             int out_dtype, void* c, int64_t ldc, void* stream) {
@@ -947,6 +955,10 @@ extern "C" int kq_mx_linear(int w_fmt, const void* a, int64_t lda, const void* w
   const uint16_t* ap = (const uint16_t*)a;
   const uint8_t* wp = (const uint8_t*)w_q;
   hipError_t e;
+  if (takes_skinny(m, k, w_scale))
+    return kq_check_launch(mx_skinny_bf16(w_fmt, out_dtype == KQ_DT_F32,
+                                          {a, nullptr, lda, wp, w_scale, c, ldc, (int)m, (int)n, (int)k}, st),
+                           "kq_mx_linear");
   if (w_fmt == KQ_FMT_MXFP8_E4M3)
     e = out_dtype == KQ_DT_BF16 ? launch_linear<0, 0>(ap, lda, wp, w_scale, c, ldc, (int)m, (int)n, (int)k, (int)k, st)
                                 : launch_linear<0, 2>(ap, lda, wp, w_scale, c, ldc, (int)m, (int)n, (int)k, (int)k, st);
@@ -982,6 +994,10 @@ extern "C" int kq_mx_linear_f32(int w_fmt, const float* a, int64_t lda, const vo
     return kq_fail(KQ_ERR_INVALID, "kq_mx_linear_f32: a, w_q and workspace must be 16-byte aligned");
   if (m == 0 || n == 0) return KQ_OK;
   hipStream_t st = (hipStream_t)stream;
+  if (takes_skinny(m, k, w_scale))
+    return kq_check_launch(mx_skinny_f32(w_fmt, {a, nullptr, lda, (const uint8_t*)w_q, w_scale, c, ldc, (int)m, (int)n,
+                                                 (int)k}, st),
+                           "kq_mx_linear_f32");
   uint16_t* a3 = static_cast<uint16_t*>(workspace);
   const int64_t quads = m * (k / 4);
   split3_bf16_kernel<<<(unsigned)((quads + 255) / 256), 256, 0, st>>>(a, lda, m, k, a3);
@@ -1033,6 +1049,10 @@ extern "C" int kq_mx_linear_mx(int a_fmt, const void* a_q, const uint8_t* a_scal
   hipStream_t st = (hipStream_t)stream;
   const uint8_t* ap = (const uint8_t*)a_q;
   const uint8_t* wp = (const uint8_t*)w_q;
+  if (m <= SKINNY_MAX_ROWS)
+    return kq_check_launch(mx_skinny_mx(out_dtype == KQ_DT_F32,
+                                        {a_q, a_scale, lda, wp, w_scale, c, ldc, (int)m, (int)n, (int)k}, st),
+                           fn);
   const hipError_t e =
       out_dtype == KQ_DT_BF16
           ? launch_linear_a8<0>(ap, a_scale, lda, wp, w_scale, c, ldc, (int)m, (int)n, (int)k, workspace, st)

@@ -225,3 +225,53 @@ def test_linear_a8_pads_k(gpu):
     ref, _, _ = _a8_oracle(x, q, s)
     c = linear.mxfp8_linear_mm(x.to(gpu), q, s, out_dtype=torch.float32).cpu().numpy()
     assert _max_rel(ref, c) <= TOL and _rel_l2(ref, c) <= A8_NORM_TOL
+
+
+@pytest.mark.parametrize("m", [1, 15, 17, 32, 33, 64])
+@pytest.mark.parametrize("n,k", [(1, 64), (33, 128), (250, 192), (8200, 1088), (8205, 1152)])
+@pytest.mark.parametrize("form", ["bf16-mxfp8", "bf16-mxfp4", "f32-mxfp8", "f32-mxfp4", "mx-mxfp8"])
+def test_few_rows(gpu, form, m, n, k):
+    """The one-pass kernel of few-row batches: both ends of each row-block
+    class, one row and ragged columns, half windows (k % 128 == 64), fewer
+    windows than waves and both workgroup widths (n from 8192 takes four
+    weight row blocks).  fp32 output, so the bound is that of fp32 sums over
+    k <= 1152 exact products (2^-24 sqrt(k) ~ 2e-6)."""
+    dtype, fmt = form.split("-")
+    if dtype == "mx" and k % 128:
+        pytest.skip("MXFP8 rows take whole 128-k windows")
+    g = torch.Generator().manual_seed(m * 31 + n + k)
+    w = (torch.randn(n, k, generator=g) * 0.02).to(torch.bfloat16).to(gpu)
+    x = torch.randn(m, k, generator=g) * torch.exp(0.5 * torch.randn(k, generator=g))
+    x = x if dtype == "f32" else x.to(torch.bfloat16)
+    q, s, wd = _quantized(fmt, w)
+    if dtype == "mx":
+        xq, xs = mxfp8.mxfp8_quantize(x.to(gpu))
+        c = linear.mxfp8_linear_mx(xq, xs, q, s, out_dtype=torch.float32)
+        xv = oracle.mx_dequant("mxfp8", xq.view(torch.uint8).cpu().numpy(), xs.cpu().numpy()).astype(np.float64)
+    else:
+        fn = linear.mxfp8_linear if fmt == "mxfp8" else linear.mxfp4_linear
+        c = fn(x.to(gpu), q, s, out_dtype=torch.float32)
+        xv = x.double().numpy()
+    ref = xv @ wd.astype(np.float64).T
+    assert _max_rel(ref, c.cpu().numpy()) <= 1e-5
+
+
+@pytest.mark.parametrize("a_byte,w_byte", [(7, 237), (100, 247), (3, 3 + 240), (240, 9)])
+def test_few_rows_extreme_scales(gpu, a_byte, w_byte):
+    """MXFP8 x MXFP8 scale bytes whose products with E4M3 leave the normal
+    bf16 range (2^-120 activations against 2^110 weights) multiply in fp32:
+    fp32 sums of 512 exact products of one sign, at most 512 x 2^-24 = 3e-5."""
+    g = torch.Generator().manual_seed(5)
+    m, n, k = 3, 40, 512
+    aq = torch.randint(0, 120, (m, k), generator=g, dtype=torch.uint8)
+    wq = torch.randint(0, 120, (n, k), generator=g, dtype=torch.uint8)
+    a_s = torch.full((m, k // 32), a_byte, dtype=torch.uint8)
+    w_s = torch.full((n, k // 32), w_byte, dtype=torch.uint8)
+    c = linear.mxfp8_linear_mx(aq.to(gpu).view(torch.float8_e4m3fn), a_s.to(gpu), wq.to(gpu), w_s.to(gpu),
+                               out_dtype=torch.float32)
+
+    def values(q, s):
+        v = q.view(torch.float8_e4m3fn).double().reshape(q.shape[0], -1, 32)
+        return (v * torch.exp2(s.double() - 127)[..., None]).reshape(q.shape).numpy()
+
+    assert _max_rel(values(aq, a_s) @ values(wq, w_s).T, c.cpu().numpy()) <= 3e-5
