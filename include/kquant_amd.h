@@ -548,7 +548,7 @@ int kq_qsrt_moe_decode(int act, float beta, float linear_beta, const void* x, in
  * fp32 [n_tiles, 256]; out_states int16 [n_tiles, 256] (the cyclic 16-bit
  * states of the path); lut: 65536 E4M3 labels in state order (device);
  * tailbite_context 1..128.  One workgroup per tile, `workgroups` of them
- * over the tiles; workspace: kq_sqg_quantize_workspace_size(bits,
+ * over the tiles (two per CU run side by side); workspace: kq_sqg_quantize_workspace_size(bits,
  * workgroups) bytes for the decisions.  Tiles whose every path cost
  * overflows fp16 (|x| in the hundreds) are outside the reference's domain. */
 int64_t kq_sqg_quantize_workspace_size(int bits, int workgroups);

@@ -17,13 +17,28 @@
 // argmin breaks ties as the reference's shuffle-down reductions do: smallest
 // (bitrev5(e % 1024 / 32), bitrev5(e % 32), e / 1024).
 //
-// MI355X mapping: one 1024-thread workgroup per tile (persistent over the
-// tiles), the label table staged once per workgroup into LDS transposed to
-// [node pair][predecessor][2] so a thread's labels of all predecessors of a
-// node pair are one 8/16/32-byte read, both cost buffers in LDS, and each
-// thread evaluating node pairs with packed fp16 arithmetic.  The decisions
-// (K bits per node and step, packed as the reference packs them) go to a
-// per-workgroup global workspace for the traceback.
+// MI355X mapping: one workgroup per tile, persistent over the tiles.  What
+// bounds the search is VALU: 2^16 edge evaluations per step and tile.
+//  * Thread t owns NPT = 2^(16-K) / T consecutive nodes, so the 2^16 / T
+//    labels it ever needs stay in its registers as packed fp16 (32 with 1,024
+//    threads, 64 with 512): no label table in LDS and no E4M3 conversion per
+//    edge, and its nodes share their predecessors (NPT / 2^K of them per k,
+//    one LDS read each), whose costs both LDS buffers hold.
+//  * The 2^K edge pairs of two nodes take a packed difference and fma each,
+//    then a tournament of packed minima and differences whose sign bits are
+//    the comparisons (costs are never negative, so their bits order as their
+//    values do): the index of the winner is picked out of the sign bits at
+//    the end.  (32-bit keys cost << 16 | k and min3: 1.33 ms at 448 tiles
+//    against 1.25.)  Steps whose decisions are not kept (the primer's first half)
+//    take the minima alone.
+//  * The traceback is a chain of dependent reads of the decisions (K bits per
+//    node and step in a per-workgroup global workspace): a wave reads the decisions of all nodes that the next
+//    two to four steps can reach at once, so one memory latency covers them.
+//  * With more tiles than CUs, 512-thread workgroups, two per CU: one tile's
+//    traceback and barriers overlap the other's search.
+// K = 3, ctx 128: 448 tiles 3.80 -> 1.25 ms, 164 tiles 1.95 -> 0.68 ms against
+// labels looked up and converted per edge, one tile per CU and one thread's
+// traceback.
 //
 // The same search runs against the two procedural EXL3 control codebooks of
 // kquant/csrc/exl3_compat/quant/codebook.cuh (sqg_quantize.cu:261-330), whose
@@ -38,15 +53,17 @@
 // so each predecessor costs an add, as in qsrt_quantize_tiles_kernel.cuh:131-145.
 #include "kq_internal.h"
 
+#include <type_traits>
+
 namespace kq {
 namespace viterbi {
 
-constexpr int THREADS = 1024;
 typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
 template <int K> constexpr int edges() { return 65536 >> K; }
+// decision bytes per step: K bits a node (3 take the room of 4)
 template <int K> constexpr int row_bytes() { return K == 2 ? edges<K>() / 4 : edges<K>() / 2; }
 
 // E4M3 (fn) byte -> fp16, exact (labels are finite).
@@ -98,197 +115,240 @@ __device__ __forceinline__ h2_t procedural_pair(uint32_t x0, uint32_t x1) {
   }
 }
 
-template <int K, int CB>
-__global__ __launch_bounds__(THREADS) void sqg_viterbi_kernel(const float* __restrict__ tiles, int64_t n_tiles,
-                                                              const uint8_t* __restrict__ lut, int ctx,
-                                                              float* __restrict__ out_tiles,
-                                                              int16_t* __restrict__ out_states,
-                                                              uint8_t* __restrict__ dec_ws) {
-  constexpr int E = edges<K>(), PAIRS = E / 2, PER = PAIRS / THREADS, Q = 1 << K;
+typedef uint16_t us2_t __attribute__((ext_vector_type(2)));
+typedef int16_t ss2_t __attribute__((ext_vector_type(2)));
+
+// Minimum of N packed cost pairs and, in the top bit of each half of bit[b],
+// bit b of the index of the first smallest (log2 N of them).  The bits of
+// costs (never negative) order as their values do.
+template <int N> struct First {
+  static constexpr int BITS = N == 2 ? 1 : First<N / 2>::BITS + 1;
+  uint32_t best;
+  uint32_t bit[BITS];
+};
+template <> struct First<1> {
+  static constexpr int BITS = 0;
+  uint32_t best;
+};
+
+template <int N>
+__device__ __forceinline__ First<N> first_smallest(const uint32_t* cost) {
+  if constexpr (N == 1) {
+    return First<1>{cost[0]};
+  } else {
+    const First<N / 2> l = first_smallest<N / 2>(cost), r = first_smallest<N / 2>(cost + N / 2);
+    First<N> f;
+    const us2_t a = __builtin_bit_cast(us2_t, l.best), b = __builtin_bit_cast(us2_t, r.best);
+    f.best = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(a, b));
+    // negative where the right half's minimum is strictly smaller
+    const uint32_t less = __builtin_bit_cast(uint32_t, __builtin_bit_cast(ss2_t, b) - __builtin_bit_cast(ss2_t, a));
+    if constexpr (N > 2) {
+#pragma unroll
+      for (int i = 0; i < First<N / 2>::BITS; ++i) f.bit[i] = (less & r.bit[i]) | (~less & l.bit[i]);
+    }
+    f.bit[First<N>::BITS - 1] = less;
+    return f;
+  }
+}
+
+// The argmin order of the reference's reductions: cost first, then node e's
+// place in its shuffle-down trees (14 bits, unique per node).
+__device__ __forceinline__ uint32_t argmin_key(uint32_t cost_bits, int e) {
+  const int t = e & 1023;
+  return cost_bits << 16 | (uint32_t)((bitrev5(t >> 5) << 5 | bitrev5(t & 31)) << 4 | e >> 10);
+}
+__device__ __forceinline__ int argmin_node(uint32_t key) {
+  const int t = (int)(key >> 4) & 1023;
+  return (int)(key & 15u) << 10 | bitrev5(t >> 5) << 5 | bitrev5(t & 31);
+}
+
+template <int K, int CB, int T>
+__global__ __launch_bounds__(T, 4) void sqg_viterbi_kernel(const float* __restrict__ tiles, int64_t n_tiles,
+                                                           const uint8_t* __restrict__ lut, int ctx,
+                                                           float* __restrict__ out_tiles,
+                                                           int16_t* __restrict__ out_states,
+                                                           uint8_t* __restrict__ dec_ws) {
+  constexpr int E = edges<K>(), NPT = E / T, NP = NPT / 2, Q = 1 << K;
+  constexpr int NIN = NPT > Q ? NPT / Q : 1;  // predecessors of a thread's nodes, per k
   constexpr int KR = 16 - K, PSTEP = 1 << (16 - 2 * K), RB = row_bytes<K>();
-  constexpr uint32_t CM = cb_mult<CB>(), CSTEP = CM << KR;
-  static_assert(PER >= 1 && PAIRS % THREADS == 0, "node pairs per thread");
-  __shared__ __attribute__((aligned(16))) uint8_t lab[CB == 0 ? 65536 : 16];  // [pair][k][2]
+  constexpr uint32_t CM = cb_mult<CB>();
+  static_assert(NPT >= 4 && E % T == 0, "nodes per thread");
+  // A thread's decisions of one step: bit b of node 2 j + h sits in half h of
+  // word NP b / 16, NP b % 16 + j places below the top; two planes of 16
+  // nodes or less share a word, and four planes of 4 nodes are cut to 16 bits.
+  constexpr int NW = NP * (K - 1) / 16 + 1, BYTES = RB / T;
+  static_assert(BYTES == 4 * NW || (BYTES == 2 && NP * K == 8), "decision bytes per thread");
+  typedef _Float16 in_t __attribute__((ext_vector_type(NIN)));
   __shared__ __attribute__((aligned(16))) _Float16 cost[2][E];
   __shared__ _Float16 w16[256];
-  __shared__ float red_c[THREADS];
-  __shared__ int red_i[THREADS];
+  __shared__ uint16_t path[256];
+  __shared__ uint32_t red[T / 64];
   __shared__ int sh_edge;
   const int tid = threadIdx.x;
   uint8_t* dec = dec_ws + (int64_t)blockIdx.x * 256 * RB;
 
-  if constexpr (CB == 0) {
-    for (int s = tid; s < 65536; s += THREADS) {
-      const int k = s >> KR, o = s & (E - 1);
-      lab[(o >> 1) * (2 * Q) + 2 * k + (o & 1)] = lut[s];
+  h2_t label[NP][Q];  // of nodes NPT tid + 2 j, + 1 and predecessor k
+#pragma unroll
+  for (int j = 0; j < NP; ++j) {
+    const int o = NPT * tid + 2 * j;
+#pragma unroll
+    for (int k = 0; k < Q; ++k) {
+      const uint32_t s = (uint32_t)(k << KR | o);
+      if constexpr (CB == 0) label[j][k] = pair_labels(*reinterpret_cast<const uint16_t*>(lut + s));
+      else label[j][k] = procedural_pair<CB>(s * CM, s * CM + CM);
     }
   }
 
   int cb = 0;  // cost[cb] = the buffer the next step writes; cost[cb ^ 1] its input
+  // one step at position ri.  first: the pass's first step (pre_state >= 0
+  // forces its predecessor); keep: write the decisions
+  auto step = [&](auto first_t, auto keep_t, int ri, int pre_state) {
+    constexpr bool first = decltype(first_t)::value, keep = decltype(keep_t)::value;
+    cb ^= 1;  // swap: the last step's output becomes this step's input
+    const _Float16* prev = cost[cb ^ 1];
+    _Float16* cur = cost[cb];
+    const _Float16 w = w16[ri];
+    h2_t w2;
+    w2[0] = w2[1] = w;
+    const int in0 = NPT * tid >> K;
+    in_t c[Q];
+    if constexpr (!first) {
+#pragma unroll
+      for (int k = 0; k < Q; ++k) c[k] = *reinterpret_cast<const in_t*>(prev + in0 + k * PSTEP);
+    }
+    uint32_t out[NP];
+    uint32_t word[NW] = {};
+#pragma unroll
+    for (int j = 0; j < NP; ++j) {
+      const int jin = 2 * j >> K;  // which of the thread's predecessors
+      auto edge = [&](int k) -> h2_t {
+        const h2_t d = label[j][k] - w2;
+        if constexpr (first) {
+          h2_t err = d * d;
+          if (pre_state >= 0 && in0 + jin + k * PSTEP != pre_state) {
+            err[0] = (_Float16)__builtin_inff();
+            err[1] = (_Float16)__builtin_inff();
+          }
+          return err;
+        } else {
+          h2_t c2;
+          if constexpr (NIN == 1) c2[0] = c2[1] = c[k][0];
+          else c2[0] = c2[1] = c[k][jin];
+          return __builtin_elementwise_fma(d, d, c2);
+        }
+      };
+      uint32_t err[Q];
+#pragma unroll
+      for (int k = 0; k < Q; ++k) err[k] = __builtin_bit_cast(uint32_t, edge(k));
+      if constexpr (keep) {
+        const First<Q> f = first_smallest<Q>(err);
+        out[j] = f.best;
+#pragma unroll
+        for (int b = 0; b < K; ++b)
+          word[NP * b / 16] |= f.bit[b] >> (NP * b % 16 + j) & 0x80008000u >> (NP * b % 16 + j);
+      } else {
+        us2_t best = __builtin_bit_cast(us2_t, err[0]);
+#pragma unroll
+        for (int k = 1; k < Q; ++k) best = __builtin_elementwise_min(best, __builtin_bit_cast(us2_t, err[k]));
+        out[j] = __builtin_bit_cast(uint32_t, best);
+      }
+    }
+    uint32_t* dst = reinterpret_cast<uint32_t*>(cur + NPT * tid);
+    if constexpr (NP >= 4) {
+#pragma unroll
+      for (int j = 0; j < NP; j += 4)
+        *reinterpret_cast<u32x4_t*>(dst + j) = u32x4_t{out[j], out[j + 1], out[j + 2], out[j + 3]};
+    } else {
+      *reinterpret_cast<u32x2_t*>(dst) = u32x2_t{out[0], out[1]};
+    }
+    if constexpr (keep) {
+      uint8_t* at = dec + ri * RB + BYTES * tid;
+      if constexpr (NW == 2) *reinterpret_cast<u32x2_t*>(at) = u32x2_t{word[0], word[1]};
+      else if constexpr (BYTES == 4) *reinterpret_cast<uint32_t*>(at) = word[0];
+      else *reinterpret_cast<uint16_t*>(at) = (uint16_t)((word[0] >> 8 & 0xffu) | (word[0] >> 16 & 0xff00u));
+    }
+    __syncthreads();
+  };
+
+  auto decision_at = [&](int ri, int e) -> int {
+    const int o = e % NPT, j = o >> 1, h = o & 1;
+    const uint8_t* at = dec + ri * RB + BYTES * (e / NPT);
+    uint32_t half[NW];  // the halves of this parity, at bits 15 .. 0
+#pragma unroll
+    for (int v = 0; v < NW; ++v)
+      half[v] = BYTES == 2 ? (uint32_t)at[h] << 8 : *reinterpret_cast<const uint16_t*>(at + 4 * v + 2 * h);
+    uint32_t k = 0;
+#pragma unroll
+    for (int b = 0; b < K; ++b) k |= (half[NP * b / 16] >> (15 - NP * b % 16 - j) & 1u) << b;
+    return (int)k;
+  };
+
+  // Walk back from `edge` through the decisions of rows - 1 .. 0 (wave 0);
+  // states go to path[] when asked.  Lane l reads the decisions that steps
+  // i .. i - DEPTH + 1 meet if its digits were the decisions of the first
+  // DEPTH - 1 of them.
+  auto trace = [&](int edge, int rows, bool keep_path) -> int {
+    constexpr int DEPTH = K == 2 ? 4 : K == 3 ? 3 : 2;
+    const int lane = tid & 63;
+    for (int i = rows - 1; i >= 0; i -= DEPTH) {
+      int b[DEPTH], e = edge;
+#pragma unroll
+      for (int d = 0; d < DEPTH; ++d) {
+        const int ri = max(i - d, 0);
+        b[d] = decision_at(ri, e);
+        e = (lane >> K * d & (Q - 1)) << (16 - 2 * K) | e >> K;
+      }
+      int who = 0;
+#pragma unroll
+      for (int d = 0; d < DEPTH; ++d) {
+        if (i - d < 0) break;
+        const int k = __builtin_amdgcn_readlane(b[d], who);
+        const int before = k << (16 - 2 * K) | edge >> K;
+        if (keep_path && lane == 0) path[i - d] = (uint16_t)(before << K | edge);
+        edge = before;
+        who |= k << K * d;
+      }
+    }
+    return edge;
+  };
+
+  constexpr std::true_type yes{};
+  constexpr std::false_type no{};
   for (int64_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
     __syncthreads();
     if (tid < 256) w16[tid] = (_Float16)tiles[tile * 256 + tid];
     __syncthreads();
 
-    // one pass: `steps` steps starting at position `roll`; decisions kept
-    // from step trace_start on; pre_state >= 0 forces the first step's
-    // predecessor
-    auto pass = [&](int roll, int steps, int pre_state, int trace_start) {
-      for (int i = 0; i < steps; ++i) {
-        cb ^= 1;  // swap: the last step's output becomes this step's input
-        const _Float16* prev = cost[cb ^ 1];
-        _Float16* cur = cost[cb];
-        const int ri = (i + roll) & 255;
-        const _Float16 w = w16[ri];
-        h2_t w2;
-        w2[0] = w;
-        w2[1] = w;
-#pragma unroll
-        for (int j = 0; j < PER; ++j) {
-          const int p = tid + THREADS * j;  // node pair (2p, 2p + 1)
-          const int in0 = (2 * p) >> K;
-          uint32_t words[Q / 2];  // two predecessors' label pairs per word
-          uint32_t x0 = (uint32_t)(2 * p) * CM;  // product of state (0 << KR) | 2p
-          if constexpr (CB != 0) {
-          } else if constexpr (K == 2) {
-            const u32x2_t v = *reinterpret_cast<const u32x2_t*>(lab + p * 2 * Q);
-            words[0] = v[0];
-            words[1] = v[1];
-          } else if constexpr (K == 3) {
-            const u32x4_t v = *reinterpret_cast<const u32x4_t*>(lab + p * 2 * Q);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) words[q] = v[q];
-          } else {
-            const u32x4_t v0 = *reinterpret_cast<const u32x4_t*>(lab + p * 2 * Q);
-            const u32x4_t v1 = *reinterpret_cast<const u32x4_t*>(lab + p * 2 * Q + 16);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              words[q] = v0[q];
-              words[4 + q] = v1[q];
-            }
-          }
-          h2_t best;
-          int k0 = 0, k1 = 0;
-#pragma unroll
-          for (int k = 0; k < Q; ++k) {
-            const int in = in0 + k * PSTEP;
-            h2_t label;
-            if constexpr (CB == 0) {
-              label = pair_labels(words[k >> 1] >> (16 * (k & 1)));
-            } else {
-              label = procedural_pair<CB>(x0, x0 + CM);
-              x0 += CSTEP;
-            }
-            const h2_t d = label - w2;
-            h2_t err;
-            if (i == 0) {
-              err = d * d;
-              if (pre_state >= 0 && in != pre_state) {
-                err[0] = (_Float16)__builtin_inff();
-                err[1] = (_Float16)__builtin_inff();
-              }
-            } else {
-              const _Float16 c = prev[in];
-              h2_t c2;
-              c2[0] = c;
-              c2[1] = c;
-              err = __builtin_elementwise_fma(d, d, c2);
-            }
-            if (k == 0) {
-              best = err;
-            } else {
-              if (err[0] < best[0]) { best[0] = err[0]; k0 = k; }
-              if (err[1] < best[1]) { best[1] = err[1]; k1 = k; }
-            }
-          }
-          *reinterpret_cast<h2_t*>(cur + 2 * p) = best;
-          if (i >= trace_start) {
-            if constexpr (K == 2) {
-              // nodes 4m .. 4m + 3 share a byte: pair p and p + 1 (thread tid + 1)
-              const int mine = k0 | (k1 << 2);
-              const int next = __shfl_down(mine, 1);
-              if ((p & 1) == 0) dec[ri * RB + (p >> 1)] = (uint8_t)(mine | (next << 4));
-            } else {
-              dec[ri * RB + p] = (uint8_t)(k0 | (k1 << 4));
-            }
-          }
-        }
-        __syncthreads();
-      }
-    };
-
-    auto decision_at = [&](int ri, int edge) -> int {
-      if constexpr (K == 2) return (dec[ri * RB + (edge >> 2)] >> ((edge & 3) * 2)) & 3;
-      else return (dec[ri * RB + (edge >> 1)] >> ((edge & 1) * 4)) & 15;
-    };
-
-    // primer
-    pass(256 - ctx, 2 * ctx, -1, ctx);
+    // primer: positions -ctx .. ctx - 1, decisions kept from position 0 on
+    step(yes, no, 256 - ctx, -1);
+    for (int i = 1; i < ctx; ++i) step(no, no, i + 256 - ctx, -1);
+    for (int i = 0; i < ctx; ++i) step(no, yes, i, -1);
+    // argmin of the incoming buffer (the second-to-last step's costs); edge 0 if none is finite
     {
-      // argmin of the incoming buffer (the second-to-last step's costs)
-      const _Float16* c = cost[cb ^ 1];
-      float bc = __builtin_inff();
-      int bi = -1;
-      for (int e = tid; e < E; e += THREADS) {
-        const float v = (float)c[e];
-        if (v < bc) {
-          bc = v;
-          bi = e;
-        }
-      }
-      red_c[tid] = bc;
-      red_i[tid] = bi;
+      const uint16_t* c = reinterpret_cast<const uint16_t*>(cost[cb ^ 1]);
+      uint32_t key = ~0u;
+      for (int e = tid; e < E; e += T) key = min(key, argmin_key(c[e], e));
+#pragma unroll
+      for (int span = 32; span > 0; span >>= 1) key = min(key, (uint32_t)__shfl_xor((int)key, span));
+      if ((tid & 63) == 0) red[tid >> 6] = key;
       __syncthreads();
-      for (int span = THREADS / 2; span > 0; span >>= 1) {
-        if (tid < span) {
-          const float ca = red_c[tid], cb2 = red_c[tid + span];
-          const int ia = red_i[tid], ib = red_i[tid + span];
-          bool take_b;
-          if (ib < 0) take_b = false;
-          else if (ia < 0) take_b = true;
-          else if (cb2 != ca) take_b = cb2 < ca;
-          else {
-            // equal costs: the reference's reduction order
-            const int ta = ia & 1023, tb = ib & 1023;
-            const int ka = (bitrev5(ta >> 5) << 5) | bitrev5(ta & 31);
-            const int kb = (bitrev5(tb >> 5) << 5) | bitrev5(tb & 31);
-            take_b = kb < ka || (kb == ka && (ib >> 10) < (ia >> 10));
-          }
-          if (take_b) {
-            red_c[tid] = cb2;
-            red_i[tid] = ib;
-          }
-        }
-        __syncthreads();
+      if (tid < 64) {
+        for (int v = 0; v < T / 64; ++v) key = min(key, red[v]);
+        const int edge = trace(key >= 0x7c000000u ? 0 : argmin_node(key), ctx, false);
+        if (tid == 0) sh_edge = edge;
       }
-    }
-    if (tid == 0) {
-      int edge = red_i[0] < 0 ? 0 : red_i[0];
-      for (int i = 2 * ctx - 1; i >= 0; --i) {
-        const int ri = (i + 256 - ctx) & 255;
-        edge = (decision_at(ri, edge) << (16 - 2 * K)) | (edge >> K);
-        if (ri == 0) break;
-      }
-      sh_edge = edge;
     }
     __syncthreads();
     const int end_state = sh_edge;
-    pass(0, 256, end_state, 0);
-    if (tid == 0) {
-      int edge = end_state;
-      for (int i = 255; i >= 0; --i) {
-        const int prev_edge = (decision_at(i, edge) << (16 - 2 * K)) | (edge >> K);
-        const int state = ((prev_edge << K) | edge) & 0xffff;
-        out_states[tile * 256 + i] = (int16_t)(uint16_t)state;
-        if constexpr (CB == 0) {
-          const int k = state >> KR, o = state & (E - 1);
-          out_tiles[tile * 256 + i] = (float)e4m3_to_f16(lab[(o >> 1) * (2 * Q) + 2 * k + (o & 1)]);
-        } else {
-          const uint32_t x = (uint32_t)state * CM;
-          out_tiles[tile * 256 + i] = (float)procedural_pair<CB>(x, x + CM)[0];
-        }
-        edge = prev_edge;
-      }
+    step(yes, yes, 0, end_state);
+    for (int i = 1; i < 256; ++i) step(no, yes, i, -1);
+    if (tid < 64) trace(end_state, 256, true);
+    __syncthreads();
+    if (tid < 256) {
+      const uint32_t state = path[tid];
+      out_states[tile * 256 + tid] = (int16_t)(uint16_t)state;
+      if constexpr (CB == 0) out_tiles[tile * 256 + tid] = (float)e4m3_to_f16(lut[state]);
+      else out_tiles[tile * 256 + tid] = (float)procedural_pair<CB>(state * CM, state * CM + CM)[0];
     }
   }
 }
@@ -306,15 +366,29 @@ extern "C" int64_t kq_sqg_quantize_workspace_size(int bits, int workgroups) {
 
 namespace {
 
-template <int CB>
-void launch_viterbi(int bits, unsigned grid, hipStream_t st, const float* tiles, int64_t n_tiles, const uint8_t* lut,
-                    int ctx, float* out_tiles, int16_t* out_states, uint8_t* ws) {
-  if (bits == 2)
-    sqg_viterbi_kernel<2, CB><<<grid, THREADS, 0, st>>>(tiles, n_tiles, lut, ctx, out_tiles, out_states, ws);
-  else if (bits == 3)
-    sqg_viterbi_kernel<3, CB><<<grid, THREADS, 0, st>>>(tiles, n_tiles, lut, ctx, out_tiles, out_states, ws);
+// 512-thread workgroups, two per CU, once there is more than one per CU to
+// run; else 1,024 threads on each tile (with one tile per CU twice the
+// threads are what shortens it).
+template <int K, int CB>
+void launch_viterbi_k(int64_t workgroups, int cus, hipStream_t st, const float* tiles, int64_t n_tiles,
+                      const uint8_t* lut, int ctx, float* out_tiles, int16_t* out_states, uint8_t* ws) {
+  const unsigned grid = (unsigned)(n_tiles < workgroups ? n_tiles : workgroups);
+  if ((int64_t)grid > cus)
+    sqg_viterbi_kernel<K, CB, 512><<<grid, 512, 0, st>>>(tiles, n_tiles, lut, ctx, out_tiles, out_states, ws);
   else
-    sqg_viterbi_kernel<4, CB><<<grid, THREADS, 0, st>>>(tiles, n_tiles, lut, ctx, out_tiles, out_states, ws);
+    sqg_viterbi_kernel<K, CB, 1024><<<grid, 1024, 0, st>>>(tiles, n_tiles, lut, ctx, out_tiles, out_states, ws);
+}
+
+template <int CB>
+hipError_t launch_viterbi(int bits, int64_t workgroups, hipStream_t st, const float* tiles, int64_t n_tiles,
+                          const uint8_t* lut, int ctx, float* out_tiles, int16_t* out_states, uint8_t* ws) {
+  int dev = 0, cus = 0;
+  hipError_t e = st ? hipStreamGetDevice(st, &dev) : hipGetDevice(&dev);
+  if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  if (e != hipSuccess) return e;
+  auto* launch = bits == 2 ? launch_viterbi_k<2, CB> : bits == 3 ? launch_viterbi_k<3, CB> : launch_viterbi_k<4, CB>;
+  launch(workgroups, cus, st, tiles, n_tiles, lut, ctx, out_tiles, out_states, ws);
+  return hipGetLastError();
 }
 
 // shared checks of both entry points; 1 = nothing to do, 0 = launch, <0 = error
@@ -342,10 +416,9 @@ extern "C" int kq_sqg_quantize_tiles(const float* tiles, int64_t n_tiles, const 
                               out_states, workspace, workspace_bytes, workgroups);
   if (rc) return rc > 0 ? KQ_OK : rc;
   if (!lut) return kq_fail(KQ_ERR_INVALID, "%s: null buffer", fn);
-  const unsigned grid = (unsigned)(n_tiles < workgroups ? n_tiles : workgroups);
-  launch_viterbi<0>(bits, grid, (hipStream_t)stream, tiles, n_tiles, lut, tailbite_context, out_tiles, out_states,
-                    (uint8_t*)workspace);
-  return kq_check_launch(hipGetLastError(), fn);
+  return kq_check_launch(launch_viterbi<0>(bits, workgroups, (hipStream_t)stream, tiles, n_tiles, lut,
+                                           tailbite_context, out_tiles, out_states, (uint8_t*)workspace),
+                         fn);
 }
 
 extern "C" int kq_sqg_quantize_tiles_procedural(const float* tiles, int64_t n_tiles, int bits, int codebook,
@@ -358,12 +431,8 @@ extern "C" int kq_sqg_quantize_tiles_procedural(const float* tiles, int64_t n_ti
   const int rc = check_search(fn, "procedural control", tiles, n_tiles, bits, tailbite_context, out_tiles,
                               out_states, workspace, workspace_bytes, workgroups);
   if (rc) return rc > 0 ? KQ_OK : rc;
-  const unsigned grid = (unsigned)(n_tiles < workgroups ? n_tiles : workgroups);
-  if (codebook == 1)
-    launch_viterbi<1>(bits, grid, (hipStream_t)stream, tiles, n_tiles, nullptr, tailbite_context, out_tiles,
-                      out_states, (uint8_t*)workspace);
-  else
-    launch_viterbi<2>(bits, grid, (hipStream_t)stream, tiles, n_tiles, nullptr, tailbite_context, out_tiles,
-                      out_states, (uint8_t*)workspace);
-  return kq_check_launch(hipGetLastError(), fn);
+  auto* launch = codebook == 1 ? launch_viterbi<1> : launch_viterbi<2>;
+  return kq_check_launch(launch(bits, workgroups, (hipStream_t)stream, tiles, n_tiles, nullptr, tailbite_context,
+                                out_tiles, out_states, (uint8_t*)workspace),
+                         fn);
 }

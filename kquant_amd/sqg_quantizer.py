@@ -34,7 +34,7 @@ _WORKSPACES: dict[tuple[torch.device, int, int], torch.Tensor] = {}
 
 
 def _workgroups(device: torch.device) -> int:
-    return torch.cuda.get_device_properties(device).multi_processor_count
+    return 2 * torch.cuda.get_device_properties(device).multi_processor_count  # two tiles per CU
 
 
 def quantize_tiles_sqg(tiles: torch.Tensor, lut: torch.Tensor, bits: int,

@@ -103,3 +103,21 @@ def test_install_hook_routes_none_to_mcg(gpu):
     assert np.array_equal(vals.cpu().numpy(), want_vals)
     with pytest.raises(ValueError, match="1 \\(MCG\\) or 2 \\(MUL1\\)"):
         sqg_quantizer.quantize_tiles_procedural(torch.from_numpy(x).to(gpu), 2, 3)
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4])
+@pytest.mark.parametrize("ctx", [1, 127])
+def test_two_tiles_per_cu(gpu, bits, ctx):
+    """More tiles than CUs take 512-thread workgroups, two per CU (other node
+    ownership and decision packing), at the shortest context and an odd one:
+    every copy of the same few tiles gives the oracle's states and values, and
+    so does the one-tile-per-CU form."""
+    x = _tiles(bits, 5 * bits + ctx)
+    lut_np = oracle.sqg_xor_cheb_t12_bytes(bits)
+    want_vals, want_states = oracle.sqg_quantize_tiles(x, lut_np, bits, ctx)
+    lut = sqg_xor_cheb_t12_bytes(bits, device=gpu)
+    cus = torch.cuda.get_device_properties(gpu).multi_processor_count
+    for copies in (1, -(-(cus + 1) // x.shape[0]), -(-(2 * cus + 1) // x.shape[0])):
+        vals, states = sqg_quantizer.quantize_tiles_sqg(torch.from_numpy(x).to(gpu).repeat(copies, 1), lut, bits, ctx)
+        assert np.array_equal(states.cpu().numpy(), np.tile(want_states, (copies, 1)))
+        assert np.array_equal(vals.cpu().numpy(), np.tile(want_vals, (copies, 1)))
