@@ -224,6 +224,17 @@ int kq_mx_linear(int w_fmt, const void* a, int64_t lda, const void* w_q,
                  const uint8_t* w_scale, int64_t m, int64_t n, int64_t k,
                  int out_dtype, void* c, int64_t ldc, void* stream);
 
+/* kq_mx_linear with a workspace: shapes whose 256 x 256 output tiles leave
+ * CUs idle run K in slices, each into its own fp32 plane of the workspace,
+ * summed in slice order by a second launch (deterministic; results agree with
+ * kq_mx_linear's to fp32 summation order).  kq_mx_linear_workspace_size gives
+ * the bytes (0 when the split does not pay; it plans for the current device);
+ * a smaller workspace runs as kq_mx_linear.  16-byte aligned, uninitialised. */
+int64_t kq_mx_linear_workspace_size(int64_t m, int64_t n, int64_t k);
+int kq_mx_linear_ws(int w_fmt, const void* a, int64_t lda, const void* w_q, const uint8_t* w_scale, int64_t m,
+                    int64_t n, int64_t k, int out_dtype, void* c, int64_t ldc, void* workspace,
+                    int64_t workspace_bytes, void* stream);
+
 /* C [m, n] = dequant(A) [m, k] x dequant(W) [n, k]^T with both operands
  * MXFP8: A E4M3 bytes [m, k] (row stride lda bytes, lda % 16 == 0) with E8M0
  * scales [m, k/32], W E4M3 bytes [n, k] with E8M0 scales [n, k/32]; the
@@ -236,7 +247,8 @@ int kq_mx_linear(int w_fmt, const void* a, int64_t lda, const void* w_q,
  * scales 4-byte aligned.  workspace (kq_mx_linear_mx_workspace_size bytes,
  * 256-byte aligned, uninitialised) takes both scale planes transposed to
  * [k/128][rows] dwords, the layout the kernel loads a 128-k stage's scales
- * from.  The matrix cores sum the 64 products of a step with a few fp32 ulps
+ * from, and the planes of a split over K as in kq_mx_linear_ws (the scale
+ * planes alone are enough: it then runs unsplit).  The matrix cores sum the 64 products of a step with a few fp32 ulps
  * of error (measured ~1e-5 relative). */
 int64_t kq_mx_linear_mx_workspace_size(int64_t m, int64_t n, int64_t k);
 int kq_mx_linear_mx(int a_fmt, const void* a_q, const uint8_t* a_scale, int64_t lda, int w_fmt,
@@ -648,6 +660,10 @@ int kq_kqsc_stats(const uint8_t* payload, int64_t payload_bytes, int64_t rows, i
 
 /* Workspace bytes of kq_mx_linear_f32 (m * 3k bf16), -1 on bad sizes. */
 int64_t kq_mx_linear_f32_workspace_size(int64_t m, int64_t k);
+
+/* kq_mx_linear_f32's workspace with room for a split over K as in
+ * kq_mx_linear_ws (taken when the workspace holds it). */
+int64_t kq_mx_linear_f32_split_workspace_size(int64_t m, int64_t n, int64_t k);
 
 /* C [m, n] fp32 = A [m, k] fp32 x dequant(W [n, k])^T at fp32-GEMM accuracy:
  * A is split exactly into three bf16 terms (a = a0 + a1 + a2) written to the

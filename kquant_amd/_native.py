@@ -50,7 +50,7 @@ _U32 = ctypes.c_uint32
 _F32 = ctypes.c_float
 _F64 = ctypes.c_double
 
-# name -> argtypes (every entry point returns int)
+# name -> argtypes (every entry point returns int, the workspace sizes int64)
 SIGNATURES: dict[str, list] = {
     "kq_mx_quantize": [_INT, _INT, _VP, _I64, _I64, _I64, _VP, _VP, _U32, _VP],
     "kq_mx_dequant": [_INT, _VP, _VP, _I64, _I64, _INT, _VP, _U32, _VP],
@@ -64,6 +64,9 @@ SIGNATURES: dict[str, list] = {
     "kq_sym_lerp": [_VP, _F32, _VP, _I64, _F32, _VP, _VP],
     "kq_cov_stats": [_VP, _I64, _VP, _VP, _VP],
     "kq_mx_linear": [_INT, _VP, _I64, _VP, _VP, _I64, _I64, _I64, _INT, _VP, _I64, _VP],
+    "kq_mx_linear_ws": [_INT, _VP, _I64, _VP, _VP, _I64, _I64, _I64, _INT, _VP, _I64, _VP, _I64, _VP],
+    "kq_mx_linear_workspace_size": [_I64, _I64, _I64],
+    "kq_mx_linear_f32_split_workspace_size": [_I64, _I64, _I64],
     "kq_mx_linear_mx": [_INT, _VP, _VP, _I64, _INT, _VP, _VP, _I64, _I64, _I64, _INT, _VP, _I64, _VP, _I64, _VP],
     "kq_mx_linear_mm": [_INT, _VP, _INT, _I64, _VP, _VP, _I64, _I64, _I64, _INT, _VP, _I64, _VP, _I64, _VP],
     "kq_moe_forward": [_INT, _F32, _F32, _VP, _I64, _I64, _I64, _VP, _VP, _INT, _INT, _I64,
@@ -165,7 +168,7 @@ def library() -> ctypes.CDLL:
         lib.kq_route_sort_workspace_size.argtypes = [_I64, _INT, _INT]
         for name, argtypes in SIGNATURES.items():
             fn = getattr(lib, name)
-            fn.restype = ctypes.c_int
+            fn.restype = ctypes.c_int64 if name.endswith("_workspace_size") else ctypes.c_int
             fn.argtypes = argtypes
         _lib = lib
     return _lib

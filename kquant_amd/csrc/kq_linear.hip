@@ -33,7 +33,7 @@ using gemm::u32x4_t;
 template <int FMT, int OUT>
 __global__ __launch_bounds__(512, 1) void mx_linear_kernel(
     const uint16_t* __restrict__ a, int64_t lda, const uint8_t* __restrict__ wq,
-    const uint8_t* __restrict__ ws, void* __restrict__ c, int64_t ldc, int M, int N, int K, int KB) {
+    const uint8_t* __restrict__ ws, void* __restrict__ c, int64_t ldc, int M, int N, int K, int KB, int64_t plane) {
   using namespace lin;
   constexpr int BROW = b_row<FMT>();
   constexpr int WBYTES = FMT == 0 ? BK : BK / 2;  // packed bytes per row per step
@@ -112,13 +112,15 @@ __global__ __launch_bounds__(512, 1) void mx_linear_kernel(
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
   const int frow = lane & 31, fk = lane >> 5;  // fragment row, k half (8 elements)
-  const int steps = K / BK;
-  load(0);
+  // blockIdx.z: slice of the K steps, written to its own plane of c
+  const int steps = K / BK, slices = (int)gridDim.z, z = (int)blockIdx.z;
+  const int s_begin = (int)((int64_t)z * steps / slices), s_end = (int)((int64_t)(z + 1) * steps / slices);
+  load(s_begin * BK);
   store(0);
   __syncthreads();
-  for (int s = 0; s < steps; ++s) {
-    const int buf = s & 1;
-    if (s + 1 < steps) load((s + 1) * BK);
+  for (int s = s_begin; s < s_end; ++s) {
+    const int buf = (s - s_begin) & 1;
+    if (s + 1 < s_end) load((s + 1) * BK);
     const unsigned char* base = lds + buf * stage_bytes<FMT>();
     const unsigned char* bb = base + A_BYTES;
     const unsigned char* sb = bb + b_bytes<FMT>();
@@ -148,7 +150,7 @@ __global__ __launch_bounds__(512, 1) void mx_linear_kernel(
         for (int j = 0; j < 4; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
     }
-    if (s + 1 < steps) store(buf ^ 1);
+    if (s + 1 < s_end) store(buf ^ 1);
     __syncthreads();
   }
 
@@ -162,7 +164,7 @@ __global__ __launch_bounds__(512, 1) void mx_linear_kernel(
         const int gm = m0 + wm + i * 32 + 8 * (r >> 2) + 4 * fk + (r & 3);
         const int gn = n0 + wn + j * 32 + frow;
         if (gm < M && gn < N) {
-          if (OUT == 2) static_cast<float*>(c)[(int64_t)gm * ldc + gn] = acc[i][j][r];
+          if (OUT == 2) static_cast<float*>(c)[z * plane + (int64_t)gm * ldc + gn] = acc[i][j][r];
           else static_cast<__bf16*>(c)[(int64_t)gm * ldc + gn] = (__bf16)acc[i][j][r];
         }
       }
@@ -533,6 +535,7 @@ __global__ __launch_bounds__(256, 1) void mx_linear_dma_kernel(
 //    bounded it (measured: 376 us of loads alone at cfg2; 139 us for twice
 //    the bytes in whole lines without per-row scale dwords).
 //  * rows past M or N read as zero (out-of-range offsets) and are not stored.
+//  * split K as in mx_linear_dma_kernel, by 128-k stages.
 namespace lin8 {
 constexpr int BK = 64, SK = 128;             // MFMA step, LDS stage
 constexpr int OP_BYTES = 256 * SK;           // one operand tile per stage
@@ -549,11 +552,12 @@ template <int OUT>
 __global__ __launch_bounds__(512, 1) void mx_linear_a8_kernel(
     const uint8_t* __restrict__ aq, int64_t lda, uint32_t a_bytes, const uint32_t* __restrict__ ast,
     uint32_t ast_bytes, const uint8_t* __restrict__ wq, uint32_t w_bytes, const uint32_t* __restrict__ wst,
-    uint32_t wst_bytes, void* __restrict__ c, int64_t ldc, int M, int N, int K, int MS, int NS) {
+    uint32_t wst_bytes, void* __restrict__ c, int64_t ldc, int M, int N, int K, int MS, int NS, int slices,
+    int64_t plane) {
   using namespace lin8;
   using dma::i32x4_t;
   constexpr int BM = lin::BM, BN = lin::BN;
-  const int mtiles = (M + BM - 1) / BM, ntiles = (N + BN - 1) / BN, total = mtiles * ntiles;
+  const int mtiles = (M + BM - 1) / BM, ntiles = (N + BN - 1) / BN, tiles = mtiles * ntiles, total = tiles * slices;
   const int G = gridDim.x;
   const int worker = (int)(blockIdx.x % 8) * (G / 8) + (int)(blockIdx.x / 8);
   if (worker >= total) return;
@@ -561,7 +565,7 @@ __global__ __launch_bounds__(512, 1) void mx_linear_a8_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const bool g0 = wave < 4;
   const int lw = wave & 3;
-  const int stages = K / SK, steps = K / BK;
+  const int stages = K / SK;
   const uint32_t lds0 = dma::lds_offset_of(lin8_lds);
   const i32x4_t a_rsrc = dma::make_rsrc(aq, a_bytes), w_rsrc = dma::make_rsrc(wq, w_bytes);
   const i32x4_t as_rsrc = dma::make_rsrc(ast, ast_bytes), ws_rsrc = dma::make_rsrc(wst, wst_bytes);
@@ -571,7 +575,7 @@ __global__ __launch_bounds__(512, 1) void mx_linear_a8_kernel(
   // slot l % 8, i.e. logical chunk (l % 8) ^ ((row / 2) % 8).  Scale dwords:
   // lane l of wave lw carries row 64 lw + l of the transposed planes
   // (MS / NS rows per 128-k chunk).
-  int lt = worker, ls = 0;
+  int lt = worker, ls = 0, ls_end = stages;
   const int prow = 8 * lw + (lane >> 3);  // + 32 q
   const int pch = (lane & 7) ^ ((prow >> 1) & 7);
   uint32_t a_base = 0, w_base = 0, as_off = 0, ws_off = 0;
@@ -579,8 +583,11 @@ __global__ __launch_bounds__(512, 1) void mx_linear_a8_kernel(
   const uint32_t a_qstep = (uint32_t)(32 * lda), w_qstep = (uint32_t)(32 * K);
   auto set_load_tile = [&]() {
     const bool live = lt < total;
+    const int sl = live ? lt / tiles : 0, tl = live ? lt - sl * tiles : 0;
+    ls = (int)((int64_t)sl * stages / slices);
+    ls_end = (int)((int64_t)(sl + 1) * stages / slices);
     int mt = 0, nt = 0;
-    if (live) lin3::tile_mn(lt, mtiles, ntiles, mt, nt);
+    if (live) lin3::tile_mn(tl, mtiles, ntiles, mt, nt);
     const int m0 = mt * BM, n0 = nt * BN;
     a_lim = live ? M - m0 - prow : 0;
     a_base = a_lim > 0 ? (uint32_t)((int64_t)(m0 + prow) * lda + 16 * pch) : 0u;
@@ -607,8 +614,7 @@ __global__ __launch_bounds__(512, 1) void mx_linear_a8_kernel(
                       base + (uint32_t)(S_OFF + 1024 + lw * 256));
   };
   auto advance = [&]() {
-    if (++ls == stages) {
-      ls = 0;
+    if (++ls == ls_end) {
       lt += G;
       set_load_tile();
     }
@@ -647,8 +653,10 @@ __global__ __launch_bounds__(512, 1) void mx_linear_a8_kernel(
   }
   int cslot = 0;
   for (int t = worker; t < total; t += G) {
+    const int sl = t / tiles, tl = t - sl * tiles;
     int mt, nt;
-    lin3::tile_mn(t, mtiles, ntiles, mt, nt);
+    lin3::tile_mn(tl, mtiles, ntiles, mt, nt);
+    const int steps = 2 * ((int)((int64_t)(sl + 1) * stages / slices) - (int)((int64_t)sl * stages / slices));
     const int m0 = mt * BM, n0 = nt * BN;
     const bool active = m0 + wm < M && n0 + wn < N;
     float16_t acc[2][4];
@@ -731,7 +739,7 @@ __global__ __launch_bounds__(512, 1) void mx_linear_a8_kernel(
             const int gm = m0 + wm + 32 * i + 8 * (r >> 2) + 4 * fg + (r & 3);
             const int gn = n0 + wn + 32 * j + fr;
             if (gm < M && gn < N) {
-              if (OUT == 2) static_cast<float*>(c)[(int64_t)gm * ldc + gn] = acc[i][j][r];
+              if (OUT == 2) static_cast<float*>(c)[sl * plane + (int64_t)gm * ldc + gn] = acc[i][j][r];
               else static_cast<__bf16*>(c)[(int64_t)gm * ldc + gn] = (__bf16)acc[i][j][r];
             }
           }
@@ -744,10 +752,18 @@ __global__ __launch_bounds__(512, 1) void mx_linear_a8_kernel(
 // Scale plane [rows, K / 32] bytes -> [K / 128][rows] dwords (the four
 // blocks of each row's 128-k window), the layout mx_linear_a8_kernel loads a
 // stage's scales from.  Dword (r, c) of the input is bytes 4c .. 4c + 3 of row r.
-__global__ __launch_bounds__(256) void scale_dwords_t_kernel(const uint32_t* __restrict__ in, int64_t rows,
-                                                             int64_t chunks, uint32_t* __restrict__ out) {
+// Both operands' planes in one launch: the first a_blocks blocks along x are
+// the activations'.
+__global__ __launch_bounds__(256) void scale_dwords_t_kernel(const uint32_t* __restrict__ a_in, int64_t a_rows,
+                                                             uint32_t* __restrict__ a_out, int a_blocks,
+                                                             const uint32_t* __restrict__ w_in, int64_t w_rows,
+                                                             uint32_t* __restrict__ w_out, int64_t chunks) {
   __shared__ uint32_t tile[32][33];
-  const int64_t r0 = (int64_t)blockIdx.x * 32, c0 = (int64_t)blockIdx.y * 32;
+  const bool is_a = (int)blockIdx.x < a_blocks;
+  const uint32_t* in = is_a ? a_in : w_in;
+  uint32_t* out = is_a ? a_out : w_out;
+  const int64_t rows = is_a ? a_rows : w_rows;
+  const int64_t r0 = (int64_t)(is_a ? blockIdx.x : blockIdx.x - a_blocks) * 32, c0 = (int64_t)blockIdx.y * 32;
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 32 x 8
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -759,6 +775,34 @@ __global__ __launch_bounds__(256) void scale_dwords_t_kernel(const uint32_t* __r
   for (int i = 0; i < 4; ++i) {
     const int64_t cc = c0 + ty + 8 * i, r = r0 + tx;
     if (r < rows && cc < chunks) out[cc * rows + r] = tile[tx][ty + 8 * i];
+  }
+}
+
+// C = the sum of the K slices' fp32 planes [slices][m, ldp] in slice order,
+// four columns (ldp % 4 == 0) per thread.
+template <int OUT>
+__global__ __launch_bounds__(256) void plane_sum_kernel(const float* __restrict__ planes, int slices, int64_t plane,
+                                                        int ldp, int m, int n, void* __restrict__ c, int64_t ldc) {
+  const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int per_row = ldp / 4;
+  const int64_t row = q / per_row;
+  const int col = (int)(q - row * per_row) * 4;
+  if (row >= m) return;
+  const float* p = planes + row * ldp + col;
+  float4_t v = *reinterpret_cast<const float4_t*>(p);
+  for (int s = 1; s < slices; ++s) v += *reinterpret_cast<const float4_t*>(p + s * plane);
+  const int64_t at = row * ldc + col;
+  if (col + 4 <= n && (reinterpret_cast<uintptr_t>(c) + at * (OUT == 2 ? 4 : 2)) % (OUT == 2 ? 16 : 8) == 0) {
+    if (OUT == 2) *reinterpret_cast<float4_t*>(static_cast<float*>(c) + at) = v;
+    else *reinterpret_cast<gemm::u32x2_t*>(static_cast<uint16_t*>(c) + at) =
+        gemm::u32x2_t{f32x2_to_bf16x2_bits(v[0], v[1]), f32x2_to_bf16x2_bits(v[2], v[3])};
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (col + j < n) {
+        if (OUT == 2) static_cast<float*>(c)[at + j] = v[j];
+        else static_cast<__bf16*>(c)[at + j] = (__bf16)v[j];
+      }
   }
 }
 
@@ -799,6 +843,55 @@ __global__ __launch_bounds__(256) void split3_bf16_kernel(const float* __restric
 }  // namespace kq
 
 using namespace kq;
+
+// Split K.  A shape whose 256 x 256 tiles leave CUs idle runs its K steps in
+// S slices, each writing its own fp32 plane in the workspace, and a second
+// launch adds the planes in slice order (deterministic).  S minimises the
+// rounds of (slice, tile) items times the steps of a slice, at the kernels'
+// measured time per 64-k step with one workgroup per CU, plus the sum's
+// launch and its plane traffic (written and read once, 5 TB/s).  M = 777,
+// N = 5000, K = 7168 (80 tiles, S = 3), MXFP8 x MXFP8:
+// 119 -> 66 us; M = 256, N = 2048, bf16 x E4M3: 140 -> 32 us; M = 512, N =
+// 12288 (96 tiles, S = 2): 145 -> 100 us.
+struct SplitPlan {
+  int slices = 1;
+  int64_t ldp = 0, plane = 0, bytes = 0;  // plane row stride and size (floats), all planes' bytes
+};
+constexpr double DMA_STEP_US = 1.25, STAGED_STEP_US = 1.6, A8_STEP_US = 0.98;
+
+static SplitPlan plan_split(int64_t m, int64_t n, int64_t k, double step_us, int cus) {
+  SplitPlan p;
+  p.ldp = (n + 3) / 4 * 4;
+  p.plane = m * p.ldp;
+  const int64_t tiles = ((m + lin::BM - 1) / lin::BM) * ((n + lin::BN - 1) / lin::BN), steps = k / lin::BK;
+  double best = 0.97 * (double)((tiles + cus - 1) / cus) * (double)steps * step_us;
+  for (int64_t s = 2; s <= 16 && s * 4 <= steps; ++s) {
+    const double t = (double)((tiles * s + cus - 1) / cus) * (double)((steps + s - 1) / s) * step_us + 6.0 +
+                     (double)(s * p.plane * 8) / 5e6;
+    if (t < best) {
+      best = t;
+      p.slices = (int)s;
+    }
+  }
+  p.bytes = p.slices > 1 ? p.slices * p.plane * 4 : 0;
+  return p;
+}
+
+static hipError_t stream_cus(hipStream_t st, int* cus) {
+  int dev = 0;
+  hipError_t e = st ? hipStreamGetDevice(st, &dev) : hipGetDevice(&dev);
+  if (e == hipSuccess) e = hipDeviceGetAttribute(cus, hipDeviceAttributeMultiprocessorCount, dev);
+  return e;
+}
+
+template <int OUT>
+static hipError_t sum_planes(const SplitPlan& p, const void* planes, int m, int n, void* c, int64_t ldc,
+                             hipStream_t st) {
+  const int64_t quads = m * (p.ldp / 4);
+  plane_sum_kernel<OUT><<<(unsigned)((quads + 255) / 256), 256, 0, st>>>(
+      static_cast<const float*>(planes), p.slices, p.plane, (int)p.ldp, m, n, c, ldc);
+  return hipGetLastError();
+}
 
 // Direct-to-LDS path: needs 4-byte aligned scale rows (KB % 128 == 0, scale
 // pointer 4-byte aligned); operands larger than one 32-bit buffer range are
@@ -842,19 +935,14 @@ static int64_t a8_scale_plane_bytes(int64_t rows, int64_t k) { return (rows * (k
 template <int OUT>
 static hipError_t launch_linear_a8(const uint8_t* aq, const uint8_t* as, int64_t lda, const uint8_t* wq,
                                    const uint8_t* ws, void* c, int64_t ldc, int M, int N, int K, void* workspace,
-                                   hipStream_t st) {
-  int dev = 0, cus = 0;
-  hipError_t e = st ? hipStreamGetDevice(st, &dev) : hipGetDevice(&dev);
-  if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  if (e != hipSuccess) return e;
+                                   int cus, hipStream_t st, int slices = 1, int64_t plane = 0) {
+  hipError_t e;
   const int64_t chunks = K / 128;
   uint32_t* ast = static_cast<uint32_t*>(workspace);
   uint32_t* wst = reinterpret_cast<uint32_t*>(static_cast<char*>(workspace) + a8_scale_plane_bytes(M, K));
-  scale_dwords_t_kernel<<<dim3((unsigned)((M + 31) / 32), (unsigned)((chunks + 31) / 32)), 256, 0, st>>>(
-      reinterpret_cast<const uint32_t*>(as), M, chunks, ast);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-  scale_dwords_t_kernel<<<dim3((unsigned)((N + 31) / 32), (unsigned)((chunks + 31) / 32)), 256, 0, st>>>(
-      reinterpret_cast<const uint32_t*>(ws), N, chunks, wst);
+  const int a_blocks = (M + 31) / 32, w_blocks = (N + 31) / 32;
+  scale_dwords_t_kernel<<<dim3((unsigned)(a_blocks + w_blocks), (unsigned)((chunks + 31) / 32)), 256, 0, st>>>(
+      reinterpret_cast<const uint32_t*>(as), M, ast, a_blocks, reinterpret_cast<const uint32_t*>(ws), N, wst, chunks);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   const int64_t m_chunk = (int64_t)(dma::MAX_RANGE / (uint64_t)lda) / lin::BM * lin::BM;
   const int64_t n_chunk = (int64_t)(dma::MAX_RANGE / (uint64_t)K) / lin::BN * lin::BN;
@@ -862,7 +950,7 @@ static hipError_t launch_linear_a8(const uint8_t* aq, const uint8_t* as, int64_t
     const int mc = (int)(M - m0 < m_chunk ? M - m0 : m_chunk);
     for (int64_t n0 = 0; n0 < N; n0 += n_chunk) {
       const int nc = (int)(N - n0 < n_chunk ? N - n0 : n_chunk);
-      const int tiles = ((mc + lin::BM - 1) / lin::BM) * ((nc + lin::BN - 1) / lin::BN);
+      const int tiles = ((mc + lin::BM - 1) / lin::BM) * ((nc + lin::BN - 1) / lin::BN) * slices;
       int grid = cus / 8 * 8 > 0 ? cus / 8 * 8 : 8;
       if (grid > (tiles + 7) / 8 * 8) grid = (tiles + 7) / 8 * 8;
       void* cp = OUT == 2 ? (void*)(static_cast<float*>(c) + m0 * ldc + n0)
@@ -872,26 +960,58 @@ static hipError_t launch_linear_a8(const uint8_t* aq, const uint8_t* as, int64_t
       const uint64_t ast_bytes = (uint64_t)((chunks - 1) * M + mc) * 4, wst_bytes = (uint64_t)((chunks - 1) * N + nc) * 4;
       mx_linear_a8_kernel<OUT><<<grid, lin::THREADS, 0, st>>>(
           aq + m0 * lda, lda, (uint32_t)(mc * lda), ast + m0, (uint32_t)ast_bytes, wq + n0 * K,
-          (uint32_t)(nc * K), wst + n0, (uint32_t)wst_bytes, cp, ldc, mc, nc, K, M, N);
+          (uint32_t)(nc * K), wst + n0, (uint32_t)wst_bytes, cp, ldc, mc, nc, K, M, N, slices, plane);
       if ((e = hipGetLastError()) != hipSuccess) return e;
     }
   }
   return hipSuccess;
 }
 
+// Whether the direct-load kernel takes these operands (else the register-
+// staged one), and whether one launch covers them.
+static bool takes_dma(int fmt, int64_t lda, const uint8_t* ws, int64_t KB) {
+  return KB % 128 == 0 && !kq_misaligned(ws, 4) && (uint64_t)lda * 2 * lin::BM <= dma::MAX_RANGE &&
+         (uint64_t)(fmt == 0 ? KB : KB / 2) * lin::BN <= dma::MAX_RANGE;
+}
+static bool one_range(int64_t lda_bytes, int64_t w_row_bytes, int64_t m, int64_t n) {
+  return (uint64_t)m * lda_bytes <= dma::MAX_RANGE && (uint64_t)n * w_row_bytes <= dma::MAX_RANGE;
+}
+
 template <int FMT, int OUT>
 static hipError_t launch_linear(const uint16_t* a, int64_t lda, const uint8_t* wq, const uint8_t* ws,
-                                void* c, int64_t ldc, int M, int N, int K, int KB, hipStream_t st) {
-  if (KB % 128 == 0 && !kq_misaligned(ws, 4) && (uint64_t)lda * 2 * lin::BM <= dma::MAX_RANGE &&
-      (uint64_t)(FMT == 0 ? KB : KB / 2) * lin::BN <= dma::MAX_RANGE)
-    return launch_linear_dma<FMT, OUT>(a, lda, wq, ws, c, ldc, M, N, K, KB, st);
+                                void* c, int64_t ldc, int M, int N, int K, int KB, hipStream_t st, int slices = 1,
+                                int64_t plane = 0) {
+  if (takes_dma(FMT, lda, ws, KB))
+    return launch_linear_dma<FMT, OUT>(a, lda, wq, ws, c, ldc, M, N, K, KB, st, slices, plane);
   const size_t lds = 2 * (size_t)lin::stage_bytes<FMT>();
   auto kern = mx_linear_kernel<FMT, OUT>;
   hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return e;
-  dim3 grid((N + lin::BN - 1) / lin::BN, (M + lin::BM - 1) / lin::BM);
-  kern<<<grid, lin::THREADS, lds, st>>>(a, lda, wq, ws, c, ldc, M, N, K, KB);
+  dim3 grid((N + lin::BN - 1) / lin::BN, (M + lin::BM - 1) / lin::BM, slices);
+  kern<<<grid, lin::THREADS, lds, st>>>(a, lda, wq, ws, c, ldc, M, N, K, KB, plane);
   return hipGetLastError();
+}
+
+// launch_linear, split over K into `planes` (plane_bytes of workspace) where
+// that pays and fits.
+template <int FMT, int OUT>
+static hipError_t launch_linear_split(const uint16_t* a, int64_t lda, const uint8_t* wq, const uint8_t* ws, void* c,
+                                      int64_t ldc, int M, int N, int K, int KB, void* planes, int64_t plane_bytes,
+                                      hipStream_t st) {
+  int cus = 0;
+  hipError_t e = stream_cus(st, &cus);
+  if (e != hipSuccess) return e;
+  const bool dma_path = takes_dma(FMT, lda, ws, KB);
+  const SplitPlan p = plan_split(M, N, K, dma_path ? DMA_STEP_US : STAGED_STEP_US, cus);
+  if (p.slices <= 1 || p.bytes > plane_bytes || !one_range(2 * lda, FMT == 0 ? KB : KB / 2, M, N))
+    return launch_linear<FMT, OUT>(a, lda, wq, ws, c, ldc, M, N, K, KB, st);
+  e = launch_linear<FMT, 2>(a, lda, wq, ws, planes, p.ldp, M, N, K, KB, st, p.slices, p.plane);
+  return e == hipSuccess ? sum_planes<OUT>(p, planes, M, N, c, ldc, st) : e;
+}
+
+static int current_cus() {
+  int cus = 0;
+  return stream_cus(nullptr, &cus) == hipSuccess ? cus : 0;
 }
 
 namespace kq {
@@ -926,17 +1046,35 @@ hipError_t split3_rows(const float* a, int64_t lda, int64_t m, int64_t k, uint16
 
 }  // namespace kq
 
-// Rows up to which the one-pass kernel of kq_skinny.hip takes the linear: a
-// 256 x 256 tile costs the same for 1 row as for 256 (N = 12288, K = 7168
-// E4M3: 137 us), the one-pass kernel 24 us at 1 row and 57 us at 64.
-constexpr int64_t SKINNY_MAX_ROWS = 64;
-static bool takes_skinny(int64_t m, int64_t k, const uint8_t* w_scale) {
-  return m <= SKINNY_MAX_ROWS && (k % 128 != 0 || !kq_misaligned(w_scale, 4));
+// Which linears take the one-pass kernel of kq_skinny.hip.  Up to 32 rows
+// always: a 256 x 256 tile costs the same for 1 row as for 256 (N = 12288, K =
+// 7168 E4M3: 137 us, the one-pass kernel 24 us at 1 row, 43 at 32; split over
+// K with its second launch ~45).  At 33 .. 64 rows the split product passes it
+// where K is long (K = 7168, N = 5000, 48 rows: 33 against 57 us) but not
+// where its two launches dominate (K = 1024: 15 against 21 us; fp32 rows, a
+// third launch, also at N <= 2048: 37 against 46 us), nor without a workspace
+// for its planes (137 us).
+static bool takes_skinny(int64_t m, int64_t n, int64_t k, bool f32_rows, const uint8_t* w_scale, bool planes_fit) {
+  if (k % 128 == 0 && kq_misaligned(w_scale, 4)) return false;
+  return m <= 32 || (m <= 64 && (k <= 2048 || (f32_rows && n <= 2048) || !planes_fit));
+}
+
+extern "C" int64_t kq_mx_linear_workspace_size(int64_t m, int64_t n, int64_t k) {
+  if (m < 0 || n < 0 || k <= 0) return -1;
+  const int cus = current_cus();
+  if (cus <= 0 || takes_skinny(m, n, k, false, nullptr, true)) return 0;
+  return plan_split(m, n, k, k % 128 ? STAGED_STEP_US : DMA_STEP_US, cus).bytes;
 }
 
 extern "C" int kq_mx_linear(int w_fmt, const void* a, int64_t lda, const void* w_q,
                             const uint8_t* w_scale, int64_t m, int64_t n, int64_t k,
                             int out_dtype, void* c, int64_t ldc, void* stream) {
+  return kq_mx_linear_ws(w_fmt, a, lda, w_q, w_scale, m, n, k, out_dtype, c, ldc, nullptr, 0, stream);
+}
+
+extern "C" int kq_mx_linear_ws(int w_fmt, const void* a, int64_t lda, const void* w_q, const uint8_t* w_scale,
+                               int64_t m, int64_t n, int64_t k, int out_dtype, void* c, int64_t ldc,
+                               void* workspace, int64_t workspace_bytes, void* stream) {
   if (w_fmt != KQ_FMT_MXFP8_E4M3 && w_fmt != KQ_FMT_MXFP4_E2M1)
     return kq_fail(KQ_ERR_INVALID, "kq_mx_linear: unknown weight format %d", w_fmt);
   if (out_dtype != KQ_DT_BF16 && out_dtype != KQ_DT_F32)
@@ -950,27 +1088,43 @@ extern "C" int kq_mx_linear(int w_fmt, const void* a, int64_t lda, const void* w
     return kq_fail(KQ_ERR_LIMIT, "kq_mx_linear: dimension too large");
   if (kq_misaligned(a, 16) || kq_misaligned(w_q, 16) || kq_misaligned(w_scale, 2))
     return kq_fail(KQ_ERR_INVALID, "kq_mx_linear: a and w_q must be 16-byte aligned");
+  if (kq_misaligned(workspace, 16))
+    return kq_fail(KQ_ERR_INVALID, "kq_mx_linear: workspace must be 16-byte aligned");
   if (m == 0 || n == 0) return KQ_OK;
+  if (!workspace) workspace_bytes = 0;
   hipStream_t st = (hipStream_t)stream;
   const uint16_t* ap = (const uint16_t*)a;
   const uint8_t* wp = (const uint8_t*)w_q;
   hipError_t e;
-  if (takes_skinny(m, k, w_scale))
+  if (takes_skinny(m, n, k, false, w_scale, workspace_bytes > 0))
     return kq_check_launch(mx_skinny_bf16(w_fmt, out_dtype == KQ_DT_F32,
                                           {a, nullptr, lda, wp, w_scale, c, ldc, (int)m, (int)n, (int)k}, st),
                            "kq_mx_linear");
+  auto split = [&](auto launch) {
+    return launch(ap, lda, wp, w_scale, c, ldc, (int)m, (int)n, (int)k, (int)k, workspace, workspace_bytes, st);
+  };
   if (w_fmt == KQ_FMT_MXFP8_E4M3)
-    e = out_dtype == KQ_DT_BF16 ? launch_linear<0, 0>(ap, lda, wp, w_scale, c, ldc, (int)m, (int)n, (int)k, (int)k, st)
-                                : launch_linear<0, 2>(ap, lda, wp, w_scale, c, ldc, (int)m, (int)n, (int)k, (int)k, st);
+    e = out_dtype == KQ_DT_BF16 ? split(launch_linear_split<0, 0>)
+                                : split(launch_linear_split<0, 2>);
   else
-    e = out_dtype == KQ_DT_BF16 ? launch_linear<1, 0>(ap, lda, wp, w_scale, c, ldc, (int)m, (int)n, (int)k, (int)k, st)
-                                : launch_linear<1, 2>(ap, lda, wp, w_scale, c, ldc, (int)m, (int)n, (int)k, (int)k, st);
+    e = out_dtype == KQ_DT_BF16 ? split(launch_linear_split<1, 0>)
+                                : split(launch_linear_split<1, 2>);
   return kq_check_launch(e, "kq_mx_linear");
 }
 
 extern "C" int64_t kq_mx_linear_f32_workspace_size(int64_t m, int64_t k) {
   if (m < 0 || k < 0) return -1;
   return m * 3 * k * 2;
+}
+
+// the split rows, then (on a 256-byte boundary) the K slices' planes
+static int64_t f32_planes_offset(int64_t m, int64_t k) { return (m * 3 * k * 2 + 255) / 256 * 256; }
+
+extern "C" int64_t kq_mx_linear_f32_split_workspace_size(int64_t m, int64_t n, int64_t k) {
+  if (m < 0 || n < 0 || k <= 0) return -1;
+  const int cus = current_cus();
+  if (cus <= 0 || takes_skinny(m, n, k, true, nullptr, true)) return m * 3 * k * 2;
+  return f32_planes_offset(m, k) + plan_split(m, n, 3 * k, k % 128 ? STAGED_STEP_US : DMA_STEP_US, cus).bytes;
 }
 
 extern "C" int kq_mx_linear_f32(int w_fmt, const float* a, int64_t lda, const void* w_q,
@@ -994,7 +1148,7 @@ extern "C" int kq_mx_linear_f32(int w_fmt, const float* a, int64_t lda, const vo
     return kq_fail(KQ_ERR_INVALID, "kq_mx_linear_f32: a, w_q and workspace must be 16-byte aligned");
   if (m == 0 || n == 0) return KQ_OK;
   hipStream_t st = (hipStream_t)stream;
-  if (takes_skinny(m, k, w_scale))
+  if (takes_skinny(m, n, k, true, w_scale, workspace_bytes > f32_planes_offset(m, k)))
     return kq_check_launch(mx_skinny_f32(w_fmt, {a, nullptr, lda, (const uint8_t*)w_q, w_scale, c, ldc, (int)m, (int)n,
                                                  (int)k}, st),
                            "kq_mx_linear_f32");
@@ -1003,10 +1157,10 @@ extern "C" int kq_mx_linear_f32(int w_fmt, const float* a, int64_t lda, const vo
   split3_bf16_kernel<<<(unsigned)((quads + 255) / 256), 256, 0, st>>>(a, lda, m, k, a3);
   if (int rc = kq_check_launch(hipGetLastError(), "kq_mx_linear_f32")) return rc;
   const uint8_t* wp = (const uint8_t*)w_q;
-  const hipError_t e =
-      w_fmt == KQ_FMT_MXFP8_E4M3
-          ? launch_linear<0, 2>(a3, 3 * k, wp, w_scale, c, ldc, (int)m, (int)n, (int)(3 * k), (int)k, st)
-          : launch_linear<1, 2>(a3, 3 * k, wp, w_scale, c, ldc, (int)m, (int)n, (int)(3 * k), (int)k, st);
+  const int64_t off = f32_planes_offset(m, k);
+  auto* launch = w_fmt == KQ_FMT_MXFP8_E4M3 ? launch_linear_split<0, 2> : launch_linear_split<1, 2>;
+  const hipError_t e = launch(a3, 3 * k, wp, w_scale, c, ldc, (int)m, (int)n, (int)(3 * k), (int)k,
+                              static_cast<char*>(workspace) + off, workspace_bytes > off ? workspace_bytes - off : 0, st);
   return kq_check_launch(e, "kq_mx_linear_f32");
 }
 
@@ -1028,9 +1182,15 @@ static int check_linear_mx(const char* fn, int a_fmt, int w_fmt, int64_t lda, in
   return KQ_OK;
 }
 
+static int64_t mx_scale_planes(int64_t m, int64_t n, int64_t k) {
+  return a8_scale_plane_bytes(m, k) + a8_scale_plane_bytes(n, k);
+}
+
 extern "C" int64_t kq_mx_linear_mx_workspace_size(int64_t m, int64_t n, int64_t k) {
   if (m < 0 || n < 0 || k <= 0) return -1;
-  return a8_scale_plane_bytes(m, k) + a8_scale_plane_bytes(n, k);
+  const int cus = current_cus();
+  if (cus <= 0 || takes_skinny(m, n, k, false, nullptr, true)) return mx_scale_planes(m, n, k);
+  return mx_scale_planes(m, n, k) + plan_split(m, n, k, A8_STEP_US, cus).bytes;
 }
 
 extern "C" int kq_mx_linear_mx(int a_fmt, const void* a_q, const uint8_t* a_scale, int64_t lda, int w_fmt,
@@ -1043,20 +1203,33 @@ extern "C" int kq_mx_linear_mx(int a_fmt, const void* a_q, const uint8_t* a_scal
   if (!a_q || !a_scale || !w_q || !w_scale || !c) return kq_fail(KQ_ERR_INVALID, "%s: null buffer", fn);
   if (kq_misaligned(a_q, 16) || kq_misaligned(w_q, 16) || kq_misaligned(a_scale, 4) || kq_misaligned(w_scale, 4))
     return kq_fail(KQ_ERR_INVALID, "%s: a_q and w_q must be 16-byte aligned, the scales 4-byte aligned", fn);
-  const int64_t need = kq_mx_linear_mx_workspace_size(m, n, k);
+  // the scale planes; the K split's planes are taken where they fit
+  const int64_t need = mx_scale_planes(m, n, k);
   if (!workspace || workspace_bytes < need || kq_misaligned(workspace, 256))
     return kq_fail(KQ_ERR_INVALID, "%s: workspace needs %lld bytes (256-byte aligned)", fn, (long long)need);
   hipStream_t st = (hipStream_t)stream;
   const uint8_t* ap = (const uint8_t*)a_q;
   const uint8_t* wp = (const uint8_t*)w_q;
-  if (m <= SKINNY_MAX_ROWS)
+  if (takes_skinny(m, n, k, false, w_scale, true))
     return kq_check_launch(mx_skinny_mx(out_dtype == KQ_DT_F32,
                                         {a_q, a_scale, lda, wp, w_scale, c, ldc, (int)m, (int)n, (int)k}, st),
                            fn);
-  const hipError_t e =
-      out_dtype == KQ_DT_BF16
-          ? launch_linear_a8<0>(ap, a_scale, lda, wp, w_scale, c, ldc, (int)m, (int)n, (int)k, workspace, st)
-          : launch_linear_a8<2>(ap, a_scale, lda, wp, w_scale, c, ldc, (int)m, (int)n, (int)k, workspace, st);
+  int cus = 0;
+  hipError_t e = stream_cus(st, &cus);
+  if (e != hipSuccess) return kq_check_launch(e, fn);
+  const SplitPlan p = plan_split(m, n, k, A8_STEP_US, cus);
+  if (p.slices > 1 && p.bytes <= workspace_bytes - need && one_range(lda, k, m, n)) {
+    void* planes = static_cast<char*>(workspace) + need;
+    e = launch_linear_a8<2>(ap, a_scale, lda, wp, w_scale, planes, p.ldp, (int)m, (int)n, (int)k, workspace, cus, st,
+                            p.slices, p.plane);
+    if (e == hipSuccess)
+      e = out_dtype == KQ_DT_BF16 ? sum_planes<0>(p, planes, (int)m, (int)n, c, ldc, st)
+                                  : sum_planes<2>(p, planes, (int)m, (int)n, c, ldc, st);
+  } else {
+    e = out_dtype == KQ_DT_BF16
+            ? launch_linear_a8<0>(ap, a_scale, lda, wp, w_scale, c, ldc, (int)m, (int)n, (int)k, workspace, cus, st)
+            : launch_linear_a8<2>(ap, a_scale, lda, wp, w_scale, c, ldc, (int)m, (int)n, (int)k, workspace, cus, st);
+  }
   return kq_check_launch(e, fn);
 }
 
@@ -1079,12 +1252,12 @@ extern "C" int kq_mx_linear_mm(int w_fmt, const void* a, int a_dtype, int64_t ld
   if (lda < k) return kq_fail(KQ_ERR_INVALID, "%s: lda < k", fn);
   if (int rc = check_linear_mx(fn, KQ_FMT_MXFP8_E4M3, w_fmt, k, m, n, k, out_dtype, ldc)) return rc;
   if (m == 0 || n == 0) return KQ_OK;
-  const int64_t need = kq_mx_linear_mm_workspace_size(m, n, k);
+  const int64_t need = mm_mx_offset(m, k) + mx_scale_planes(m, n, k);
   if (!workspace || workspace_bytes < need || kq_misaligned(workspace, 256))
     return kq_fail(KQ_ERR_INVALID, "%s: workspace needs %lld bytes (256-byte aligned)", fn, (long long)need);
   uint8_t* xq = static_cast<uint8_t*>(workspace);
   uint8_t* xs = xq + mm_scale_offset(m, k);
   if (int rc = kq_mx_quantize(KQ_FMT_MXFP8_E4M3, a_dtype, a, lda, m, k, xq, xs, 0, stream)) return rc;
   return kq_mx_linear_mx(KQ_FMT_MXFP8_E4M3, xq, xs, k, w_fmt, w_q, w_scale, m, n, k, out_dtype, c, ldc,
-                         xq + mm_mx_offset(m, k), need - mm_mx_offset(m, k), stream);
+                         xq + mm_mx_offset(m, k), workspace_bytes - mm_mx_offset(m, k), stream);
 }

@@ -58,15 +58,17 @@ def _linear(fmt: int, source: torch.Tensor, weight: torch.Tensor, scale: torch.T
     m = a.shape[0]
     if exact_f32:
         out = torch.empty(m, n, dtype=torch.float32, device=gpu)
-        ws = torch.empty(max(int(N.library().kq_mx_linear_f32_workspace_size(m, k)), 16),
+        ws = torch.empty(max(int(N.library().kq_mx_linear_f32_split_workspace_size(m, n, k)), 16),
                          dtype=torch.uint8, device=gpu)
         N.call("kq_mx_linear_f32", fmt, N.ptr(a), k, N.ptr(w), N.ptr(s), m, n, k, N.ptr(out), n,
                N.ptr(ws), ws.numel(), N.stream(gpu))
         out = out.to(out_dtype)
     else:
         out = torch.empty(m, n, dtype=out_dtype, device=gpu)
-        N.call("kq_mx_linear", fmt, N.ptr(a), k, N.ptr(w), N.ptr(s), m, n, k,
-               N.DTYPE_CODES[out_dtype], N.ptr(out), n, N.stream(gpu))
+        need = int(N.library().kq_mx_linear_workspace_size(m, n, k))
+        ws = torch.empty(need, dtype=torch.uint8, device=gpu) if need > 0 else None  # a K split's planes
+        N.call("kq_mx_linear_ws", fmt, N.ptr(a), k, N.ptr(w), N.ptr(s), m, n, k,
+               N.DTYPE_CODES[out_dtype], N.ptr(out), n, N.ptr(ws), max(need, 0), N.stream(gpu))
     out = out.reshape(*lead, n)
     return out if host is None else out.to(host)
 

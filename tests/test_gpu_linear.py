@@ -275,3 +275,42 @@ def test_few_rows_extreme_scales(gpu, a_byte, w_byte):
         return (v * torch.exp2(s.double() - 127)[..., None]).reshape(q.shape).numpy()
 
     assert _max_rel(values(aq, a_s) @ values(wq, w_s).T, c.cpu().numpy()) <= 3e-5
+
+
+@pytest.mark.parametrize("m,n,k", [(33, 130, 2176), (64, 8200, 4224), (65, 70, 4160), (257, 300, 1024), (300, 515, 2112),
+                                   (777, 1030, 3200)])
+@pytest.mark.parametrize("form", ["bf16-mxfp8", "bf16-mxfp4", "f32-mxfp8", "mx-mxfp8"])
+def test_split_k(gpu, form, m, n, k):
+    """Shapes of few tiles run K in slices (ragged rows and columns, odd N,
+    K % 128 == 64 on the register-staged kernel, slices of unequal steps):
+    fp32 output against float64 within the fp32 sums' 1e-5 (MXFP8 x MXFP8:
+    the matrix cores' 64-product sums, 5e-5), bf16 output within one ulp; the
+    unsplit call without a workspace agrees to fp32 summation order."""
+    dtype, fmt = form.split("-")
+    if dtype == "mx" and k % 128:
+        pytest.skip("MXFP8 rows take K % 128 == 0")
+    g = torch.Generator().manual_seed(m + n + k)
+    w = (torch.randn(n, k, generator=g) * 0.02).to(torch.bfloat16).to(gpu)
+    x = torch.randn(m, k, generator=g) * torch.exp(0.5 * torch.randn(k, generator=g))
+    x = x if dtype == "f32" else x.to(torch.bfloat16)
+    q, s, wd = _quantized(fmt, w)
+    if dtype == "mx":
+        xq, xs = mxfp8.mxfp8_quantize(x.to(gpu))
+        xv = oracle.mx_dequant("mxfp8", xq.view(torch.uint8).cpu().numpy(), xs.cpu().numpy()).astype(np.float64)
+        run = lambda out: linear.mxfp8_linear_mx(xq, xs, q, s, out_dtype=out)  # noqa: E731
+    else:
+        xv = x.double().numpy()
+        fn = linear.mxfp8_linear if fmt == "mxfp8" else linear.mxfp4_linear
+        run = lambda out: fn(x.to(gpu), q, s, out_dtype=out)  # noqa: E731
+    ref = xv @ wd.astype(np.float64).T
+    c = run(torch.float32)
+    assert _max_rel(ref, c.cpu().numpy()) <= (5e-5 if dtype == "mx" else 1e-5)
+    assert torch.equal(c, run(torch.float32))  # slices are summed in order
+    if dtype == "bf16":
+        check_bf16_output(ref, run(torch.bfloat16).float().cpu().numpy())
+        from kquant_amd import _native as N
+        plain = torch.empty(m, n, dtype=torch.float32, device=gpu)
+        xg, qg = x.to(gpu), q.view(torch.uint8)
+        N.call("kq_mx_linear", N.FMT_MXFP8_E4M3 if fmt == "mxfp8" else N.FMT_MXFP4_E2M1, N.ptr(xg), k, N.ptr(qg),
+               N.ptr(s), m, n, k, N.DT_F32, N.ptr(plain), n, N.stream(gpu))
+        assert _max_rel(ref, plain.cpu().numpy()) <= 1e-5
