@@ -13,16 +13,15 @@
 //    or columns in LDS (adds only), then one scale (1/128 exactly for both
 //    sides, fl(1/sqrt(128)) for one).
 //  * Cholesky (lower, fp32): blocked over 64-column panels grouped into
-//    super-panels (four panels for batches of 8 and more, else one), all
-//    matrices of a batch per launch.  Within a super-panel one launch per
+//    super-panels (two to eight panels), all matrices of a batch per launch.  Within a super-panel one launch per
 //    panel brings its block column up to date with the super-panel's earlier
-//    panels and computes the panel below the diagonal as A21 inv(L11)^T;
-//    diagonal blocks are factored and inverted by one wave in registers, by
-//    the workgroup that completes them.  One update A22 -= L21 L21^T over
-//    the super-panel's columns then covers the trailing matrix.  Products on
+//    panels, factors and inverts the diagonal block in the workgroup that
+//    completes it, and computes the panel below as A21 inv(L11)^T; the first
+//    launch of the next super-panel also applies A22 -= L21 L21^T over the
+//    super-panel's columns to the whole trailing matrix.  Products on
 //    v_mfma_f32_16x16x4f32 from LDS.  A failing pivot (<= 0 or NaN) records
-//    the leading-minor order in info (LAPACK's convention) and the
-//    factorization continues with pivot 1, so every launch still completes.
+//    the leading-minor order in info (LAPACK's convention) and leaves NaN
+//    behind it; every launch still completes.
 //  * block LDL: every b x b diagonal block DL_i of L is inverted, each block
 //    column multiplied by its inverse and the diagonal blocks set to I.
 #include "kq_dma.h"
@@ -160,140 +159,147 @@ __device__ __forceinline__ float readlane_f(float v, int lane) {
 
 // The workgroup's 256 threads (4 waves) factor the 64 x 64 block a (LDS;
 // rows past the matrix padded with the identity) into L, written back to a
-// with zeros above the diagonal, and write inv(L) to xi.  By 16-column
-// panels, right-looking; per panel:
-//  * wave 0 factors the 16 x 16 diagonal block: lane r holds row r, column
-//    c is broadcast from lane c with readlane, and each step takes the
+// with zeros above the diagonal, and write inv(L) to xi.  This is the serial
+// chain of the whole factorization (a panel's launch cannot start before its
+// diagonal block is done), so what counts is its length in cycles.  By
+// 16-column panels, right-looking; per panel:
+//  * wave 0 eliminates the 16 x 16 diagonal block and the identity's columns
+//    at once: lane r holds row r (by symmetry column r) of the block, lane
+//    16 + c column c of the identity, and step j scales entry j by the
 //    pivot's reciprocal square root (hardware v_rsq: within an ulp or two,
-//    far inside the factorization's own rounding), scales the column by it
-//    and updates the trailing columns with one FMA per entry; then lane j
-//    solves column j of the block's inverse X by forward substitution, the
-//    rows of L broadcast the same way;
+//    far inside the factorization's own rounding) and subtracts L[r][j]
+//    (broadcast from lane r with readlane) times it from entry r > j.  The
+//    identity's columns become the block's inverse X without a step of their
+//    own.
 //  * the rows below take L21 = A21 X^T and the trailing lower tiles
 //    A22 -= L21 L21^T, both on v_mfma_f32_16x16x4f32, a 16 x 16 tile per
 //    wave.
 // The off-diagonal blocks of inv(L) follow by block rows i = 1, 2, 3:
 // X[i][j] = -X[i][i] (sum over k = j .. i - 1 of L[i][k] X[k][j]) on the
-// MFMAs, one block per wave; rows 1 and 2 on waves 1 .. i while wave 0
-// factors the next diagonal block, row 3 after the last one.  Returns (uniformly) the first failing
-// column + 1, or 0; a failing pivot is replaced by 1.  Ends with a barrier:
-// a and xi are complete for every thread.
+// MFMAs, one block per wave: rows 1 and 2, and the sums of row 3, on two of
+// the idle waves during the later eliminations.  Loading, factoring and
+// storing one block takes 18 us against 25 with the inverses solved after the
+// blocks by one wave; with the wider super-panels of kq_cholesky 16 matrices
+// of n = 2048 went from 2,100 to 1,355 us (block LDL included), one of n =
+// 7168 from 4,820 to 3,685.
+// Returns (uniformly) the first failing column + 1, or 0 (a failing pivot
+// leaves NaN in the rest of the factor).  Ends with a barrier: a and xi are
+// complete for every thread.
 __device__ __forceinline__ int factor64_wg(float (*a)[LD], float (*xi)[LD]) {
   constexpr int PB = 16;  // panel width
   __shared__ float tb[3][PB][PB + 1];
-  __shared__ float dg[2][PB];  // L[c][c] and 1 / L[c][c] of the current diagonal block
   __shared__ int s_bad;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int li = lane & 15, lk = lane >> 4;  // v_mfma_f32_16x16x4f32 operand position
-  // block (i, j) of inv(L), j < i, on the calling wave: X[i][j] = -X[i][i] T with
-  // T = sum over k = j .. i - 1 of L[i][k] X[k][j]
-  auto inv_block = [&](int i, int j) {
-    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-    for (int k = j; k < i; ++k) {
+  // acc += the 16 x 16 block of M at (r, c) times B, whose row k column li is b(k), in k
+  // order: rows of L and X end in their largest entry, and added last it rounds once
+  auto mul = [&](f32x4_t& acc, const float (*M)[LD], int r, int c, auto b) {
+    float m[4], v[4];
 #pragma unroll
-      for (int u = 0; u < PB; u += 4)
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[PB * i + li][PB * k + u + lk], xi[PB * k + u + lk][PB * j + li],
-                                                   acc, 0, 0, 0);
+    for (int e = 0; e < 4; ++e) {
+      m[e] = M[r + li][c + 4 * e + lk];
+      v[e] = b(4 * e + lk);
     }
 #pragma unroll
-    for (int q = 0; q < 4; ++q) tb[j][4 * lk + q][li] = acc[q];
-    // one wave's LDS accesses complete in order: the T it stored is read back below
-    f32x4_t x = {0.f, 0.f, 0.f, 0.f};
+    for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(m[e], v[e], acc, 0, 0, 0);
+  };
+  // tb[j] = sum over k = j .. i - 1 of L[i][k] X[k][j] (X = inv(L), 16 x 16 blocks)
+  auto inv_sum = [&](int i, int j) {
+    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+    for (int k = j; k < i; ++k)
+      mul(acc, a, PB * i, PB * k, [&](int kk) { return xi[PB * k + kk][PB * j + li]; });
 #pragma unroll
-    for (int u = 0; u < PB; u += 4)
-      x = __builtin_amdgcn_mfma_f32_16x16x4f32(xi[PB * i + li][PB * i + u + lk], tb[j][u + lk][li], x, 0, 0, 0);
+    for (int q = 0; q < 4; ++q) tb[j][4 * lk + q][li] = acc[q];
+  };
+  // X[i][j] = -X[i][i] tb[j] (one wave's LDS accesses complete in order)
+  auto inv_block = [&](int i, int j) {
+    f32x4_t x = {0.f, 0.f, 0.f, 0.f};
+    mul(x, xi, PB * i, PB * i, [&](int kk) { return tb[j][kk][li]; });
 #pragma unroll
     for (int q = 0; q < 4; ++q) xi[PB * i + 4 * lk + q][PB * j + li] = -x[q];
   };
   if (tid == 0) s_bad = 0;
-  // zeros above the diagonal blocks of xi (the blocks themselves are written whole)
-  for (int e = tid; e < NB * NB; e += 256) {
-    const int rr = e / NB, cc = e % NB;
-    if ((cc >> 4) > (rr >> 4)) xi[rr][cc] = 0.f;
+  // the diagonal blocks symmetric, zeros in the blocks above them (and of inv(L))
+  {
+    const int r = tid >> 4, c = tid & 15;
+#pragma unroll
+    for (int d = 0; d < NB; d += PB)
+      if (c > r) a[d + r][d + c] = a[d + c][d + r];
+#pragma unroll
+    for (int d = 0; d < NB; d += PB)
+#pragma unroll
+      for (int q = d + PB; q < NB; q += PB) {
+        a[d + r][q + c] = 0.f;
+        xi[d + r][q + c] = 0.f;
+      }
   }
   __syncthreads();
+#pragma unroll
   for (int p = 0; p < NB / PB; ++p) {
     const int c0 = PB * p;
+    const int nt = NB / PB - 1 - p;
     if (wave == 0) {
       float v[PB];
+      const float* row = a[c0 + li] + c0;
 #pragma unroll
-      for (int c = 0; c < PB; ++c) v[c] = a[c0 + li][c0 + c];
-      int bad = 0;
+      for (int c = 0; c < PB; c += 4) {
+        const f32x4_t q = *reinterpret_cast<const f32x4_t*>(row + c);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[c + e] = lk == 0 ? q[e] : (c + e == li ? 1.f : 0.f);
+      }
+      uint32_t failed = 0;  // a failing pivot leaves NaN behind it, so the first one counts
 #pragma unroll
       for (int c = 0; c < PB; ++c) {
-        float d = readlane_f(v[c], c);
-        if (!(d > 0.f)) {
-          if (bad == 0) bad = c0 + c + 1;
-          d = 1.f;
+        const float d = readlane_f(v[c], c);
+        v[c] *= __builtin_amdgcn_rsqf(d);  // L[r][c]; in the diagonal's lane d / sqrt(d)
+#pragma unroll
+        for (int q = c + 1; q < PB; ++q) v[q] = fmaf(-readlane_f(v[c], q), v[c], v[q]);
+        failed |= (uint32_t)!(d > 0.f) << c;
+      }
+      if (lane == 0 && failed != 0 && s_bad == 0) s_bad = c0 + __builtin_ctz(failed) + 1;
+      if (lk == 0) {
+#pragma unroll
+        for (int c = 0; c < PB; c += 4) {
+          f32x4_t q;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) q[e] = c + e <= li ? v[c + e] : 0.f;
+          *reinterpret_cast<f32x4_t*>(&a[c0 + li][c0 + c]) = q;
         }
-        const float rs = __builtin_amdgcn_rsqf(d);  // 1 / L[c][c]
-        dg[0][c] = d * rs;                          // L[c][c] (every lane stores the same value)
-        dg[1][c] = rs;
-        v[c] *= rs;  // L[r][c] for r > c (row c's diagonal is in dg)
+      } else if (lk == 1) {
 #pragma unroll
-        for (int q = c + 1; q < PB; ++q) v[q] = fmaf(-v[c], readlane_f(v[c], q), v[q]);
+        for (int c = 0; c < PB; ++c) xi[c0 + c][c0 + li] = v[c];
       }
-      if (lane < PB) {
-        const float dv = dg[0][li];
-#pragma unroll
-        for (int c = 0; c < PB; ++c) a[c0 + li][c0 + c] = c < li ? v[c] : (c == li ? dv : 0.f);
-      }
-      // column li of the block's inverse: x[i] = (delta - sum_{k<i} L[i][k] x[k]) / L[i][i]
-      float x[PB];
-#pragma unroll
-      for (int i = 0; i < PB; ++i) {
-        float acc = i == li ? 1.f : 0.f;
-#pragma unroll
-        for (int k = 0; k < i; ++k) acc = fmaf(-readlane_f(v[k], i), x[k], acc);
-        x[i] = acc * dg[1][i];
-      }
-      if (lane < PB) {
-#pragma unroll
-        for (int i = 0; i < PB; ++i) xi[c0 + i][c0 + li] = x[i];
-      }
-      if (lane == 0 && bad != 0 && s_bad == 0) s_bad = bad;
-    } else if (p >= 2 && wave < p) {
-      // meanwhile block row p - 1 of inv(L): its L blocks and X[p - 1][p - 1] are done
-      inv_block(p - 1, wave - 1);
+    } else if (p == 2 && wave == 2) {
+      inv_sum(1, 0);
+      inv_block(1, 0);
+    } else if (p == 3 && wave >= 2) {
+      inv_sum(2, wave - 2);
+      inv_block(2, wave - 2);
+      inv_sum(3, wave - 2);
+      if (wave == 3) inv_sum(3, 2);
     }
     __syncthreads();
-    // the panel below: L21 = A21 X^T, row tile w (rows c0 + 16 (1 + w) ..) on wave w
-    const int nt = NB / PB - 1 - p;
-    f32x4_t l21 = {0.f, 0.f, 0.f, 0.f};
+    if (!nt) break;
+    // the rows below: L21 = A21 X^T, each wave its own 16 rows
     if (wave < nt) {
       const int r0 = c0 + PB * (1 + wave);
+      f32x4_t l21 = {0.f, 0.f, 0.f, 0.f};
+      mul(l21, a, r0, c0, [&](int kk) { return xi[c0 + li][c0 + kk]; });
 #pragma unroll
-      for (int k = 0; k < PB; k += 4)
-        l21 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[r0 + li][c0 + k + lk], xi[c0 + li][c0 + k + lk], l21, 0, 0,
-                                                   0);
-    }
-    __syncthreads();  // every wave has read A21
-    if (wave < nt) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) a[c0 + PB * (1 + wave) + 4 * lk + j][c0 + li] = l21[j];
+      for (int j = 0; j < 4; ++j) a[r0 + 4 * lk + j][c0 + li] = l21[j];
     }
     __syncthreads();
     // trailing lower tiles (ti >= tj) -= L21[ti] L21[tj]^T
     for (int t = wave; t < nt * (nt + 1) / 2; t += 4) {
-      int ti = 0;
-      while ((ti + 1) * (ti + 2) / 2 <= t) ++ti;
-      const int tj = t - ti * (ti + 1) / 2;
+      const int ti = t < 1 ? 0 : t < 3 ? 1 : 2, tj = t - ti * (ti + 1) / 2;
       const int r0 = c0 + PB * (1 + ti), q0 = c0 + PB * (1 + tj);
-      f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int k = 0; k < PB; k += 4)
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[r0 + li][c0 + k + lk], a[q0 + li][c0 + k + lk], acc, 0, 0, 0);
+      f32x4_t acc = {0.f, 0.f, 0.f, 0.f};  // the products alone: subtracted once, as one rounding
+      mul(acc, a, r0, c0, [&](int kk) { return a[q0 + li][c0 + kk]; });
 #pragma unroll
       for (int j = 0; j < 4; ++j) a[r0 + 4 * lk + j][q0 + li] -= acc[j];
     }
     __syncthreads();
   }
-  // zeros above the diagonal of L (the diagonal blocks' upper parts are zero already)
-  for (int e = tid; e < NB * NB; e += 256) {
-    const int rr = e / NB, cc = e % NB;
-    if ((cc >> 4) > (rr >> 4)) a[rr][cc] = 0.f;
-  }
-  // the last block row of inv(L)
   if (wave < NB / PB - 1) inv_block(NB / PB - 1, wave);
   __syncthreads();
   return s_bad;
@@ -314,18 +320,32 @@ __device__ __forceinline__ void store_diag_wg(float (*a)[LD], float (*xi)[LD], f
   if (threadIdx.x == 0 && bad != 0 && *info == 0) *info = (int)(c0 + bad);
 }
 
-// L = tril(A) (upper part zero); info = 0.  a and l may be the same buffer.
+// L = tril(A) (upper part zero); info = 0.  a and l may be the same buffer
+// (then only the upper part is written).  Four columns per thread; VEC: rows
+// of both are 16-byte aligned and n % 4 == 0.
+template <bool VEC>
 __global__ __launch_bounds__(256) void chol_init_kernel(const float* a, int64_t lda, int64_t sa, float* l,
                                                         int64_t ldl, int64_t sl, int64_t n, int* __restrict__ info,
                                                         int* __restrict__ diag_done) {
-  const int64_t b = blockIdx.z, i = blockIdx.y, j = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t b = blockIdx.z, i = blockIdx.y, j = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
   if (i == 0 && j == 0) {
     info[b] = 0;
     diag_done[b] = -1;
   }
-  if (j >= n) return;
-  const float v = j <= i ? a[b * sa + i * lda + j] : 0.f;
-  l[b * sl + i * ldl + j] = v;
+  if (j >= n || (a == l && j + 3 <= i)) return;
+  const float* src = a + b * sa + i * lda + j;
+  float* dst = l + b * sl + i * ldl + j;
+  if (VEC) {
+    f32x4_t v = {0.f, 0.f, 0.f, 0.f};
+    if (j <= i) v = *reinterpret_cast<const f32x4_t*>(src);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = j + e <= i ? v[e] : 0.f;
+    *reinterpret_cast<f32x4_t*>(dst) = v;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (j + e < n) dst[e] = j + e <= i ? src[e] : 0.f;
+  }
 }
 
 // inv(L11) of panel p lives in slot p % 2 of the matrix's two winv slots
@@ -337,8 +357,8 @@ __global__ __launch_bounds__(256) void chol_init_kernel(const float* a, int64_t 
 // writing L11 back (zeros above its diagonal) and inv(L11) to slot 0.
 __global__ __launch_bounds__(256) void chol_diag_kernel(float* __restrict__ l, int64_t n, int64_t ldl, int64_t sl,
                                                         float* __restrict__ winv, int* __restrict__ info) {
-  __shared__ float a[NB][LD];
-  __shared__ float xi[NB][LD];
+  __shared__ __attribute__((aligned(16))) float a[NB][LD];
+  __shared__ __attribute__((aligned(16))) float xi[NB][LD];
   const int64_t b = blockIdx.x;
   float* L = l + b * sl;
   const int nb = (int)(n < NB ? n : NB);
@@ -354,19 +374,38 @@ __global__ __launch_bounds__(256) void chol_diag_kernel(float* __restrict__ l, i
 // acc (this wave's 32x32 of a 64x64 tile, as 2x2 16x16 blocks) += X Y^T over
 // k < NB, X and Y row-major in LDS.  v_mfma_f32_16x16x4f32: lane l gives
 // A[l % 16][l / 16] and B[l / 16][l % 16]; D block rows 4 (l / 16) + j,
-// column l % 16.
+// column l % 16.  ORDERED sums in k order, for a Y whose rows end in their
+// largest entry (inv(L): added last it rounds once; another order loses 3 %
+// of the factor's accuracy); otherwise a lane reads its k values 16 bytes at
+// a time and MFMA e of a 16-wide block sums k0 + 4 (l / 16) + e.
+template <bool ORDERED = false>
 __device__ __forceinline__ void mm_nt(const float (*X)[LD], const float (*Y)[LD], f32x4_t acc[2][2]) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int rb = 32 * (wave >> 1), cb = 32 * (wave & 1);
   const int li = lane & 15, lk = lane >> 4;
-#pragma unroll 4
-  for (int k = 0; k < NB; k += 4) {
-    const float a0 = X[rb + li][k + lk], a1 = X[rb + 16 + li][k + lk];
-    const float b0 = Y[cb + li][k + lk], b1 = Y[cb + 16 + li][k + lk];
-    acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, b0, acc[0][0], 0, 0, 0);
-    acc[0][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, b1, acc[0][1], 0, 0, 0);
-    acc[1][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, b0, acc[1][0], 0, 0, 0);
-    acc[1][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, b1, acc[1][1], 0, 0, 0);
+#pragma unroll
+  for (int k0 = 0; k0 < NB; k0 += 16) {
+    f32x4_t x[2], y[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if constexpr (ORDERED) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          x[h][e] = X[rb + 16 * h + li][k0 + 4 * e + lk];
+          y[h][e] = Y[cb + 16 * h + li][k0 + 4 * e + lk];
+        }
+      } else {
+        x[h] = *reinterpret_cast<const f32x4_t*>(&X[rb + 16 * h + li][k0 + 4 * lk]);
+        y[h] = *reinterpret_cast<const f32x4_t*>(&Y[cb + 16 * h + li][k0 + 4 * lk]);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i][e], y[j][e], acc[i][j], 0, 0, 0);
   }
 }
 
@@ -375,14 +414,12 @@ __device__ __forceinline__ void mm_nt(const float (*X)[LD], const float (*Y)[LD]
 __device__ __forceinline__ void load_tile(float (*T)[LD], const float* M, int64_t ld, int64_t n, int64_t r0,
                                           int64_t c0) {
   if (c0 + NB <= n && ld % 4 == 0 && (reinterpret_cast<uintptr_t>(M) & 15) == 0) {
-    for (int i = threadIdx.x; i < NB * NB / 4; i += 256) {
-      const int r = i / (NB / 4), c = 4 * (i % (NB / 4));
+#pragma unroll
+    for (int u = 0; u < NB * NB / 4 / 256; ++u) {
+      const int i = (int)threadIdx.x + 256 * u, r = i / (NB / 4), c = 4 * (i % (NB / 4));
       f32x4_t v = {0.f, 0.f, 0.f, 0.f};
       if (r0 + r < n) v = *reinterpret_cast<const f32x4_t*>(M + (r0 + r) * ld + c0 + c);
-      T[r][c] = v[0];
-      T[r][c + 1] = v[1];
-      T[r][c + 2] = v[2];
-      T[r][c + 3] = v[3];
+      *reinterpret_cast<f32x4_t*>(&T[r][c]) = v;
     }
     return;
   }
@@ -399,46 +436,19 @@ __device__ __forceinline__ void mm_pos(int bi, int bj, int q, int& r, int& c) {
   c = 32 * (wave & 1) + 16 * bj + (lane & 15);
 }
 
-// Panel p of the super-panel [s0, s1), row block i = p + 1 + blockIdx.x:
-// A[i, p] -= sum over q in [s0, p) of L[i, q] L[p, q]^T (the updates of the
-// super-panel's earlier panels, left-looking), then L[i, p] = A[i, p]
-// inv(L[p, p])^T.  The workgroup of row block p + 1, when that is still in
-// the super-panel, then brings the diagonal block (p + 1, p + 1) up to date
-// with panels s0 .. p and factors it.
-__global__ __launch_bounds__(256) void chol_panel_kernel(float* __restrict__ l, int64_t n, int64_t ldl, int64_t sl,
-                                                         int p, int s0, int s1, float* __restrict__ winv,
-                                                         int* __restrict__ info) {
-  __shared__ float av[NB][LD];
-  __shared__ float xi[NB][LD];
-  __shared__ float xj[NB][LD];
+// Panel 0, row block 1 + blockIdx.x: L[i, 0] = A[i, 0] inv(L[0, 0])^T.
+__global__ __launch_bounds__(256) void chol_panel0_kernel(float* __restrict__ l, int64_t n, int64_t ldl, int64_t sl,
+                                                          const float* __restrict__ winv) {
+  __shared__ __attribute__((aligned(16))) float av[NB][LD];
+  __shared__ __attribute__((aligned(16))) float xi[NB][LD];
   const int64_t b = blockIdx.y;
   float* L = l + b * sl;
-  const int64_t r0 = (int64_t)(p + 1 + blockIdx.x) * NB, c0 = (int64_t)p * NB;
-  f32x4_t acc[2][2] = {};
-  for (int q = s0; q < p; ++q) {
-    if (q > s0) __syncthreads();
-    load_tile(xi, L, ldl, n, r0, (int64_t)q * NB);
-    load_tile(xj, L, ldl, n, c0, (int64_t)q * NB);
-    __syncthreads();
-    mm_nt(xi, xj, acc);
-  }
-  load_tile(av, L, ldl, n, r0, c0);
-  const float* W = winv + (b * 2 + (p & 1)) * NB * NB;
-  __syncthreads();  // every wave is done with xi / xj; av is loaded
-  for (int i = threadIdx.x; i < NB * NB; i += 256) xi[i / NB][i % NB] = W[i];
-#pragma unroll
-  for (int bi = 0; bi < 2; ++bi)
-#pragma unroll
-    for (int bj = 0; bj < 2; ++bj)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        int r, c;
-        mm_pos(bi, bj, q, r, c);
-        av[r][c] -= acc[bi][bj][q];
-      }
+  const int64_t r0 = (int64_t)(1 + blockIdx.x) * NB;
+  load_tile(av, L, ldl, n, r0, 0);
+  load_tile(xi, winv + b * 2 * NB * NB, NB, NB, 0, 0);
   __syncthreads();
   f32x4_t lp[2][2] = {};
-  mm_nt(av, xi, lp);
+  mm_nt<true>(av, xi, lp);
 #pragma unroll
   for (int bi = 0; bi < 2; ++bi)
 #pragma unroll
@@ -447,47 +457,8 @@ __global__ __launch_bounds__(256) void chol_panel_kernel(float* __restrict__ l, 
       for (int q = 0; q < 4; ++q) {
         int r, c;
         mm_pos(bi, bj, q, r, c);
-        if (r0 + r < n && c0 + c < n) L[(r0 + r) * ldl + c0 + c] = lp[bi][bj][q];
+        if (r0 + r < n && c < n) L[(r0 + r) * ldl + c] = lp[bi][bj][q];
       }
-  if (blockIdx.x != 0 || p + 1 >= s1) return;
-  // diagonal block p + 1: A[p + 1, p + 1] -= sum over q in [s0, p] of
-  // L[p + 1, q] L[p + 1, q]^T, where L[p + 1, p] is this workgroup's lp
-  __syncthreads();  // every wave is done reading av / xi
-#pragma unroll
-  for (int bi = 0; bi < 2; ++bi)
-#pragma unroll
-    for (int bj = 0; bj < 2; ++bj)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        int r, c;
-        mm_pos(bi, bj, q, r, c);
-        av[r][c] = lp[bi][bj][q];  // rows past n are zero (their A rows are)
-      }
-  __syncthreads();
-  f32x4_t dg[2][2] = {};
-  mm_nt(av, av, dg);
-  for (int q = s0; q < p; ++q) {
-    __syncthreads();
-    load_tile(xi, L, ldl, n, r0, (int64_t)q * NB);
-    __syncthreads();
-    mm_nt(xi, xi, dg);
-  }
-  __syncthreads();
-  const int wave = threadIdx.x >> 6;
-#pragma unroll
-  for (int bi = 0; bi < 2; ++bi)
-#pragma unroll
-    for (int bj = 0; bj < 2; ++bj)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        int r, c;
-        mm_pos(bi, bj, q, r, c);
-        xi[r][c] = (r0 + r < n && r0 + c < n) ? L[(r0 + r) * ldl + r0 + c] - dg[bi][bj][q] : (r == c ? 1.f : 0.f);
-      }
-  __syncthreads();
-  const int bad = factor64_wg(xi, xj);
-  const int nb = (int)(n - r0 < NB ? n - r0 : NB);
-  store_diag_wg(xi, xj, L, ldl, r0, nb, winv + (b * 2 + ((p + 1) & 1)) * NB * NB, bad, info + b);
 }
 
 // Trailing update A[bi, bj] -= sum over panels q in [q0, q1) of
@@ -544,7 +515,20 @@ __global__ __launch_bounds__(256, DMA ? 2 : 4) void chol_update_kernel(float* __
         const int64_t r = ri + lr, c = rj + lc;
         av[bi][bj][q] = r < n && c < n ? L[r * ldl + c] : 0.f;
       }
+  // A -= two panels' products at a time, whatever the super-panel: longer sums
+  // round more often (n = 2048, 8 panels: 24 % more error in the factor than
+  // with 2), and so do more subtractions (n = 4096, one panel: 14 % more)
   f32x4_t acc[2][2] = {};
+  auto subtract = [&]() {
+#pragma unroll
+    for (int bi = 0; bi < 2; ++bi)
+#pragma unroll
+      for (int bj = 0; bj < 2; ++bj) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) av[bi][bj][q] -= acc[bi][bj][q];
+        acc[bi][bj] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      }
+  };
   if constexpr (DMA) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const uint32_t lds0 = dma::lds_offset_of(ring);
@@ -590,6 +574,7 @@ __global__ __launch_bounds__(256, DMA ? 2 : 4) void chol_update_kernel(float* __
           acc[1][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1[e], b1v[e], acc[1][1], 0, 0, 0);
         }
       }
+      if ((q & 1) || q + 1 == q1) subtract();
       if (q + 2 < q1) {
         __syncthreads();  // every wave is done reading the slot
         issue(q + 2, slot);
@@ -602,10 +587,11 @@ __global__ __launch_bounds__(256, DMA ? 2 : 4) void chol_update_kernel(float* __
       load_tile(xj, L, ldl, n, rj, (int64_t)q * NB);
       __syncthreads();
       mm_nt(xi, xj, acc);
+      if ((q & 1) || q + 1 == q1) subtract();
     }
   }
   const bool next_diag = t == 0;  // tile (b0, b0): panel b0's diagonal block
-  const bool panel = diag_done != nullptr && j == 0 && i > 0;  // fused: a tile of panel b0 below it
+  const bool panel = j == 0 && i > 0;  // a tile of panel b0 below it
   if (next_diag || panel) __syncthreads();  // every wave is done reading the tiles xi / xj alias
 #pragma unroll
   for (int bi = 0; bi < 2; ++bi)
@@ -617,7 +603,7 @@ __global__ __launch_bounds__(256, DMA ? 2 : 4) void chol_update_kernel(float* __
         mm_pos(bi, bj, q, lr, lc);
         const int64_t r = ri + lr, c = rj + lc;
         if (r < n && c < n) {
-          const float v = av[bi][bj][q] - acc[bi][bj][q];
+          const float v = av[bi][bj][q];
           if (next_diag || panel) xi[lr][lc] = v;
           else L[r * ldl + c] = v;
         } else if (next_diag) {
@@ -631,15 +617,11 @@ __global__ __launch_bounds__(256, DMA ? 2 : 4) void chol_update_kernel(float* __
     __syncthreads();
     const int bad = factor64_wg(xi, xj);
     const int nb = (int)(n - ri < NB ? n - ri : NB);
-    if (diag_done) {
-      // inv(L[b0][b0]) written through to where every XCD reads it, then the count
-      store_diag_wg<true>(xi, xj, L, ldl, ri, nb, W, bad, info + b);
-      __builtin_amdgcn_s_waitcnt(dma::waitcnt_vm(0));
-      __syncthreads();
-      if (threadIdx.x == 0) __hip_atomic_store(diag_done + b, b0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    } else {
-      store_diag_wg(xi, xj, L, ldl, ri, nb, W, bad, info + b);
-    }
+    // inv(L[b0][b0]) written through to where every XCD reads it, then the count
+    store_diag_wg<true>(xi, xj, L, ldl, ri, nb, W, bad, info + b);
+    __builtin_amdgcn_s_waitcnt(dma::waitcnt_vm(0));
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(diag_done + b, b0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return;
   }
   if (!panel) return;
@@ -666,7 +648,7 @@ __global__ __launch_bounds__(256, DMA ? 2 : 4) void chol_update_kernel(float* __
     xj[e / NB][e % NB] = __hip_atomic_load(W + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __syncthreads();
   f32x4_t lp[2][2] = {};
-  mm_nt(xi, xj, lp);
+  mm_nt<true>(xi, xj, lp);
 #pragma unroll
   for (int bi = 0; bi < 2; ++bi)
 #pragma unroll
@@ -705,34 +687,56 @@ __global__ __launch_bounds__(64) void ldl_inv_kernel(const float* __restrict__ l
   for (int i = threadIdx.x; i < bs * bs; i += 64) W[i] = xi[i / bs][i % bs];
 }
 
-// Column block cb: rows below it times inv(DL_cb); its diagonal block set to
-// I (its diagonal to 0 with zero_diag); rows above it are zero and stay so.
+// Rows below each b x b diagonal block times the block's inverse; the blocks
+// themselves set to I (the diagonal to 0 with zero_diag); rows above are zero
+// and stay so.  One 64 x 64 tile of the lower triangle per workgroup, through
+// LDS so that both passes over the matrix move whole rows of 256 bytes (16
+// matrices of n = 2048: 98 us with a thread per row and block, 82 here).
 template <int BS>
 __global__ __launch_bounds__(256) void ldl_apply_kernel(float* __restrict__ l, int64_t ldl, int64_t sl, int64_t n,
                                                         const float* __restrict__ winv, int zero_diag) {
-  constexpr int bs = BS;
-  __shared__ float iv[BS * BS];
-  const int64_t b = blockIdx.z, cb = blockIdx.y;
-  const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const float* W = winv + (b * (n / bs) + cb) * bs * bs;
-  for (int i = threadIdx.x; i < bs * bs; i += 256) iv[i] = W[i];
+  __shared__ __attribute__((aligned(16))) float t[NB][LD];
+  __shared__ float iv[NB][BS];  // row k of the tile's columns: row k % BS of block k / BS's inverse
+  const int64_t b = blockIdx.y;
+  int64_t i = (int64_t)((sqrt(8.0 * (double)blockIdx.x + 1.0) - 1.0) * 0.5);
+  while ((i + 1) * (i + 2) / 2 <= (int64_t)blockIdx.x) ++i;
+  while (i * (i + 1) / 2 > (int64_t)blockIdx.x) --i;
+  const int64_t r0 = i * NB, c0 = ((int64_t)blockIdx.x - i * (i + 1) / 2) * NB;
+  float* L = l + b * sl;
+  load_tile(t, L, ldl, n, r0, c0);
+  const float* W = winv + (b * n + c0) * BS;  // [n / BS][BS][BS]
+  for (int e = threadIdx.x; e < NB * BS; e += 256) iv[e / BS][e % BS] = c0 + e / BS < n ? W[e] : 0.f;
   __syncthreads();
-  const int64_t c0 = cb * bs;
-  if (r >= n || r < c0) return;
-  float* row = l + b * sl + r * ldl + c0;
-  if (r < c0 + bs) {
-    for (int c = 0; c < bs; ++c) row[c] = (c0 + c == r && !zero_diag) ? 1.f : 0.f;
-    return;
-  }
-  float v[BS];
+  const int row = (int)threadIdx.x >> 2, q = 16 * ((int)threadIdx.x & 3);
+  float out[16];
 #pragma unroll
-  for (int k = 0; k < BS; ++k) v[k] = row[k];
-#pragma unroll
-  for (int c = 0; c < BS; ++c) {
+  for (int cc = 0; cc < 16; ++cc) {
+    const int c = q + cc, end = (c / BS + 1) * BS;
     float acc = 0.f;
+    for (int k = c; k < end; ++k) acc += t[row][k] * iv[k][c % BS];
+    const int64_t first = c0 + c / BS * BS;  // the block's first row
+    out[cc] = r0 + row >= first + BS ? acc
+              : r0 + row >= first    ? (r0 + row == c0 + c && !zero_diag ? 1.f : 0.f)
+                                     : t[row][c];
+  }
+  __syncthreads();
 #pragma unroll
-    for (int k = c; k < BS; ++k) acc += v[k] * iv[k * BS + c];
-    row[c] = acc;
+  for (int cc = 0; cc < 16; cc += 4)
+    *reinterpret_cast<f32x4_t*>(&t[row][q + cc]) = f32x4_t{out[cc], out[cc + 1], out[cc + 2], out[cc + 3]};
+  __syncthreads();
+  const bool vec = c0 + NB <= n && ldl % 4 == 0 && (reinterpret_cast<uintptr_t>(L) & 15) == 0;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int e = (int)threadIdx.x + 256 * u, r = e >> 4, c = 4 * (e & 15);
+    if (r0 + r >= n) continue;
+    float* dst = L + (r0 + r) * ldl + c0 + c;
+    if (vec) {
+      *reinterpret_cast<f32x4_t*>(dst) = *reinterpret_cast<const f32x4_t*>(&t[r][c]);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (c0 + c + j < n) dst[j] = t[r][c + j];
+    }
   }
 }
 
@@ -782,9 +786,6 @@ extern "C" int64_t kq_cholesky_workspace_size(int64_t n, int64_t batch) {
   return batch * 2 * NB * NB * (int64_t)sizeof(float) + (batch * (int64_t)sizeof(int) + 255) / 256 * 256;
 }
 
-#ifndef KQ_CHOL_R
-#define KQ_CHOL_R 2
-#endif
 extern "C" int kq_cholesky(const float* a, int64_t lda, int64_t stride_a, float* l, int64_t ldl, int64_t stride_l,
                            int64_t n, int64_t batch, int32_t* info, void* workspace, int64_t workspace_bytes,
                            void* stream) {
@@ -802,7 +803,10 @@ extern "C" int kq_cholesky(const float* a, int64_t lda, int64_t stride_a, float*
   hipStream_t st = (hipStream_t)stream;
   float* winv = (float*)workspace;
   int* diag_done = (int*)(winv + batch * 2 * NB * NB);
-  chol_init_kernel<<<dim3((unsigned)((n + 255) / 256), (unsigned)n, (unsigned)batch), 256, 0, st>>>(
+  const bool vec = n % 4 == 0 && lda % 4 == 0 && ldl % 4 == 0 && !kq_misaligned(a, 16) && !kq_misaligned(l, 16) &&
+                   (batch == 1 || (stride_a % 4 == 0 && stride_l % 4 == 0));
+  auto* init = vec ? chol_init_kernel<true> : chol_init_kernel<false>;
+  init<<<dim3((unsigned)((n + 1023) / 1024), (unsigned)n, (unsigned)batch), 256, 0, st>>>(
       a, lda, stride_a, l, ldl, stride_l, n, info, diag_done);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return kq_check_launch(e, "kq_cholesky/init");
@@ -813,53 +817,33 @@ extern "C" int kq_cholesky(const float* a, int64_t lda, int64_t stride_a, float*
                       (batch == 1 || stride_l % 4 == 0) && (uint64_t)NB * ldl * 4 <= kq::dma::MAX_RANGE;
   chol_diag_kernel<<<(unsigned)batch, 256, 0, st>>>(l, n, ldl, stride_l, winv, info);
   if ((e = hipGetLastError()) != hipSuccess) return kq_check_launch(e, "kq_cholesky/diag");
-  if (batch < 8) {
-    // One launch per panel after the first, in super-panels of R panels:
-    // the launch of a super-panel's first panel S applies the previous
-    // super-panel's panels to the whole trailing matrix (rank 64 R, so the
-    // trailing matrix is read and written once per super-panel), the launch
-    // of panel s inside it applies panels S .. s - 1 to block column s only.
-    // Each launch then factors diagonal block s (its first workgroup) and,
-    // in the workgroups of the tiles below that block, once it is factored,
-    // computes panel s itself.
-    constexpr int R = KQ_CHOL_R;
-    if (m > 1) {
-      chol_panel_kernel<<<dim3((unsigned)(m - 1), (unsigned)batch), 256, 0, st>>>(l, n, ldl, stride_l, 0, 0, 1,
-                                                                                 winv, info);
-      if ((e = hipGetLastError()) != hipSuccess) return kq_check_launch(e, "kq_cholesky/panel");
-    }
-    for (int s = 1; s < m; ++s) {
-      const int64_t q = m - s;
-      const int S = s / R * R;  // this super-panel's first panel
-      const dim3 grid((unsigned)(s == S ? q * (q + 1) / 2 : q), (unsigned)batch);
-      const int qa = s == S ? s - R : S, col = s == S ? 0 : 1;
-      if (dma_ok) chol_update_kernel<true><<<grid, 256, 0, st>>>(l, n, ldl, stride_l, s, qa, s, winv, info, diag_done, col);
-      else chol_update_kernel<false><<<grid, 256, 0, st>>>(l, n, ldl, stride_l, s, qa, s, winv, info, diag_done, col);
-      if ((e = hipGetLastError()) != hipSuccess) return kq_check_launch(e, "kq_cholesky/update");
-    }
-    return KQ_OK;
+  // One launch per panel after the first, in super-panels of R panels: the
+  // launch of a super-panel's first panel S applies the previous super-panel's
+  // panels to the whole trailing matrix (rank 64 R, so the trailing matrix is
+  // read and written once per super-panel), the launch of panel s inside it
+  // applies panels S .. s - 1 to block column s only.  Each launch then
+  // factors diagonal block s (its first workgroup of every matrix) and, in the
+  // workgroups of the tiles below that block, once it is factored, computes
+  // panel s itself.  R grows with the tiles a whole-matrix launch has: what
+  // those launches cost against the longer products of the column launches
+  // (us, block LDL included, R = 2 / 4 / 8: one matrix of n = 2048 714 / 741 /
+  // 805, 16 of them 1559 / 1392 / 1343, 48 3820 / 3302 / 3098, one of n = 7168
+  // 3809 / 3685 / 3780; a launch for each panel and one for the trailing
+  // update, four panels: 16 matrices 1518).
+  const int64_t work = batch * m * m;
+  const int R = work < 3000 ? 2 : work < 14000 ? 4 : 8;
+  if (m > 1) {
+    chol_panel0_kernel<<<dim3((unsigned)(m - 1), (unsigned)batch), 256, 0, st>>>(l, n, ldl, stride_l, winv);
+    if ((e = hipGetLastError()) != hipSuccess) return kq_check_launch(e, "kq_cholesky/panel");
   }
-  // Super-panels of four panels: one launch per panel (its block column
-  // brought up to date with the super-panel's earlier panels, the panel
-  // below its diagonal block, and the next diagonal block factored), then one
-  // rank-256 update of everything to the right, so the trailing matrix is
-  // read and written once per super-panel (measured on MI355X, 48 matrices
-  // of n = 2048: 3.90 ms with four panels, 4.12 with two or eight).
-  const int rank = 4;
-  for (int s0 = 0; s0 < m; s0 += rank) {
-    const int s1 = s0 + rank < m ? s0 + rank : m;
-    for (int p = s0; p < s1 && p + 1 < m; ++p) {
-      chol_panel_kernel<<<dim3((unsigned)(m - p - 1), (unsigned)batch), 256, 0, st>>>(l, n, ldl, stride_l, p, s0,
-                                                                                     s1, winv, info);
-      if ((e = hipGetLastError()) != hipSuccess) return kq_check_launch(e, "kq_cholesky/panel");
-    }
-    if (s1 < m) {
-      const int64_t q = m - s1;
-      const dim3 grid((unsigned)(q * (q + 1) / 2), (unsigned)batch);
-      if (dma_ok) chol_update_kernel<true><<<grid, 256, 0, st>>>(l, n, ldl, stride_l, s1, s0, s1, winv, info, nullptr, 0);
-      else chol_update_kernel<false><<<grid, 256, 0, st>>>(l, n, ldl, stride_l, s1, s0, s1, winv, info, nullptr, 0);
-      if ((e = hipGetLastError()) != hipSuccess) return kq_check_launch(e, "kq_cholesky/update");
-    }
+  for (int s = 1; s < m; ++s) {
+    const int64_t q = m - s;
+    const int S = s / R * R;  // this super-panel's first panel
+    const dim3 grid((unsigned)(s == S ? q * (q + 1) / 2 : q), (unsigned)batch);
+    const int qa = s == S ? s - R : S, col = s == S ? 0 : 1;
+    if (dma_ok) chol_update_kernel<true><<<grid, 256, 0, st>>>(l, n, ldl, stride_l, s, qa, s, winv, info, diag_done, col);
+    else chol_update_kernel<false><<<grid, 256, 0, st>>>(l, n, ldl, stride_l, s, qa, s, winv, info, diag_done, col);
+    if ((e = hipGetLastError()) != hipSuccess) return kq_check_launch(e, "kq_cholesky/update");
   }
   return KQ_OK;
 }
@@ -886,7 +870,9 @@ extern "C" int kq_block_ldl(float* l, int64_t ld, int64_t stride, int64_t n, int
   ldl_inv_kernel<<<dim3((unsigned)(n / b), (unsigned)batch), 64, 0, st>>>(l, ld, stride, n, b, winv);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return kq_check_launch(e, "kq_block_ldl/inv");
-  const dim3 grid((unsigned)((n + 255) / 256), (unsigned)(n / b), (unsigned)batch);
+  const int64_t tiles = (n + NB - 1) / NB;
+  if (tiles * (tiles + 1) / 2 > INT32_MAX) return kq_fail(KQ_ERR_LIMIT, "kq_block_ldl: matrix too large");
+  const dim3 grid((unsigned)(tiles * (tiles + 1) / 2), (unsigned)batch);
   const int zd = (flags & KQ_LDL_ZERO_DIAGONAL) ? 1 : 0;
   switch (b) {
 #define KQ_LDL_CASE(B) \

@@ -72,14 +72,16 @@ def blockwise_preapply_had_r_(x: torch.Tensor, had_dim):
     _hadamard_(x, had_dim, 2)
 
 
-def _cholesky_(h: torch.Tensor, batch: int = 1) -> torch.Tensor:
-    """In-place lower Cholesky of [batch, n, n] (or [n, n]); returns info."""
+def _cholesky_(h: torch.Tensor, batch: int = 1, source: torch.Tensor | None = None) -> torch.Tensor:
+    """Lower Cholesky of [batch, n, n] (or [n, n]) into h, of ``source`` (same
+    strides) or in place; returns info."""
     n = h.shape[-1]
+    source = h if source is None else source
     ws = torch.empty(max(int(N.library().kq_cholesky_workspace_size(n, batch)), 256), dtype=torch.uint8,
                      device=h.device)
     info = torch.empty(batch, dtype=torch.int32, device=h.device)
     stride = n * h.stride(-2)
-    N.call("kq_cholesky", N.ptr(h), h.stride(-2), stride, N.ptr(h), h.stride(-2), stride, n, batch,
+    N.call("kq_cholesky", N.ptr(source), h.stride(-2), stride, N.ptr(h), h.stride(-2), stride, n, batch,
            N.ptr(info), N.ptr(ws), ws.numel(), N.stream(h.device))
     return info
 
@@ -152,8 +154,9 @@ def block_ldl_batched(H: torch.Tensor, b: int = 16) -> tuple[torch.Tensor, torch
     experts, n, _ = H.shape
     if n % b:
         raise ValueError("n must be a multiple of b")
-    lower = H.contiguous().clone()
-    info = _cholesky_(lower, experts)
+    source = H.contiguous()
+    lower = torch.empty_like(source)
+    info = _cholesky_(lower, experts, source)
     _block_ldl_(lower, b, experts)
     return lower, info
 
