@@ -188,8 +188,17 @@ def ptr(t: torch.Tensor | None) -> ctypes.c_void_p:
     return ctypes.c_void_p(0 if t is None else t.data_ptr())
 
 
+def stream_handle(device: torch.device) -> int:
+    """The hipStream_t of torch's current stream on ``device`` (0: the default
+    stream), without building a ``torch.cuda.Stream`` (4 us a call, a third of
+    a small linear's host time)."""
+
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+
+
 def stream(device: torch.device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    return ctypes.c_void_p(stream_handle(device))
 
 
 def require_gpu() -> torch.device:

@@ -58,7 +58,7 @@ def _split_workspace(gpu: torch.device, dtype_code: int, n: int, k: int, weighte
     need = int(N.library().kq_syrk_accumulate_workspace_size(dtype_code, n, k, int(weighted)))
     if need <= 0:
         return None
-    key = (gpu, torch.cuda.current_stream(gpu).stream_id)
+    key = (gpu, N.stream_handle(gpu))
     ws = _SPLIT_WORKSPACES.get(key)
     if ws is None or ws.numel() < need:
         ws = torch.empty(need, dtype=torch.uint8, device=gpu)

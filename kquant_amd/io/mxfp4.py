@@ -105,9 +105,11 @@ def dequant(packed: torch.Tensor, scale: torch.Tensor, *, dtype: torch.dtype = t
     if packed.dtype != torch.uint8:
         raise TypeError(f"expected uint8, got {packed.dtype}")
     k = _check_scale_blocks(packed, scale)
-    lead = torch.broadcast_shapes(packed.shape[:-1], scale.shape[:-1])
-    packed = packed.expand(*lead, packed.shape[-1])
-    scale = scale.expand(*lead, scale.shape[-1])
+    lead = packed.shape[:-1]
+    if scale.shape[:-1] != lead:
+        lead = torch.broadcast_shapes(lead, scale.shape[:-1])
+        packed = packed.expand(*lead, packed.shape[-1])
+        scale = scale.expand(*lead, scale.shape[-1])
     (p, s), gpu, host = N.to_gpu([packed, scale])
     p, s = N.aligned(p), N.aligned(s)
     rows = p.numel() // max(p.shape[-1], 1) if p.shape[-1] else 0

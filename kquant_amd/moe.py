@@ -33,7 +33,7 @@ _WORKSPACES: dict[tuple[torch.device, int], torch.Tensor] = {}
 def _workspace(device: torch.device, nbytes: int) -> torch.Tensor:
     """The forward's workspace, one per (device, stream): calls on one stream
     serialize, calls on different streams must not share it."""
-    key = (device, torch.cuda.current_stream(device).stream_id)
+    key = (device, N.stream_handle(device))
     buf = _WORKSPACES.get(key)
     if buf is None or buf.numel() < nbytes:
         buf = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=device)

@@ -67,7 +67,7 @@ def quantize_tiles_sqg(tiles: torch.Tensor, lut: torch.Tensor, bits: int,
 def _workspace(device: torch.device, bits: int) -> torch.Tensor:
     """Decision workspace, one per (device, stream, rate)."""
     need = int(N.library().kq_sqg_quantize_workspace_size(bits, _workgroups(device)))
-    key = (device, torch.cuda.current_stream(device).stream_id, bits)
+    key = (device, N.stream_handle(device), bits)
     ws = _WORKSPACES.get(key)
     if ws is None or ws.numel() < need:
         ws = torch.empty(need, dtype=torch.uint8, device=device)
