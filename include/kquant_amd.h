@@ -293,14 +293,19 @@ int kq_syrk_accumulate(int in_dtype, const void* x, int64_t ld, int64_t n, int64
  * 0 writes the tile, the others write partial slots, and a second launch
  * adds each tile's slots, in chunk order, to it.  Results are deterministic
  * for a given CU count and agree with kq_syrk_accumulate to fp32 summation
- * order.  Only unweighted bf16 rows take the split; other calls, or a
- * workspace smaller than kq_syrk_accumulate_workspace_size (0 when the
+ * order.  With a workspace of kq_syrk_sliced_workspace_size bytes weighted,
+ * fp16 and fp32 rows whose tiles fill the CUs badly are cut into row slices,
+ * each with an accumulator of its own (k <= 16384), added in order.  Other
+ * calls, or a workspace smaller than kq_syrk_accumulate_workspace_size (0 when the
  * split does not pay), run as kq_syrk_accumulate.  workspace: 256-byte
  * aligned, uninitialised, used by one call at a time.  The size function
  * assumes dense rows (ld == k) and the CU count of the current device; the
  * call plans with the CU count of its stream's device, so make that device
  * current when sizing. */
 int64_t kq_syrk_accumulate_workspace_size(int in_dtype, int64_t n, int64_t k, int weighted);
+/* The workspace with which kq_syrk_accumulate_ws splits any of its calls
+ * (0 when it does not pay). */
+int64_t kq_syrk_sliced_workspace_size(int in_dtype, int64_t n, int64_t k, int weighted);
 int kq_syrk_accumulate_ws(int in_dtype, const void* x, int64_t ld, int64_t n, int64_t k,
                           const float* weights, float* acc, int64_t ld_acc, uint32_t flags,
                           void* workspace, int64_t workspace_bytes, void* stream);
@@ -352,6 +357,21 @@ int kq_segment_weight_sums(const float* weights, const int64_t* offsets, int gro
  * denominator <= 0 gives zeros.  acc, out: [groups, k, k]; no aliasing. */
 int kq_syrk_finalize_grouped(const float* acc, int64_t k, int groups, const double* denominators,
                              float* out, void* stream);
+
+/* kq_syrk_grouped, kq_segment_weight_sums and kq_syrk_finalize_grouped in one
+ * call: out[g] = sym(sum w x x^T) / sum w over group g's rows (zeros for a
+ * group without weight), denominators[g] the f64 sum.  Groups longer than the
+ * launch can balance are cut into row slices with accumulators of their own,
+ * added in order at the end (deterministic).  rows: an upper bound of
+ * offsets[groups] that sizes the slices (the number of listed rows).  out
+ * [groups, k, k], denominators [groups] (device).  workspace:
+ * kq_grouped_covariance_workspace_size bytes (it holds the accumulators),
+ * 256-byte aligned, uninitialised; both plan for the current device. */
+int64_t kq_grouped_covariance_workspace_size(int in_dtype, int64_t rows, int64_t k, int groups);
+int kq_grouped_covariance(int in_dtype, const void* x, int64_t ld, const int64_t* offsets, int groups,
+                          const int32_t* row_index, const float* weights, int64_t rows, int64_t k, float* out,
+                          double* denominators, uint32_t flags, void* workspace, int64_t workspace_bytes,
+                          void* stream);
 
 /* Sums of covariance_comparison (kquant/candidate_hessian.py:219-258) for
  * fp32 [k, k] reference R and candidate C, in f64: out[8] = {sum (C-R)^2,

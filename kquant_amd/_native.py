@@ -98,6 +98,9 @@ SIGNATURES: dict[str, list] = {
     "kq_comparison_sums": [_INT, _VP, _INT, _VP, _I64, _VP, _VP, _VP],
     "kq_kimi_topk": [_INT, _VP, _I64, _VP, _I64, _INT, _INT, _F32, _VP, _VP, _VP],
     "kq_syrk_grouped": [_INT, _VP, _I64, _VP, _INT, _VP, _VP, _I64, _VP, _U32, _VP],
+    "kq_syrk_sliced_workspace_size": [_INT, _I64, _I64, _INT],
+    "kq_grouped_covariance_workspace_size": [_INT, _I64, _I64, _INT],
+    "kq_grouped_covariance": [_INT, _VP, _I64, _VP, _INT, _VP, _VP, _I64, _I64, _VP, _VP, _U32, _VP, _I64, _VP],
     "kq_segment_weight_sums": [_VP, _VP, _INT, _U32, _VP, _VP],
     "kq_syrk_finalize_grouped": [_VP, _I64, _INT, _VP, _VP, _VP],
     "kq_route_sort": [_VP, _I64, _INT, _INT, _VP, _VP, _VP, _VP, _VP, _VP, _I64, _VP],

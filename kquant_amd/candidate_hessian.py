@@ -49,15 +49,18 @@ def _prepare_rows(rows: torch.Tensor, gpu: torch.device) -> tuple[torch.Tensor, 
     return x, k
 
 
+_CACHED_WORKSPACE_BYTES = 256 << 20  # larger ones come from torch's allocator on each call
 _SPLIT_WORKSPACES: dict[tuple[torch.device, int], torch.Tensor] = {}
 
 
 def _split_workspace(gpu: torch.device, dtype_code: int, n: int, k: int, weighted: bool) -> torch.Tensor | None:
     """Partial-tile slots of the split launch (None when it does not pay),
     cached per device and stream: calls sharing slots must not overlap."""
-    need = int(N.library().kq_syrk_accumulate_workspace_size(dtype_code, n, k, int(weighted)))
+    need = int(N.library().kq_syrk_sliced_workspace_size(dtype_code, n, k, int(weighted)))
     if need <= 0:
         return None
+    if need > _CACHED_WORKSPACE_BYTES:
+        return torch.empty(need, dtype=torch.uint8, device=gpu)
     key = (gpu, N.stream_handle(gpu))
     ws = _SPLIT_WORKSPACES.get(key)
     if ws is None or ws.numel() < need:
@@ -328,19 +331,19 @@ def covariance_comparison(reference: torch.Tensor, candidate: torch.Tensor) -> d
 # -------------------------------------------------------- per-expert Hessians --
 
 def _grouped(x: torch.Tensor, k: int, offsets: torch.Tensor, groups: int, index, weights,
-             flags: int) -> tuple[torch.Tensor, torch.Tensor]:
-    """Finalized [groups, k, k] covariances and f64 denominators [groups]."""
+             flags: int, rows: int) -> tuple[torch.Tensor, torch.Tensor]:
+    """Finalized [groups, k, k] covariances and f64 denominators [groups];
+    ``rows`` bounds the listed rows."""
     gpu = x.device
     kp = x.shape[1]
-    acc = torch.empty(groups, kp, kp, dtype=torch.float32, device=gpu)
-    N.call("kq_syrk_grouped", N.DTYPE_CODES[x.dtype], N.ptr(x), kp, N.ptr(offsets), groups, N.ptr(index),
-           N.ptr(weights), kp, N.ptr(acc), flags, N.stream(gpu))
-    sq = N.SYRK_SQUARE_WEIGHTS if flags & N.SYRK_SQUARE_WEIGHTS else 0
-    denominators = _weight_sums(weights, offsets, groups, sq)
-    out = torch.empty_like(acc)
-    N.call("kq_syrk_finalize_grouped", N.ptr(acc), kp, groups, N.ptr(denominators), N.ptr(out),
-           N.stream(gpu))
-    del acc
+    code = N.DTYPE_CODES[x.dtype]
+    need = int(N.library().kq_grouped_covariance_workspace_size(code, rows, kp, groups))
+    ws = torch.empty(max(need, 256), dtype=torch.uint8, device=gpu)
+    out = torch.empty(groups, kp, kp, dtype=torch.float32, device=gpu)
+    denominators = torch.empty(groups, dtype=torch.float64, device=gpu)
+    N.call("kq_grouped_covariance", code, N.ptr(x), kp, N.ptr(offsets), groups, N.ptr(index), N.ptr(weights), rows,
+           kp, N.ptr(out), N.ptr(denominators), flags, N.ptr(ws), ws.numel(), N.stream(gpu))
+    del ws
     if kp != k:
         out = out[:, :k, :k].contiguous()
     return out, denominators
@@ -383,7 +386,7 @@ def expert_hessians(
     N.call("kq_route_sort", N.ptr(ids), tokens, topk, experts, N.ptr(g), N.ptr(offsets), N.ptr(rows),
            None, N.ptr(sorted_w), N.ptr(ws), ws.numel(), N.stream(gpu))
     flags = N.SYRK_SQUARE_WEIGHTS if gate_square else 0
-    h, denominators = _grouped(x, k, offsets, experts, rows, sorted_w, flags)
+    h, denominators = _grouped(x, k, offsets, experts, rows, sorted_w, flags, tokens * topk)
     return h, denominators, offsets[1:] - offsets[:-1]
 
 
@@ -416,7 +419,7 @@ def expert_hessians_from_rows(
     if w is not None:
         w = N.aligned(w.float(), 4)
     flags = N.SYRK_SQUARE_WEIGHTS if square_weights else 0
-    return _grouped(x, k, o, int(o.numel()) - 1, None, w, flags)
+    return _grouped(x, k, o, int(o.numel()) - 1, None, w, flags, int(host_offsets[-1]))
 
 
 def build_expert_hessians(

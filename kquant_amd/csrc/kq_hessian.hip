@@ -78,6 +78,9 @@ __device__ __forceinline__ void split_bf16(float v, uint32_t& hi, uint32_t& lo) 
 // than LPT_MAX_GROUPS groups the quadratic ranking costs more than it saves
 // and row r is group r.
 constexpr int LPT_MAX_GROUPS = 1024;
+// `overwrite` of a launch over row slices (SlicePlan below): empty groups are
+// unused slots, which nothing reads, and write nothing
+constexpr int SYRK_SLOTS = 2;
 __device__ __forceinline__ int64_t group_of_row(const int64_t* __restrict__ offsets, int groups, int r) {
   if (groups > LPT_MAX_GROUPS) return r;
   __shared__ int s_group;
@@ -111,6 +114,7 @@ __global__ __launch_bounds__(256, 1) void syrk_upper_kernel(
     const int64_t g = group_of_row(offsets, gridDim.y, blockIdx.y);
     list0 = offsets[g];
     n = offsets[g + 1] - list0;
+    if (n == 0 && overwrite == SYRK_SLOTS) return;
     acc += g * acc_stride;
   }
   // ---- tile coordinates: linear index -> (ti <= tj) over the upper triangle
@@ -360,6 +364,7 @@ __global__ __launch_bounds__(512, 1) void syrk256_kernel(
     const int64_t g = group_of_row(offsets, gridDim.y, blockIdx.y);
     list0 = offsets[g];
     n = offsets[g + 1] - list0;
+    if (n == 0 && overwrite == SYRK_SLOTS) return;
     acc += g * acc_stride;
   }
   int ti, tj;
@@ -848,17 +853,23 @@ __device__ __forceinline__ void syrk4_wait(int n) {
   asm volatile("" ::: "memory");
 }
 
-// Persistent: `gridDim.x` workgroups walk the items (group rank, tile) in
-// snake order (round q gives item q G + b to workgroup b, reversed on odd
-// rounds).  Ranks order the groups by row count, largest first (ties by
-// index), computed once per workgroup in LDS for up to LPT_MAX_GROUPS groups
-// (natural order beyond); every item's result is independent of the order.
+// Persistent: the `gridDim.x` workgroups take the items (group rank, tile) in
+// order, each its next one from a counter (`queue`, zero before the launch)
+// when it has done the last: ranks order the groups by row count, largest
+// first (ties by index, computed once per workgroup in LDS for up to
+// LPT_MAX_GROUPS groups, natural order beyond), so this is longest-first
+// scheduling.  Without a queue they walk them in snake order (round q gives
+// item q G + b to workgroup b, reversed on odd rounds), which leaves the
+// longest workgroup 20 % over the mean at 65,536 routed rows over 48 experts
+// of Zipf(1.1) popularity (the queue: 1 %).  Every item's result is
+// independent of the order.
 __shared__ int syrk4_rank_order[LPT_MAX_GROUPS];
 __shared__ int syrk4_rank_size[LPT_MAX_GROUPS];
+__shared__ int syrk4_next[2];
 
 __global__ __launch_bounds__(512, 1) void syrk256w_dma_kernel(
     const uint16_t* __restrict__ x, int64_t ld, int64_t k, const float* __restrict__ w, float* __restrict__ acc,
-    int nt, const int64_t* __restrict__ offsets, int groups, int square_w) {
+    int nt, const int64_t* __restrict__ offsets, int groups, int square_w, int* __restrict__ queue, int skip_empty) {
   using namespace syrk4;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -911,9 +922,11 @@ __global__ __launch_bounds__(512, 1) void syrk256w_dma_kernel(
     offb[j] = trow * ROW + (((f >> 3) ^ xorv) << 4) + (f & 7) * 2;
   }
 
-  for (int64_t q = 0;; ++q) {
-    const int64_t item = q * grid + ((q & 1) ? grid - 1 - blockIdx.x : blockIdx.x);
-    if (item >= items) break;
+  int64_t item = blockIdx.x;
+  for (int64_t q = 0; item < items; ++q) {
+    // the next item's number is on its way while this one runs
+    int taken = 0;
+    if (queue && tid == 0) taken = grid + atomicAdd(queue, 1);
     const int rank = (int)(item / ntiles);
     const int64_t g = lpt ? syrk4_rank_order[rank] : rank;
     int ti, tj;
@@ -954,7 +967,10 @@ __global__ __launch_bounds__(512, 1) void syrk256w_dma_kernel(
           global_load_to_lds4(wg + wp, wl0 + (uint32_t)(stage * BK * 4));
         }
       };
-      // rows past the end get weight 0: finite rows then convert to zeros
+      // rows past the end (loads of the last row) get weight 0: finite rows then
+      // convert to zeros.  A non-finite last row puts NaN, where its features
+      // meet others, in entries that its own product already makes Inf or NaN.
+      // (Zeroing both operands instead costs 3 to 5 % on short groups.)
       auto convert = [&](int stage, int t0) {
         unsigned char* st = syrk4_lds + STAGE * stage;
 #pragma unroll
@@ -1035,19 +1051,29 @@ __global__ __launch_bounds__(512, 1) void syrk256w_dma_kernel(
       __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // the loads issued past the end have landed
       __syncthreads();                            // every wave is done with the ring
     }
-    syrk3_store(accv, acc + g * k * k + row0 * k + col0, k, k - row0, k - col0, true, wave, lane);
+    if (n > 0 || !skip_empty)
+      syrk3_store(accv, acc + g * k * k + row0 * k + col0, k, k - row0, k - col0, true, wave, lane);
+    if (queue) {
+      // two slots: the one written now was last read before the previous barrier
+      if (tid == 0) syrk4_next[q & 1] = taken;
+      __syncthreads();
+      item = syrk4_next[q & 1];
+    } else {
+      item = (q + 1) * grid + ((q & 1) ? blockIdx.x : grid - 1 - blockIdx.x);
+    }
   }
 }
 
 static hipError_t launch_syrk256w_dma(const void* x, int64_t ld, int64_t k, const float* w, float* acc,
-                                      const int64_t* offsets, int groups, int square_w, hipStream_t st) {
+                                      const int64_t* offsets, int groups, int square_w, hipStream_t st,
+                                      int* queue = nullptr, int skip_empty = 0) {
   const int nt = (int)((k + syrk4::TILE - 1) / syrk4::TILE);
   const int64_t items = (int64_t)(nt * (nt + 1) / 2) * groups;
   int cus = device_cus(st);
   if (cus <= 0) cus = 256;
   const int grid = (int)(items < cus ? items : cus);
   syrk256w_dma_kernel<<<dim3(grid), dim3(512), 0, st>>>((const uint16_t*)x, ld, k, w, acc, nt, offsets, groups,
-                                                          square_w);
+                                                          square_w, items > grid ? queue : nullptr, skip_empty);
   return hipGetLastError();
 }
 
@@ -1080,7 +1106,8 @@ constexpr int FIN_B = 64;
 template <bool FULL>
 __device__ __forceinline__ void finalize_pair_impl(const float* __restrict__ a, int64_t lda, int64_t k,
                                                    float inv, float* __restrict__ o, int64_t ldo, int64_t bi,
-                                                   int64_t bj, float (*t)[FIN_B][FIN_B + 1]) {
+                                                   int64_t bj, float (*t)[FIN_B][FIN_B + 1], int planes,
+                                                   int64_t plane) {
 #pragma clang fp contract(off)
   const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
   const int64_t i0 = bi * FIN_B, j0 = bj * FIN_B;
@@ -1092,15 +1119,27 @@ __device__ __forceinline__ void finalize_pair_impl(const float* __restrict__ a, 
 #pragma unroll
   for (int q = 0; q < R; ++q) {
     const int64_t i = i0 + ty + 4 * q, j = j0 + tx;
-    u[q] = FULL || (i < k && j < k) ? a[i * lda + j] : 0.0f;
+    u[q] = planes > 0 && (FULL || (i < k && j < k)) ? a[i * lda + j] : 0.0f;
   }
+  for (int p = 1; p < planes; ++p)  // a group's row slices, in order
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const int64_t i = i0 + ty + 4 * q, j = j0 + tx;
+      if (FULL || (i < k && j < k)) u[q] += a[p * plane + i * lda + j];
+    }
   if (two) {
     float l[R];
 #pragma unroll
     for (int q = 0; q < R; ++q) {
       const int64_t p = j0 + ty + 4 * q, c = i0 + tx;
-      l[q] = FULL || (p < k && c < k) ? a[p * lda + c] : 0.0f;
+      l[q] = planes > 0 && (FULL || (p < k && c < k)) ? a[p * lda + c] : 0.0f;
     }
+    for (int s = 1; s < planes; ++s)
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        const int64_t p = j0 + ty + 4 * q, c = i0 + tx;
+        if (FULL || (p < k && c < k)) l[q] += a[s * plane + p * lda + c];
+      }
 #pragma unroll
     for (int q = 0; q < R; ++q) t[1][ty + 4 * q][tx] = l[q];
   }
@@ -1134,11 +1173,11 @@ __device__ __forceinline__ void finalize_pair_impl(const float* __restrict__ a, 
 
 __device__ __forceinline__ void finalize_pair(const float* __restrict__ a, int64_t lda, int64_t k, float inv,
                                               float* __restrict__ o, int64_t ldo, int64_t bi, int64_t bj,
-                                              float (*t)[FIN_B][FIN_B + 1]) {
+                                              float (*t)[FIN_B][FIN_B + 1], int planes = 1, int64_t plane = 0) {
   if ((bj + 1) * FIN_B <= k)  // bi <= bj: the whole pair is inside the matrix
-    finalize_pair_impl<true>(a, lda, k, inv, o, ldo, bi, bj, t);
+    finalize_pair_impl<true>(a, lda, k, inv, o, ldo, bi, bj, t, planes, plane);
   else
-    finalize_pair_impl<false>(a, lda, k, inv, o, ldo, bi, bj, t);
+    finalize_pair_impl<false>(a, lda, k, inv, o, ldo, bi, bj, t, planes, plane);
 }
 
 // block pair b of the upper triangle of nb x nb blocks -> (bi <= bj)
@@ -1246,42 +1285,144 @@ __global__ __launch_bounds__(256) void cov_stats_final_kernel(const double* __re
 }
 
 // Grouped finalize: out[g] = sym(acc[g]) / denominators[g] (zeros when the
-// group has no weight), blockIdx.y = group.
+// group has no weight), blockIdx.y = group.  With `first`, acc holds row
+// slices: group g is the sum of planes first[g] .. first[g + 1] - 1.
 __global__ __launch_bounds__(256) void syrk_finalize_grouped_kernel(
     const float* __restrict__ acc, int64_t k, const double* __restrict__ denominators,
-    float* __restrict__ out) {
+    float* __restrict__ out, const int* __restrict__ first) {
   __shared__ float t[2][FIN_B][FIN_B + 1];
   const int64_t g = blockIdx.y;
   const double d = denominators[g];
   const float inv = d > 0.0 ? (float)(1.0 / d) : 0.0f;
   int64_t bi, bj;
   finalize_pair_of(blockIdx.x, bi, bj);
-  finalize_pair(acc + g * k * k, k, k, inv, out + g * k * k, k, bi, bj, t);
+  const int64_t p0 = first ? first[g] : g;
+  finalize_pair(acc + p0 * k * k, k, k, inv, out + g * k * k, k, bi, bj, t, first ? first[g + 1] - first[g] : 1, k * k);
+}
+
+// Row slices.  A group whose tiles are too few or too long for the CUs (one
+// layer's weighted Hessian at k = 413: 3 tiles; a hot expert) is cut into
+// slices of at most `rows` rows (equal, multiples of 64), each accumulated as
+// a group of its own into its slot's k x k plane; the finalize (or
+// slot_sum_kernel) adds a group's slots in order, so results stay
+// deterministic.  One slice -> sliced: weighted bf16 6110 rows x 416 486 -> 73 us,
+// 4820 x 3824 435 -> 262; f32 5446 x 2832 1057 -> 709; 17 routed experts of
+// 10293 rows x 552 156 -> 106; 65536 rows in 48 Zipf groups x 2048 928 -> 883 (the
+// queue and the slices of the hot experts; the planes' finalize reads no more
+// than the accumulators' did).  One workgroup writes the slots' row offsets (slot s owns
+// list positions [slot_offsets[s], slot_offsets[s + 1]); unused slots at the
+// end are empty), each group's first slot, and clears the item queue.
+__device__ __forceinline__ void slice_rows(const int64_t* __restrict__ offsets, int64_t n, int groups, int64_t rows,
+                                           int slots, int64_t* __restrict__ slot_offsets, int* __restrict__ first,
+                                           int* __restrict__ queue) {
+  __shared__ int scan[16];
+  const int t = threadIdx.x;
+  int carry = 0;
+  auto off = [&](int g) { return offsets ? offsets[g] : (g ? n : 0); };  // no offsets: one group of n rows
+  if (t == 0) *queue = 0;
+  for (int base = 0; base < groups; base += 1024) {
+    const int g = base + t;
+    const int64_t o = g < groups ? off(g) : 0, m = g < groups ? off(g + 1) - o : 0;
+    const int c = m > 0 ? (int)((m + rows - 1) / rows) : 0;
+    int incl = c;
+#pragma unroll
+    for (int h = 1; h < 64; h <<= 1) {
+      const int v = __shfl_up(incl, h, 64);
+      if ((t & 63) >= h) incl += v;
+    }
+    if ((t & 63) == 63) scan[t >> 6] = incl;
+    __syncthreads();
+    int total = 0;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      if (v == t >> 6) incl += total;
+      total += scan[v];
+    }
+    const int f = carry + incl - c;
+    if (g < groups) {  // `slots` bounds what is written and read also where the caller's row bound is too low
+      first[g] = f < slots ? f : slots;
+      const int64_t part = c ? ((m + c - 1) / c + 63) / 64 * 64 : 0;
+      for (int q = 0; q < c && f + q < slots; ++q) slot_offsets[f + q] = o + (q * part < m ? q * part : m);
+    }
+    carry += total;
+    __syncthreads();
+  }
+  if (t == 0) first[groups] = carry < slots ? carry : slots;
+  for (int s = carry + t; s <= slots; s += 1024) slot_offsets[s] = off(groups);
+}
+
+__global__ __launch_bounds__(1024) void slice_rows_kernel(const int64_t* __restrict__ offsets, int64_t n, int groups,
+                                                          int64_t rows, int slots, int64_t* __restrict__ slot_offsets,
+                                                          int* __restrict__ first, int* __restrict__ queue) {
+  slice_rows(offsets, n, groups, rows, slots, slot_offsets, first, queue);
+}
+
+// acc's upper tiles = or += the sum of `slots` planes in order, one entry per
+// thread, eight planes' loads in flight.
+__global__ __launch_bounds__(256) void slot_sum_kernel(const float* __restrict__ planes, int slots, int64_t k,
+                                                       int tile, float* __restrict__ acc, int64_t ld_acc,
+                                                       int overwrite) {
+  const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x, r = blockIdx.y;
+  if (c >= k || c / tile < r / tile) return;
+  const float* p = planes + r * k + c;
+  float v = overwrite ? 0.0f : acc[r * ld_acc + c];
+  int s = 0;
+  for (; s + 8 <= slots; s += 8) {
+    float u[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) u[i] = p[(s + i) * k * k];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v += u[i];
+  }
+  for (; s < slots; ++s) v += p[s * k * k];
+  acc[r * ld_acc + c] = v;
 }
 
 // Per-group f64 sums of the row weights (of their fp32 squares with
 // square_w; of 1 per row without weights): one workgroup per group, a fixed
-// reduction tree, so the result is deterministic.
-__global__ __launch_bounds__(256) void segment_weight_sum_kernel(const float* __restrict__ w,
-                                                                 const int64_t* __restrict__ offsets,
-                                                                 int square_w, double* __restrict__ out) {
-  __shared__ double part[256];
+// reduction tree, so the result is deterministic; 1,024 threads with four
+// loads each in flight (8,000 rows of a group: 16 us with 256 and one).
+__device__ __forceinline__ void segment_weight_sum(const float* __restrict__ w, const int64_t* __restrict__ offsets,
+                                                   int square_w, double* __restrict__ out) {
+  __shared__ double part[1024];
   const int64_t g = blockIdx.x;
   const int64_t p0 = offsets[g], p1 = offsets[g + 1];
   double s = 0.0;
-  for (int64_t p = p0 + threadIdx.x; p < p1; p += 256) {
-    float v = w ? w[p] : 1.0f;
-    if (square_w == 1) v = v * v;  // fp32 square, then f64 sum
-    const double d = (double)v;
-    s += square_w == 2 ? d * d : d;  // f64 square
+  for (int64_t p = p0 + threadIdx.x; p < p1; p += 4096) {
+    float v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = p + 1024 * i < p1 ? (w ? w[p + 1024 * i] : 1.0f) : 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (square_w == 1) v[i] = v[i] * v[i];  // fp32 square, then f64 sum
+      const double d = (double)v[i];
+      s += square_w == 2 ? d * d : d;  // f64 square
+    }
   }
   part[threadIdx.x] = s;
   __syncthreads();
-  for (int h = 128; h > 0; h >>= 1) {
+  for (int h = 512; h > 0; h >>= 1) {
     if ((int)threadIdx.x < h) part[threadIdx.x] += part[threadIdx.x + h];
     __syncthreads();
   }
   if (threadIdx.x == 0) out[g] = part[0];
+}
+
+__global__ __launch_bounds__(1024) void segment_weight_sum_kernel(const float* __restrict__ w,
+                                                                  const int64_t* __restrict__ offsets,
+                                                                  int square_w, double* __restrict__ out) {
+  segment_weight_sum(w, offsets, square_w, out);
+}
+
+// Both in one launch: blocks 0 .. groups - 1 the weight sums, the last one the
+// slices.
+__global__ __launch_bounds__(1024) void prepare_groups_kernel(const float* __restrict__ w,
+                                                              const int64_t* __restrict__ offsets, int square_w,
+                                                              double* __restrict__ sums, int groups, int64_t rows,
+                                                              int slots, int64_t* __restrict__ slot_offsets,
+                                                              int* __restrict__ first, int* __restrict__ queue) {
+  if ((int)blockIdx.x < groups) segment_weight_sum(w, offsets, square_w, sums);
+  else slice_rows(offsets, 0, groups, rows, slots, slot_offsets, first, queue);
 }
 
 // Sums behind covariance_comparison (kquant/candidate_hessian.py:219-258), in
@@ -1377,6 +1518,79 @@ static hipError_t launch_syrk(const void* x, int64_t ld, int64_t n, int64_t k, c
   return hipGetLastError();
 }
 
+// One grouped launch over acc [groups, k, k].  overwrite: 1, or SYRK_SLOTS
+// (empty groups write nothing); queue: a zeroed item counter or NULL.
+static hipError_t launch_grouped(int in_dtype, const void* x, int64_t ld, const int64_t* offsets, int groups,
+                                 const int32_t* index, const float* w, int64_t k, float* acc, int overwrite, int sq,
+                                 int* queue, hipStream_t st) {
+  if (in_dtype == KQ_DT_BF16) {
+    if (w && !index) return launch_syrk256w_dma(x, ld, k, w, acc, offsets, groups, sq, st, queue, overwrite == SYRK_SLOTS);
+    return w ? launch_syrk256<true, true>(x, ld, 0, k, w, acc, k, overwrite, st, offsets, index, groups, sq)
+             : launch_syrk256<false, true>(x, ld, 0, k, w, acc, k, overwrite, st, offsets, index, groups, sq);
+  }
+  if (in_dtype == KQ_DT_F16)
+    return w ? launch_syrk<1, true, true, true>(x, ld, 0, k, w, acc, k, overwrite, st, offsets, index, groups, sq)
+             : launch_syrk<1, true, false, true>(x, ld, 0, k, w, acc, k, overwrite, st, offsets, index, groups, sq);
+  return w ? launch_syrk<2, true, true, true>(x, ld, 0, k, w, acc, k, overwrite, st, offsets, index, groups, sq)
+           : launch_syrk<2, true, false, true>(x, ld, 0, k, w, acc, k, overwrite, st, offsets, index, groups, sq);
+}
+
+// Row slices of a launch: at most `rows` rows each, in `slots` planes.
+struct SlicePlan {
+  int64_t rows;
+  int slots;
+};
+struct SliceSpace {  // workspace offsets: item queue, first slots, slot offsets, planes
+  int64_t first, offsets, planes, total;
+};
+static SliceSpace slice_space(int groups, int slots, int64_t k) {
+  SliceSpace s;
+  s.first = 256;
+  s.offsets = s.first + ((int64_t)(groups + 1) * 4 + 255) / 256 * 256;
+  s.planes = s.offsets + ((int64_t)(slots + 1) * 8 + 255) / 256 * 256;
+  s.total = s.planes + (int64_t)slots * k * k * 4;
+  return s;
+}
+static int64_t upper_tiles(int in_dtype, int64_t k) {
+  const int64_t tile = in_dtype == KQ_DT_BF16 ? syrk2::TILE : syrk::TILE, nt = (k + tile - 1) / tile;
+  return nt * (nt + 1) / 2;
+}
+
+// Grouped rows (`rows` in all at most): no slice longer than a CU's mean
+// share of the rows (twice that where the groups give a CU half to four items:
+// shorter slices would only add rounds), and none shorter than 256 rows (16
+// steps of the matrix loop against the 4 us of a tile's stores).
+static SlicePlan plan_group_slices(int in_dtype, int64_t rows, int64_t k, int groups, int cus) {
+  const int64_t tiles = upper_tiles(in_dtype, k), share = rows * tiles / (cus > 0 ? cus : 256);
+  int64_t cut = tiles * groups >= 4 * cus || 2 * tiles * groups < cus ? share : 2 * share;
+  // 65535: the grid's limit on slots
+  const int64_t least = groups < 65535 ? rows / (65536 - groups) + 1 : rows + 1;
+  cut = cut < 256 ? 256 : cut;
+  cut = ((cut < least ? least : cut) + 63) / 64 * 64;
+  return {cut, groups + (int)(rows / cut)};
+}
+
+// One group of n rows: S slices minimising the rounds of (tile, slice) items
+// times a slice's time (measured per row and tile, a few us to write it) plus
+// the planes written and summed at 4.5 TB/s.
+static SlicePlan plan_row_slices(int in_dtype, int64_t n, int64_t k, int cus) {
+  const double row_us = in_dtype == KQ_DT_BF16 ? 0.07 : 0.10;
+  const int64_t tiles = upper_tiles(in_dtype, k), tile = in_dtype == KQ_DT_BF16 ? syrk2::TILE : syrk::TILE;
+  SlicePlan best{(n + 63) / 64 * 64, 1};
+  if (cus <= 0) return best;
+  double best_us = 0.95 * ((double)((tiles + cus - 1) / cus) * ((double)n * row_us + 4.0));
+  for (int64_t s = 2; s <= 64 && n / s >= 128; ++s) {
+    const int64_t part = ((n + s - 1) / s + 63) / 64 * 64;
+    const double us = (double)((tiles * s + cus - 1) / cus) * ((double)part * row_us + 4.0) + 10.0 +
+                      (double)(s * tiles * tile * tile * 8) / 4.5e6;
+    if (us < best_us) {
+      best_us = us;
+      best = {part, (int)((n + part - 1) / part)};
+    }
+  }
+  return best;
+}
+
 // The direct-load kernel serves unweighted bf16 rows whose byte range fits
 // the buffer descriptor's 32-bit offsets.
 static bool dma_syrk(int in_dtype, const void* weights, int64_t n, int64_t ld) {
@@ -1386,6 +1600,7 @@ static bool dma_syrk(int in_dtype, const void* weights, int64_t n, int64_t ld) {
 static int syrk_accumulate(int in_dtype, const void* x, int64_t ld, int64_t n, int64_t k, const float* weights,
                            float* acc, int64_t ld_acc, uint32_t flags, void* workspace, int64_t ws_bytes,
                            void* stream);
+constexpr int64_t SLICE_MAX_K = 16384;  // the grouped kernels' limit
 
 extern "C" int64_t kq_syrk_accumulate_workspace_size(int in_dtype, int64_t n, int64_t k, int weighted) {
   if (n < 0 || k <= 0) return -1;
@@ -1394,6 +1609,15 @@ extern "C" int64_t kq_syrk_accumulate_workspace_size(int in_dtype, int64_t n, in
   if (!dma_syrk(in_dtype, weighted ? (const void*)1 : nullptr, n, k)) return 0;
   const int nt = (int)((k + syrk3::TILE - 1) / syrk3::TILE);
   return tail_slot_bytes(plan_tail(nt * (nt + 1) / 2, device_cus(), n));
+}
+
+extern "C" int64_t kq_syrk_sliced_workspace_size(int in_dtype, int64_t n, int64_t k, int weighted) {
+  if (n < 0 || k <= 0 || in_dtype < KQ_DT_BF16 || in_dtype > KQ_DT_F32) return -1;
+  if (dma_syrk(in_dtype, weighted ? (const void*)1 : nullptr, n, k))
+    return kq_syrk_accumulate_workspace_size(in_dtype, n, k, weighted);
+  if (k > SLICE_MAX_K) return 0;
+  const SlicePlan p = plan_row_slices(in_dtype, n, k, device_cus());
+  return p.slots > 1 ? slice_space(1, p.slots, k).total : 0;
 }
 
 extern "C" int kq_syrk_accumulate_ws(int in_dtype, const void* x, int64_t ld, int64_t n, int64_t k,
@@ -1428,6 +1652,22 @@ static int syrk_accumulate(int in_dtype, const void* x, int64_t ld, int64_t n, i
   hipStream_t st = (hipStream_t)stream;
   hipError_t e;
   const bool weighted = weights != nullptr;
+  if (workspace && k <= SLICE_MAX_K && !dma_syrk(in_dtype, weights, n, ld)) {
+    const SlicePlan p = plan_row_slices(in_dtype, n, k, device_cus(st));
+    const SliceSpace sp = slice_space(1, p.slots, k);
+    if (p.slots > 1 && sp.total <= ws_bytes) {
+      unsigned char* w = (unsigned char*)workspace;
+      int64_t* so = (int64_t*)(w + sp.offsets);
+      float* planes = (float*)(w + sp.planes);
+      slice_rows_kernel<<<1, 1024, 0, st>>>(nullptr, n, 1, p.rows, p.slots, so, (int*)(w + sp.first), (int*)w);
+      if ((e = hipGetLastError()) != hipSuccess) return kq_check_launch(e, "kq_syrk_accumulate/slices");
+      e = launch_grouped(in_dtype, x, ld, so, p.slots, nullptr, weights, k, planes, SYRK_SLOTS, 0, (int*)w, st);
+      if (e != hipSuccess) return kq_check_launch(e, "kq_syrk_accumulate/sliced");
+      slot_sum_kernel<<<dim3((unsigned)((k + 255) / 256), (unsigned)k), 256, 0, st>>>(
+          planes, p.slots, k, in_dtype == KQ_DT_BF16 ? syrk2::TILE : syrk::TILE, acc, ld_acc, overwrite);
+      return kq_check_launch(hipGetLastError(), "kq_syrk_accumulate/sum");
+    }
+  }
   if (in_dtype == KQ_DT_BF16) {
     if (weighted)
       e = launch_syrk256<true, false>(x, ld, n, k, weights, acc, ld_acc, overwrite, st);
@@ -1484,20 +1724,8 @@ extern "C" int kq_syrk_grouped(int in_dtype, const void* x, int64_t ld, const in
     return kq_fail(KQ_ERR_INVALID, "kq_syrk_grouped: misaligned rows, offsets, index or weights");
   if (k > 16384) return kq_fail(KQ_ERR_LIMIT, "kq_syrk_grouped: k=%lld exceeds 16384", (long long)k);
   const int sq = (flags & KQ_SYRK_SQUARE_WEIGHTS) ? 1 : 0;
-  hipStream_t st = (hipStream_t)stream;
-  hipError_t e;
-  const bool weighted = weights != nullptr;
-  if (in_dtype == KQ_DT_BF16)
-    e = weighted && !row_index
-            ? launch_syrk256w_dma(x, ld, k, weights, acc, offsets, groups, sq, st)
-        : weighted ? launch_syrk256<true, true>(x, ld, 0, k, weights, acc, k, 1, st, offsets, row_index, groups, sq)
-                 : launch_syrk256<false, true>(x, ld, 0, k, weights, acc, k, 1, st, offsets, row_index, groups, sq);
-  else if (in_dtype == KQ_DT_F16)
-    e = weighted ? launch_syrk<1, true, true, true>(x, ld, 0, k, weights, acc, k, 1, st, offsets, row_index, groups, sq)
-                 : launch_syrk<1, true, false, true>(x, ld, 0, k, weights, acc, k, 1, st, offsets, row_index, groups, sq);
-  else
-    e = weighted ? launch_syrk<2, true, true, true>(x, ld, 0, k, weights, acc, k, 1, st, offsets, row_index, groups, sq)
-                 : launch_syrk<2, true, false, true>(x, ld, 0, k, weights, acc, k, 1, st, offsets, row_index, groups, sq);
+  const hipError_t e = launch_grouped(in_dtype, x, ld, offsets, groups, row_index, weights, k, acc, 1, sq, nullptr,
+                                      (hipStream_t)stream);
   return kq_check_launch(e, "kq_syrk_grouped");
 }
 
@@ -1506,7 +1734,7 @@ extern "C" int kq_segment_weight_sums(const float* weights, const int64_t* offse
   if (groups < 1 || !offsets || !out || kq_misaligned(offsets, 8) || kq_misaligned(out, 8))
     return kq_fail(KQ_ERR_INVALID, "kq_segment_weight_sums: bad arguments");
   const int mode = (flags & KQ_SUM_SQUARE_F64) ? 2 : (flags & KQ_SYRK_SQUARE_WEIGHTS) ? 1 : 0;
-  segment_weight_sum_kernel<<<groups, 256, 0, (hipStream_t)stream>>>(weights, offsets, mode, out);
+  segment_weight_sum_kernel<<<groups, 1024, 0, (hipStream_t)stream>>>(weights, offsets, mode, out);
   return kq_check_launch(hipGetLastError(), "kq_segment_weight_sums");
 }
 
@@ -1520,8 +1748,53 @@ extern "C" int kq_syrk_finalize_grouped(const float* acc, int64_t k, int groups,
   hipStream_t st = (hipStream_t)stream;
   const int64_t nb = (k + FIN_B - 1) / FIN_B;
   syrk_finalize_grouped_kernel<<<dim3((unsigned)(nb * (nb + 1) / 2), (unsigned)groups), 256, 0, st>>>(
-      acc, k, denominators, out);
+      acc, k, denominators, out, nullptr);
   return kq_check_launch(hipGetLastError(), "kq_syrk_finalize_grouped");
+}
+
+extern "C" int64_t kq_grouped_covariance_workspace_size(int in_dtype, int64_t rows, int64_t k, int groups) {
+  if (rows < 0 || k <= 0 || groups < 1 || in_dtype < KQ_DT_BF16 || in_dtype > KQ_DT_F32) return -1;
+  return slice_space(groups, plan_group_slices(in_dtype, rows, k, groups, device_cus()).slots, k).total;
+}
+
+extern "C" int kq_grouped_covariance(int in_dtype, const void* x, int64_t ld, const int64_t* offsets, int groups,
+                                     const int32_t* row_index, const float* weights, int64_t rows, int64_t k,
+                                     float* out, double* denominators, uint32_t flags, void* workspace,
+                                     int64_t workspace_bytes, void* stream) {
+  const char* fn = "kq_grouped_covariance";
+  if (in_dtype < KQ_DT_BF16 || in_dtype > KQ_DT_F32)
+    return kq_fail(KQ_ERR_INVALID, "%s: unknown input dtype %d", fn, in_dtype);
+  if (groups < 1 || groups > 65535 || k <= 0 || k % 8 != 0 || ld < k || ld % 8 != 0 || rows < 0 || !offsets || !out ||
+      !denominators || !workspace)
+    return kq_fail(KQ_ERR_INVALID,
+                   "%s: need 1 <= groups <= 65535, k %% 8 == 0, ld >= k, ld %% 8 == 0, rows >= 0 "
+                   "(groups=%d k=%lld ld=%lld rows=%lld)",
+                   fn, groups, (long long)k, (long long)ld, (long long)rows);
+  if (kq_misaligned(x, 16) || kq_misaligned(offsets, 8) || kq_misaligned(row_index, 4) || kq_misaligned(weights, 4) ||
+      kq_misaligned(workspace, 256))
+    return kq_fail(KQ_ERR_INVALID, "%s: misaligned buffer", fn);
+  if (k > SLICE_MAX_K) return kq_fail(KQ_ERR_LIMIT, "%s: k=%lld exceeds %lld", fn, (long long)k, (long long)SLICE_MAX_K);
+  hipStream_t st = (hipStream_t)stream;
+  // the plan of the current device's CU count, as the size function makes it
+  const SlicePlan p = plan_group_slices(in_dtype, rows, k, groups, device_cus());
+  const SliceSpace sp = slice_space(groups, p.slots, k);
+  if (workspace_bytes < sp.total)
+    return kq_fail(KQ_ERR_INVALID, "%s: workspace needs %lld bytes", fn, (long long)sp.total);
+  unsigned char* w = (unsigned char*)workspace;
+  int* first = (int*)(w + sp.first);
+  int64_t* so = (int64_t*)(w + sp.offsets);
+  float* planes = (float*)(w + sp.planes);
+  hipError_t e;
+  const int sq = (flags & KQ_SYRK_SQUARE_WEIGHTS) ? 1 : 0;
+  prepare_groups_kernel<<<groups + 1, 1024, 0, st>>>(weights, offsets, sq, denominators, groups, p.rows, p.slots, so,
+                                                     first, (int*)w);
+  if ((e = hipGetLastError()) != hipSuccess) return kq_check_launch(e, fn);
+  e = launch_grouped(in_dtype, x, ld, so, p.slots, row_index, weights, k, planes, SYRK_SLOTS, sq, (int*)w, st);
+  if (e != hipSuccess) return kq_check_launch(e, fn);
+  const int64_t nb = (k + FIN_B - 1) / FIN_B;
+  syrk_finalize_grouped_kernel<<<dim3((unsigned)(nb * (nb + 1) / 2), (unsigned)groups), 256, 0, st>>>(
+      planes, k, denominators, out, first);
+  return kq_check_launch(hipGetLastError(), fn);
 }
 
 extern "C" int kq_covariance_comparison_sums(const float* reference, const float* candidate, int64_t k,

@@ -415,3 +415,63 @@ def test_finalize_is_bitwise_mirror_scale_average(gpu, k, ld):
     assert np.array_equal(outg[1], _finalize_expected(accg[1].cpu().numpy(), k, np.float32(1.0 / 3.0)))
     # no weight: acc * 0, i.e. zeros where acc is finite and NaN where it is not
     assert np.array_equal(outg[2], _finalize_expected(acc.numpy(), k, np.float32(0.0)), equal_nan=True)
+
+
+def _f64_covariance(x, w):
+    x = x.double()
+    return (x * w.double()[:, None]).T @ x / float(w.double().sum())
+
+
+@pytest.mark.parametrize("n,k", [(12001, 200), (30000, 413), (257, 1100)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_sliced_layer_rows(gpu, n, k, dtype):
+    """Few tiles: the rows are cut into slices summed in order (the last shape
+    is too short for one).  TOL as everywhere here; repeats are bitwise equal."""
+    print(f"case sliced n={n} k={k} {dtype}", flush=True)
+    x = workloads.student_t4(n, k, seed=n + k, dtype=dtype).to(gpu)
+    w = (torch.rand(n, generator=torch.Generator().manual_seed(n)) + 0.1).to(gpu)
+    for weights in (w, torch.ones_like(w)):
+        h, _ = ch.weighted_covariance(x, weights, device=gpu, return_cpu=False)
+        ref = _f64_covariance(x, weights)
+        assert float((h.double() - ref).norm() / ref.norm()) <= TOL
+        assert torch.equal(h, h.T)
+        assert torch.equal(h, ch.weighted_covariance(x, weights, device=gpu, return_cpu=False)[0])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("k,experts", [(200, 3), (1100, 40), (256, 300)])
+def test_sliced_groups(gpu, k, experts, dtype):
+    """Groups of very different sizes (empty ones, one row, one with most of
+    the rows): sliced, with and without the item queue, as a list of rows and
+    through a routing."""
+    print(f"case sliced groups k={k} experts={experts} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(k + experts)
+    counts = torch.randint(0, 90, (experts,), generator=g)
+    counts[::4] = 0
+    counts[1], counts[2] = 4001, 1
+    offsets = torch.zeros(experts + 1, dtype=torch.int64)
+    offsets[1:] = counts.cumsum(0)
+    total = int(offsets[-1])
+    x = workloads.student_t4(total, k, seed=k, dtype=dtype).to(gpu)
+    w = (torch.rand(total, generator=g) + 0.1).to(gpu)
+    perm = torch.randperm(total, generator=g)
+    ids = torch.repeat_interleave(torch.arange(experts), counts)
+    routed_ids = torch.empty(total, 1, dtype=torch.int32)
+    routed_ids[perm, 0] = ids.to(torch.int32)
+    routed_x, routed_w = torch.empty_like(x), torch.empty_like(w)
+    routed_x[perm.to(gpu)], routed_w[perm.to(gpu)] = x, w
+
+    def runs():
+        yield ch.expert_hessians_from_rows(x, offsets, w, square_weights=True)[0], w.double().square()
+        yield ch.expert_hessians_from_rows(x, offsets)[0], torch.ones_like(w)
+        yield ch.expert_hessians(routed_x, routed_ids.to(gpu), routed_w[:, None], experts)[0], w.double().square()
+
+    for (h, wt), (again, _) in zip(runs(), runs()):
+        assert torch.equal(h, again)
+        for e in range(experts):
+            a, b = int(offsets[e]), int(offsets[e + 1])
+            if a == b:
+                assert not h[e].any()
+                continue
+            ref = _f64_covariance(x[a:b], wt[a:b])
+            assert float((h[e].double() - ref).norm() / ref.norm()) <= TOL, e
