@@ -49,26 +49,6 @@ def _prepare_rows(rows: torch.Tensor, gpu: torch.device) -> tuple[torch.Tensor, 
     return x, k
 
 
-_CACHED_WORKSPACE_BYTES = 256 << 20  # larger ones come from torch's allocator on each call
-_SPLIT_WORKSPACES: dict[tuple[torch.device, int], torch.Tensor] = {}
-
-
-def _split_workspace(gpu: torch.device, dtype_code: int, n: int, k: int, weighted: bool) -> torch.Tensor | None:
-    """Partial-tile slots of the split launch (None when it does not pay),
-    cached per device and stream: calls sharing slots must not overlap."""
-    need = int(N.library().kq_syrk_sliced_workspace_size(dtype_code, n, k, int(weighted)))
-    if need <= 0:
-        return None
-    if need > _CACHED_WORKSPACE_BYTES:
-        return torch.empty(need, dtype=torch.uint8, device=gpu)
-    key = (gpu, N.stream_handle(gpu))
-    ws = _SPLIT_WORKSPACES.get(key)
-    if ws is None or ws.numel() < need:
-        ws = torch.empty(need, dtype=torch.uint8, device=gpu)
-        _SPLIT_WORKSPACES[key] = ws
-    return ws
-
-
 def _syrk(x: torch.Tensor, weights: torch.Tensor | None, gpu: torch.device) -> torch.Tensor:
     """Upper-tile accumulator of X^T diag(w) X, [kp, kp] fp32 (kp = padded k)."""
     n, kp = x.shape
@@ -77,7 +57,9 @@ def _syrk(x: torch.Tensor, weights: torch.Tensor | None, gpu: torch.device) -> t
     if weights is not None:
         w = N.aligned(weights.detach().to(device=gpu, dtype=torch.float32))
     code = N.DTYPE_CODES[x.dtype]
-    ws = _split_workspace(gpu, code, n, kp, w is not None)
+    # the split launches' planes, the call's own: nothing is shared between streams or captured graphs
+    need = int(N.library().kq_syrk_sliced_workspace_size(code, n, kp, int(w is not None)))
+    ws = torch.empty(need, dtype=torch.uint8, device=gpu) if need > 0 else None
     N.call("kq_syrk_accumulate_ws", code, N.ptr(x), kp, n, kp, N.ptr(w), N.ptr(acc), kp, N.SYRK_OVERWRITE,
            N.ptr(ws), 0 if ws is None else ws.numel(), N.stream(gpu))
     return acc

@@ -1348,7 +1348,8 @@ __device__ __forceinline__ void slice_rows(const int64_t* __restrict__ offsets, 
     __syncthreads();
   }
   if (t == 0) first[groups] = carry < slots ? carry : slots;
-  for (int s = carry + t; s <= slots; s += 1024) slot_offsets[s] = off(groups);
+  // the list's end: of the unused slots, and of the last one where the caller's bound is too low
+  for (int s = (carry < slots ? carry : slots) + t; s <= slots; s += 1024) slot_offsets[s] = off(groups);
 }
 
 __global__ __launch_bounds__(1024) void slice_rows_kernel(const int64_t* __restrict__ offsets, int64_t n, int groups,
