@@ -323,7 +323,9 @@ def _grouped(x: torch.Tensor, k: int, offsets: torch.Tensor, groups: int, index,
     ws = torch.empty(max(need, 256), dtype=torch.uint8, device=gpu)
     out = torch.empty(groups, kp, kp, dtype=torch.float32, device=gpu)
     denominators = torch.empty(groups, dtype=torch.float64, device=gpu)
-    N.call("kq_grouped_covariance", code, N.ptr(x), kp, N.ptr(offsets), groups, N.ptr(index), N.ptr(weights), rows,
+    # offsets from the host last: the copy waits for the stream, and what is done after it is not hidden
+    o = N.aligned(offsets.to(gpu, torch.int64), 8)
+    N.call("kq_grouped_covariance", code, N.ptr(x), kp, N.ptr(o), groups, N.ptr(index), N.ptr(weights), rows,
            kp, N.ptr(out), N.ptr(denominators), flags, N.ptr(ws), ws.numel(), N.stream(gpu))
     del ws
     if kp != k:
@@ -395,13 +397,12 @@ def expert_hessians_from_rows(
         raise ValueError("offsets must rise from 0 to at most the number of rows")
     if weights is not None and (weights.ndim != 1 or weights.shape[0] < int(host_offsets[-1])):
         raise ValueError("weights must cover every grouped row")
-    (x, o, w), gpu, _ = N.to_gpu([rows, offsets, weights])
+    (x, w, _), gpu, _ = N.to_gpu([rows, weights, offsets if offsets.is_cuda else None])
     x, k = _prepare_rows(x, gpu)
-    o = N.aligned(o.to(torch.int64), 8)
     if w is not None:
         w = N.aligned(w.float(), 4)
     flags = N.SYRK_SQUARE_WEIGHTS if square_weights else 0
-    return _grouped(x, k, o, int(o.numel()) - 1, None, w, flags, int(host_offsets[-1]))
+    return _grouped(x, k, offsets.detach(), int(offsets.numel()) - 1, None, w, flags, int(host_offsets[-1]))
 
 
 def build_expert_hessians(

@@ -854,8 +854,8 @@ __device__ __forceinline__ void syrk4_wait(int n) {
 }
 
 // Persistent: the `gridDim.x` workgroups take the items (group rank, tile) in
-// order, each its next one from a counter (`queue`, zero before the launch)
-// when it has done the last: ranks order the groups by row count, largest
+// order, each its next one from a counter (`queue`, zero before the launch,
+// with unused slots' groups empty and last) when it has done the last: ranks order the groups by row count, largest
 // first (ties by index, computed once per workgroup in LDS for up to
 // LPT_MAX_GROUPS groups, natural order beyond), so this is longest-first
 // scheduling.  Without a queue they walk them in snake order (round q gives
@@ -924,9 +924,6 @@ __global__ __launch_bounds__(512, 1) void syrk256w_dma_kernel(
 
   int64_t item = blockIdx.x;
   for (int64_t q = 0; item < items; ++q) {
-    // the next item's number is on its way while this one runs
-    int taken = 0;
-    if (queue && tid == 0) taken = grid + atomicAdd(queue, 1);
     const int rank = (int)(item / ntiles);
     const int64_t g = lpt ? syrk4_rank_order[rank] : rank;
     int ti, tj;
@@ -935,6 +932,7 @@ __global__ __launch_bounds__(512, 1) void syrk256w_dma_kernel(
     const int64_t row0 = (int64_t)ti * TILE, col0 = (int64_t)tj * TILE;
     const int64_t list0 = offsets[g];
     const int n = (int)(offsets[g + 1] - list0);
+    if (queue && n == 0) break;  // an unused slot: the rest are too
     const int per_step = LPW * (share ? 1 : 2) + (wave == 0 ? 1 : 0);
 
     float16_t accv[2][4];
@@ -946,6 +944,7 @@ __global__ __launch_bounds__(512, 1) void syrk256w_dma_kernel(
         for (int r = 0; r < 16; ++r) accv[i][j][r] = 0.0f;
 
     const int steps = (n + BK - 1) / BK;
+    int taken = 0;
     if (steps > 0) {
       // a chunk past feature k (edge tiles) reads feature 0 instead: such
       // features only reach accumulator rows / columns past k, never stored
@@ -1003,6 +1002,15 @@ __global__ __launch_bounds__(512, 1) void syrk256w_dma_kernel(
       // which keeps the per-step count of outstanding loads fixed.
 #pragma unroll
       for (int st = 0; st < NS - 1; ++st) issue(st, st * BK);
+      // the next item's number, on its way while this one runs (wave 0's waits
+      // count one operation more than they need until it has come)
+      if (queue && tid == 0) {
+        // an offset the compiler takes for a lane's own: an add to a uniform
+        // address is waited for at once, to share its result out over the wave
+        int at = 0;
+        asm volatile("" : "+v"(at));
+        taken = atomicAdd(queue + at, 1);
+      }
       syrk4_wait(per_step * (NS - 2));  // step 0 has landed
       convert(0, 0);
       int stage = 0;
@@ -1048,19 +1056,14 @@ __global__ __launch_bounds__(512, 1) void syrk256w_dma_kernel(
         }
         stage = next;
       }
+      // two slots: the one written now was last read before the previous barrier
+      if (queue && tid == 0) syrk4_next[q & 1] = grid + taken;
       __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // the loads issued past the end have landed
       __syncthreads();                            // every wave is done with the ring
     }
     if (n > 0 || !skip_empty)
       syrk3_store(accv, acc + g * k * k + row0 * k + col0, k, k - row0, k - col0, true, wave, lane);
-    if (queue) {
-      // two slots: the one written now was last read before the previous barrier
-      if (tid == 0) syrk4_next[q & 1] = taken;
-      __syncthreads();
-      item = syrk4_next[q & 1];
-    } else {
-      item = (q + 1) * grid + ((q & 1) ? blockIdx.x : grid - 1 - blockIdx.x);
-    }
+    item = queue ? syrk4_next[q & 1] : (q + 1) * grid + ((q & 1) ? blockIdx.x : grid - 1 - blockIdx.x);
   }
 }
 
@@ -1103,7 +1106,8 @@ static hipError_t launch_syrk256(const void* x, int64_t ld, int64_t n, int64_t k
 // halves, (acc[i][j] inv + acc[j][i] inv) / 2 (kquant's (H + H^T) / 2), each
 // product and the sum rounded on its own, with the diagonal acc[i][i] inv.
 constexpr int FIN_B = 64;
-template <bool FULL>
+// SLICED: acc is the sum of `planes` (0: zeros), `plane` floats apart.
+template <bool FULL, bool SLICED>
 __device__ __forceinline__ void finalize_pair_impl(const float* __restrict__ a, int64_t lda, int64_t k,
                                                    float inv, float* __restrict__ o, int64_t ldo, int64_t bi,
                                                    int64_t bj, float (*t)[FIN_B][FIN_B + 1], int planes,
@@ -1119,27 +1123,29 @@ __device__ __forceinline__ void finalize_pair_impl(const float* __restrict__ a, 
 #pragma unroll
   for (int q = 0; q < R; ++q) {
     const int64_t i = i0 + ty + 4 * q, j = j0 + tx;
-    u[q] = planes > 0 && (FULL || (i < k && j < k)) ? a[i * lda + j] : 0.0f;
+    u[q] = (!SLICED || planes > 0) && (FULL || (i < k && j < k)) ? a[i * lda + j] : 0.0f;
   }
-  for (int p = 1; p < planes; ++p)  // a group's row slices, in order
+  if constexpr (SLICED)
+    for (int p = 1; p < planes; ++p)  // a group's row slices, in order
 #pragma unroll
-    for (int q = 0; q < R; ++q) {
-      const int64_t i = i0 + ty + 4 * q, j = j0 + tx;
-      if (FULL || (i < k && j < k)) u[q] += a[p * plane + i * lda + j];
-    }
+      for (int q = 0; q < R; ++q) {
+        const int64_t i = i0 + ty + 4 * q, j = j0 + tx;
+        if (FULL || (i < k && j < k)) u[q] += a[p * plane + i * lda + j];
+      }
   if (two) {
     float l[R];
 #pragma unroll
     for (int q = 0; q < R; ++q) {
       const int64_t p = j0 + ty + 4 * q, c = i0 + tx;
-      l[q] = planes > 0 && (FULL || (p < k && c < k)) ? a[p * lda + c] : 0.0f;
+      l[q] = (!SLICED || planes > 0) && (FULL || (p < k && c < k)) ? a[p * lda + c] : 0.0f;
     }
-    for (int s = 1; s < planes; ++s)
+    if constexpr (SLICED)
+      for (int s = 1; s < planes; ++s)
 #pragma unroll
-      for (int q = 0; q < R; ++q) {
-        const int64_t p = j0 + ty + 4 * q, c = i0 + tx;
-        if (FULL || (p < k && c < k)) l[q] += a[s * plane + p * lda + c];
-      }
+        for (int q = 0; q < R; ++q) {
+          const int64_t p = j0 + ty + 4 * q, c = i0 + tx;
+          if (FULL || (p < k && c < k)) l[q] += a[s * plane + p * lda + c];
+        }
 #pragma unroll
     for (int q = 0; q < R; ++q) t[1][ty + 4 * q][tx] = l[q];
   }
@@ -1171,13 +1177,14 @@ __device__ __forceinline__ void finalize_pair_impl(const float* __restrict__ a, 
   }
 }
 
+template <bool SLICED = false>
 __device__ __forceinline__ void finalize_pair(const float* __restrict__ a, int64_t lda, int64_t k, float inv,
                                               float* __restrict__ o, int64_t ldo, int64_t bi, int64_t bj,
                                               float (*t)[FIN_B][FIN_B + 1], int planes = 1, int64_t plane = 0) {
   if ((bj + 1) * FIN_B <= k)  // bi <= bj: the whole pair is inside the matrix
-    finalize_pair_impl<true>(a, lda, k, inv, o, ldo, bi, bj, t, planes, plane);
+    finalize_pair_impl<true, SLICED>(a, lda, k, inv, o, ldo, bi, bj, t, planes, plane);
   else
-    finalize_pair_impl<false>(a, lda, k, inv, o, ldo, bi, bj, t, planes, plane);
+    finalize_pair_impl<false, SLICED>(a, lda, k, inv, o, ldo, bi, bj, t, planes, plane);
 }
 
 // block pair b of the upper triangle of nb x nb blocks -> (bi <= bj)
@@ -1285,19 +1292,31 @@ __global__ __launch_bounds__(256) void cov_stats_final_kernel(const double* __re
 }
 
 // Grouped finalize: out[g] = sym(acc[g]) / denominators[g] (zeros when the
-// group has no weight), blockIdx.y = group.  With `first`, acc holds row
-// slices: group g is the sum of planes first[g] .. first[g + 1] - 1.
+// group has no weight), blockIdx.y = group.  SLICED: acc holds row slices, and
+// group g is the sum of planes first[g] .. first[g + 1] - 1.  Otherwise, with
+// `offsets`, a group without rows has no plane (SYRK_SLOTS) and is zeros.
+template <bool SLICED>
 __global__ __launch_bounds__(256) void syrk_finalize_grouped_kernel(
     const float* __restrict__ acc, int64_t k, const double* __restrict__ denominators,
-    float* __restrict__ out, const int* __restrict__ first) {
+    float* __restrict__ out, const int* __restrict__ first, const int64_t* __restrict__ offsets) {
   __shared__ float t[2][FIN_B][FIN_B + 1];
   const int64_t g = blockIdx.y;
   const double d = denominators[g];
   const float inv = d > 0.0 ? (float)(1.0 / d) : 0.0f;
   int64_t bi, bj;
   finalize_pair_of(blockIdx.x, bi, bj);
-  const int64_t p0 = first ? first[g] : g;
-  finalize_pair(acc + p0 * k * k, k, k, inv, out + g * k * k, k, bi, bj, t, first ? first[g + 1] - first[g] : 1, k * k);
+  float* o = out + g * k * k;
+  if constexpr (SLICED) {
+    finalize_pair<true>(acc + first[g] * k * k, k, k, inv, o, k, bi, bj, t, first[g + 1] - first[g], k * k);
+  } else if (offsets && offsets[g + 1] == offsets[g]) {
+    for (int e = threadIdx.x; e < FIN_B * FIN_B; e += 256) {
+      const int64_t r = e / FIN_B, c = e % FIN_B, i0 = bi * FIN_B, j0 = bj * FIN_B;
+      if (i0 + r < k && j0 + c < k) o[(i0 + r) * k + j0 + c] = 0.0f;
+      if (j0 + r < k && i0 + c < k) o[(j0 + r) * k + i0 + c] = 0.0f;
+    }
+  } else {
+    finalize_pair(acc + g * k * k, k, k, inv, o, k, bi, bj, t);
+  }
 }
 
 // Row slices.  A group whose tiles are too few or too long for the CUs (one
@@ -1306,10 +1325,9 @@ __global__ __launch_bounds__(256) void syrk_finalize_grouped_kernel(
 // a group of its own into its slot's k x k plane; the finalize (or
 // slot_sum_kernel) adds a group's slots in order, so results stay
 // deterministic.  One slice -> sliced: weighted bf16 6110 rows x 416 486 -> 73 us,
-// 4820 x 3824 435 -> 262; f32 5446 x 2832 1057 -> 709; 17 routed experts of
-// 10293 rows x 552 156 -> 106; 65536 rows in 48 Zipf groups x 2048 928 -> 883 (the
-// queue and the slices of the hot experts; the planes' finalize reads no more
-// than the accumulators' did).  One workgroup writes the slots' row offsets (slot s owns
+// 4820 x 3824 435 -> 262; f32 5446 x 2832 1057 -> 709; 17 experts of
+// 40000 rows x 552 282 -> 128; 65536 rows in 48 Zipf groups x 2048 943 -> 890 (the
+// queue; the planes' finalize reads no more than the accumulators' did).  One workgroup writes the slots' row offsets (slot s owns
 // list positions [slot_offsets[s], slot_offsets[s + 1]); unused slots at the
 // end are empty), each group's first slot, and clears the item queue.
 __device__ __forceinline__ void slice_rows(const int64_t* __restrict__ offsets, int64_t n, int groups, int64_t rows,
@@ -1519,13 +1537,18 @@ static hipError_t launch_syrk(const void* x, int64_t ld, int64_t n, int64_t k, c
   return hipGetLastError();
 }
 
+// Weighted bf16 rows without an index: syrk256w_dma_kernel.
+static bool dma_groups(int in_dtype, const void* weights, const void* row_index) {
+  return in_dtype == KQ_DT_BF16 && weights && !row_index;
+}
+
 // One grouped launch over acc [groups, k, k].  overwrite: 1, or SYRK_SLOTS
 // (empty groups write nothing); queue: a zeroed item counter or NULL.
 static hipError_t launch_grouped(int in_dtype, const void* x, int64_t ld, const int64_t* offsets, int groups,
                                  const int32_t* index, const float* w, int64_t k, float* acc, int overwrite, int sq,
                                  int* queue, hipStream_t st) {
   if (in_dtype == KQ_DT_BF16) {
-    if (w && !index) return launch_syrk256w_dma(x, ld, k, w, acc, offsets, groups, sq, st, queue, overwrite == SYRK_SLOTS);
+    if (dma_groups(in_dtype, w, index)) return launch_syrk256w_dma(x, ld, k, w, acc, offsets, groups, sq, st, queue, overwrite == SYRK_SLOTS);
     return w ? launch_syrk256<true, true>(x, ld, 0, k, w, acc, k, overwrite, st, offsets, index, groups, sq)
              : launch_syrk256<false, true>(x, ld, 0, k, w, acc, k, overwrite, st, offsets, index, groups, sq);
   }
@@ -1536,20 +1559,22 @@ static hipError_t launch_grouped(int in_dtype, const void* x, int64_t ld, const 
            : launch_syrk<2, true, false, true>(x, ld, 0, k, w, acc, k, overwrite, st, offsets, index, groups, sq);
 }
 
-// Row slices of a launch: at most `rows` rows each, in `slots` planes.
+// Row slices of a launch: at most `rows` rows each, in `slots` planes; not
+// `sliced`, a plane for each group.
 struct SlicePlan {
   int64_t rows;
   int slots;
+  bool sliced;
 };
-struct SliceSpace {  // workspace offsets: item queue, first slots, slot offsets, planes
-  int64_t first, offsets, planes, total;
+struct SliceSpace {  // workspace: the planes at 0, then item queue, first slots, slot offsets
+  int64_t queue, first, offsets, total;
 };
-static SliceSpace slice_space(int groups, int slots, int64_t k) {
+static SliceSpace slice_space(int groups, const SlicePlan& p, int64_t k) {
   SliceSpace s;
-  s.first = 256;
+  s.queue = (int64_t)p.slots * k * k * 4;  // k % 8 == 0: a multiple of 256
+  s.first = s.queue + 256;
   s.offsets = s.first + ((int64_t)(groups + 1) * 4 + 255) / 256 * 256;
-  s.planes = s.offsets + ((int64_t)(slots + 1) * 8 + 255) / 256 * 256;
-  s.total = s.planes + (int64_t)slots * k * k * 4;
+  s.total = p.sliced ? s.offsets + ((int64_t)(p.slots + 1) * 8 + 255) / 256 * 256 : s.queue;
   return s;
 }
 static int64_t upper_tiles(int in_dtype, int64_t k) {
@@ -1557,27 +1582,42 @@ static int64_t upper_tiles(int in_dtype, int64_t k) {
   return nt * (nt + 1) / 2;
 }
 
-// Grouped rows (`rows` in all at most): no slice longer than a CU's mean
-// share of the rows (twice that where the groups give a CU half to four items:
-// shorter slices would only add rounds), and none shorter than 256 rows (16
-// steps of the matrix loop against the 4 us of a tile's stores).
-static SlicePlan plan_group_slices(int in_dtype, int64_t rows, int64_t k, int groups, int cus) {
-  const int64_t tiles = upper_tiles(in_dtype, k), share = rows * tiles / (cus > 0 ? cus : 256);
-  int64_t cut = tiles * groups >= 4 * cus || 2 * tiles * groups < cus ? share : 2 * share;
+// Grouped rows (`rows` in all at most).  No slice is longer than a CU's mean
+// share of the rows (twice that where the groups give a CU half to four
+// items, and in between what fills the CUs once: shorter slices would only
+// add rounds), and none shorter than 256 rows (16 steps of the matrix loop
+// against the 4 us of a tile's stores).
+//
+// Slicing costs a launch ahead of the SYRK, the slots' bookkeeping and more
+// planes to add, so it is done where it can shorten the longest group by 14 us
+// of the kernel's time per row; the longest is taken to hold an eighth of the
+// rows (an expert that every token chooses among its eight) or the mean.  The
+// direct-load kernel also takes the item queue that comes with the slices from
+// two items a CU on.  Weighted bf16, rows in all, k, groups of Zipf popularity, us
+// without / with slices: 2048 x 1024, 48: 111 / 116; 4096 x 1024, 48: 120 / 121;
+// 30000 x 1200, 20: 254 / 271 | 4096 x 512, 48: 81 / 72; 8192 x 1024, 48: 143 / 135;
+// 16384 x 256, 24: 138 / 69; 8192 x 2048, 16 (the queue): 203 / 195.  f32 8192 x
+// 1024, 48: 295 / 297; 8192 x 256, 4: 264 / 75.
+static SlicePlan plan_group_slices(int in_dtype, int64_t rows, int64_t k, int groups, bool dma, int cus) {
+  if (cus <= 0) cus = 256;
+  const int64_t tiles = upper_tiles(in_dtype, k), items = tiles * groups, share = rows * tiles / cus;
+  int64_t cut = items >= 4 * cus ? share : 2 * items >= cus ? 2 * share : rows * tiles / (cus - items);
   // 65535: the grid's limit on slots
   const int64_t least = groups < 65535 ? rows / (65536 - groups) + 1 : rows + 1;
   cut = cut < 256 ? 256 : cut;
   cut = ((cut < least ? least : cut) + 63) / 64 * 64;
-  return {cut, groups + (int)(rows / cut)};
+  const double row_us = dma ? 0.055 : 0.09;
+  const int64_t longest = groups < 8 ? (rows + groups - 1) / groups : rows / 8;
+  if ((double)(longest - cut) * row_us < 14.0 && !(dma && items >= 2 * cus)) return {rows, groups, false};
+  return {cut, groups + (int)(rows / cut), true};
 }
-
 // One group of n rows: S slices minimising the rounds of (tile, slice) items
 // times a slice's time (measured per row and tile, a few us to write it) plus
 // the planes written and summed at 4.5 TB/s.
 static SlicePlan plan_row_slices(int in_dtype, int64_t n, int64_t k, int cus) {
   const double row_us = in_dtype == KQ_DT_BF16 ? 0.07 : 0.10;
   const int64_t tiles = upper_tiles(in_dtype, k), tile = in_dtype == KQ_DT_BF16 ? syrk2::TILE : syrk::TILE;
-  SlicePlan best{(n + 63) / 64 * 64, 1};
+  SlicePlan best{(n + 63) / 64 * 64, 1, false};
   if (cus <= 0) return best;
   double best_us = 0.95 * ((double)((tiles + cus - 1) / cus) * ((double)n * row_us + 4.0));
   for (int64_t s = 2; s <= 64 && n / s >= 128; ++s) {
@@ -1586,7 +1626,7 @@ static SlicePlan plan_row_slices(int in_dtype, int64_t n, int64_t k, int cus) {
                       (double)(s * tiles * tile * tile * 8) / 4.5e6;
     if (us < best_us) {
       best_us = us;
-      best = {part, (int)((n + part - 1) / part)};
+      best = {part, (int)((n + part - 1) / part), true};
     }
   }
   return best;
@@ -1618,7 +1658,7 @@ extern "C" int64_t kq_syrk_sliced_workspace_size(int in_dtype, int64_t n, int64_
     return kq_syrk_accumulate_workspace_size(in_dtype, n, k, weighted);
   if (k > SLICE_MAX_K) return 0;
   const SlicePlan p = plan_row_slices(in_dtype, n, k, device_cus());
-  return p.slots > 1 ? slice_space(1, p.slots, k).total : 0;
+  return p.sliced ? slice_space(1, p, k).total : 0;
 }
 
 extern "C" int kq_syrk_accumulate_ws(int in_dtype, const void* x, int64_t ld, int64_t n, int64_t k,
@@ -1655,14 +1695,15 @@ static int syrk_accumulate(int in_dtype, const void* x, int64_t ld, int64_t n, i
   const bool weighted = weights != nullptr;
   if (workspace && k <= SLICE_MAX_K && !dma_syrk(in_dtype, weights, n, ld)) {
     const SlicePlan p = plan_row_slices(in_dtype, n, k, device_cus(st));
-    const SliceSpace sp = slice_space(1, p.slots, k);
-    if (p.slots > 1 && sp.total <= ws_bytes) {
+    const SliceSpace sp = slice_space(1, p, k);
+    if (p.sliced && sp.total <= ws_bytes) {
       unsigned char* w = (unsigned char*)workspace;
       int64_t* so = (int64_t*)(w + sp.offsets);
-      float* planes = (float*)(w + sp.planes);
-      slice_rows_kernel<<<1, 1024, 0, st>>>(nullptr, n, 1, p.rows, p.slots, so, (int*)(w + sp.first), (int*)w);
+      float* planes = (float*)w;
+      int* queue = (int*)(w + sp.queue);
+      slice_rows_kernel<<<1, 1024, 0, st>>>(nullptr, n, 1, p.rows, p.slots, so, (int*)(w + sp.first), queue);
       if ((e = hipGetLastError()) != hipSuccess) return kq_check_launch(e, "kq_syrk_accumulate/slices");
-      e = launch_grouped(in_dtype, x, ld, so, p.slots, nullptr, weights, k, planes, SYRK_SLOTS, 0, (int*)w, st);
+      e = launch_grouped(in_dtype, x, ld, so, p.slots, nullptr, weights, k, planes, SYRK_SLOTS, 0, queue, st);
       if (e != hipSuccess) return kq_check_launch(e, "kq_syrk_accumulate/sliced");
       slot_sum_kernel<<<dim3((unsigned)((k + 255) / 256), (unsigned)k), 256, 0, st>>>(
           planes, p.slots, k, in_dtype == KQ_DT_BF16 ? syrk2::TILE : syrk::TILE, acc, ld_acc, overwrite);
@@ -1748,14 +1789,17 @@ extern "C" int kq_syrk_finalize_grouped(const float* acc, int64_t k, int groups,
   if (k > 65535) return kq_fail(KQ_ERR_LIMIT, "kq_syrk_finalize_grouped: k too large");
   hipStream_t st = (hipStream_t)stream;
   const int64_t nb = (k + FIN_B - 1) / FIN_B;
-  syrk_finalize_grouped_kernel<<<dim3((unsigned)(nb * (nb + 1) / 2), (unsigned)groups), 256, 0, st>>>(
-      acc, k, denominators, out, nullptr);
+  syrk_finalize_grouped_kernel<false><<<dim3((unsigned)(nb * (nb + 1) / 2), (unsigned)groups), 256, 0, st>>>(
+      acc, k, denominators, out, nullptr, nullptr);
   return kq_check_launch(hipGetLastError(), "kq_syrk_finalize_grouped");
 }
 
 extern "C" int64_t kq_grouped_covariance_workspace_size(int in_dtype, int64_t rows, int64_t k, int groups) {
   if (rows < 0 || k <= 0 || groups < 1 || in_dtype < KQ_DT_BF16 || in_dtype > KQ_DT_F32) return -1;
-  return slice_space(groups, plan_group_slices(in_dtype, rows, k, groups, device_cus()).slots, k).total;
+  const int cus = device_cus();
+  const int64_t a = slice_space(groups, plan_group_slices(in_dtype, rows, k, groups, false, cus), k).total;
+  const int64_t b = slice_space(groups, plan_group_slices(in_dtype, rows, k, groups, in_dtype == KQ_DT_BF16, cus), k).total;
+  return a > b ? a : b;
 }
 
 extern "C" int kq_grouped_covariance(int in_dtype, const void* x, int64_t ld, const int64_t* offsets, int groups,
@@ -1777,24 +1821,33 @@ extern "C" int kq_grouped_covariance(int in_dtype, const void* x, int64_t ld, co
   if (k > SLICE_MAX_K) return kq_fail(KQ_ERR_LIMIT, "%s: k=%lld exceeds %lld", fn, (long long)k, (long long)SLICE_MAX_K);
   hipStream_t st = (hipStream_t)stream;
   // the plan of the current device's CU count, as the size function makes it
-  const SlicePlan p = plan_group_slices(in_dtype, rows, k, groups, device_cus());
-  const SliceSpace sp = slice_space(groups, p.slots, k);
+  const SlicePlan p = plan_group_slices(in_dtype, rows, k, groups, dma_groups(in_dtype, weights, row_index), device_cus());
+  const SliceSpace sp = slice_space(groups, p, k);
   if (workspace_bytes < sp.total)
     return kq_fail(KQ_ERR_INVALID, "%s: workspace needs %lld bytes", fn, (long long)sp.total);
   unsigned char* w = (unsigned char*)workspace;
   int* first = (int*)(w + sp.first);
   int64_t* so = (int64_t*)(w + sp.offsets);
-  float* planes = (float*)(w + sp.planes);
+  float* planes = (float*)w;
+  int* queue = (int*)(w + sp.queue);
   hipError_t e;
   const int sq = (flags & KQ_SYRK_SQUARE_WEIGHTS) ? 1 : 0;
-  prepare_groups_kernel<<<groups + 1, 1024, 0, st>>>(weights, offsets, sq, denominators, groups, p.rows, p.slots, so,
-                                                     first, (int*)w);
-  if ((e = hipGetLastError()) != hipSuccess) return kq_check_launch(e, fn);
-  e = launch_grouped(in_dtype, x, ld, so, p.slots, row_index, weights, k, planes, SYRK_SLOTS, sq, (int*)w, st);
-  if (e != hipSuccess) return kq_check_launch(e, fn);
   const int64_t nb = (k + FIN_B - 1) / FIN_B;
-  syrk_finalize_grouped_kernel<<<dim3((unsigned)(nb * (nb + 1) / 2), (unsigned)groups), 256, 0, st>>>(
-      planes, k, denominators, out, first);
+  const dim3 pairs((unsigned)(nb * (nb + 1) / 2), (unsigned)groups);
+  if (!p.sliced) {
+    e = launch_grouped(in_dtype, x, ld, offsets, groups, row_index, weights, k, planes, SYRK_SLOTS, sq, nullptr, st);
+    if (e != hipSuccess) return kq_check_launch(e, fn);
+    segment_weight_sum_kernel<<<groups, 1024, 0, st>>>(weights, offsets, sq, denominators);
+    if ((e = hipGetLastError()) != hipSuccess) return kq_check_launch(e, fn);
+    syrk_finalize_grouped_kernel<false><<<pairs, 256, 0, st>>>(planes, k, denominators, out, nullptr, offsets);
+    return kq_check_launch(hipGetLastError(), fn);
+  }
+  prepare_groups_kernel<<<groups + 1, 1024, 0, st>>>(weights, offsets, sq, denominators, groups, p.rows, p.slots, so,
+                                                     first, queue);
+  if ((e = hipGetLastError()) != hipSuccess) return kq_check_launch(e, fn);
+  e = launch_grouped(in_dtype, x, ld, so, p.slots, row_index, weights, k, planes, SYRK_SLOTS, sq, queue, st);
+  if (e != hipSuccess) return kq_check_launch(e, fn);
+  syrk_finalize_grouped_kernel<true><<<pairs, 256, 0, st>>>(planes, k, denominators, out, first, nullptr);
   return kq_check_launch(hipGetLastError(), fn);
 }
 

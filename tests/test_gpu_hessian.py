@@ -475,3 +475,33 @@ def test_sliced_groups(gpu, k, experts, dtype):
                 continue
             ref = _f64_covariance(x[a:b], wt[a:b])
             assert float((h[e].double() - ref).norm() / ref.norm()) <= TOL, e
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("k,groups,most", [(264, 30, 40), (1100, 40, 15)])
+def test_short_groups(gpu, k, groups, most, dtype):
+    """Groups too short to slice, first and last one empty: a plane each (the
+    first shape, and every kernel but the weighted bf16 list's), or the item
+    queue over whole groups (the second: two items a CU)."""
+    print(f"case short groups k={k} groups={groups} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(k)
+    counts = torch.randint(0, most, (groups,), generator=g)
+    counts[0] = counts[7] = counts[-1] = 0
+    offsets = torch.zeros(groups + 1, dtype=torch.int64)
+    offsets[1:] = counts.cumsum(0)
+    total = int(offsets[-1])
+    x = workloads.student_t4(total, k, seed=k, dtype=dtype).to(gpu)
+    w = (torch.rand(total, generator=g) + 0.1).to(gpu)
+    ids = torch.repeat_interleave(torch.arange(groups), counts).to(torch.int32)[:, None]
+    torch.full((groups, k, k), float("nan"), device=gpu)  # planes that nothing writes hold NaN
+    for h, den in (ch.expert_hessians_from_rows(x, offsets, w),
+                   ch.expert_hessians_from_rows(x, offsets.to(gpu), w),
+                   ch.expert_hessians(x, ids.to(gpu), w[:, None], groups, gate_square=False)[:2]):
+        for e in range(groups):
+            a, b = int(offsets[e]), int(offsets[e + 1])
+            if a == b:
+                assert float(den[e]) == 0.0 and torch.equal(h[e], torch.zeros_like(h[e]))
+                continue
+            ref = _f64_covariance(x[a:b], w[a:b])
+            assert float((h[e].double() - ref).norm() / ref.norm()) <= TOL, e
+            assert float(den[e]) == pytest.approx(float(w[a:b].double().sum()), rel=1e-12)

@@ -78,6 +78,22 @@ def test_linear_a8_argument_errors_need_no_gpu():
     assert lib.kq_mx_linear_mm(*bad) == _native.KQ_ERR_INVALID and b"input dtype" in lib.kq_last_error()
 
 
+def test_grouped_covariance_slices_only_where_it_pays():
+    """The workspace tells the plan (without a GPU it is that of 256 CUs): a
+    k x k plane per group where no group is sliced, more and the slices'
+    bookkeeping where a hot group is long against a CU's share."""
+    size = _native.library().kq_grouped_covariance_workspace_size
+    planes = lambda slots, k: slots * k * k * 4  # noqa: E731
+    for dtype, rows, k, groups in ((_native.DT_BF16, 1024, 1024, 30), (_native.DT_BF16, 2048, 768, 24),
+                                   (_native.DT_BF16, 4096, 1536, 12), (_native.DT_F32, 8192, 1024, 48),
+                                   (_native.DT_F32, 512, 1624, 5), (_native.DT_F16, 2048, 1024, 48)):
+        assert size(dtype, rows, k, groups) == planes(groups, k)
+    # an item queue for many short groups of the direct-load kernel: bookkeeping, and a few more planes
+    assert planes(48, 2048) < size(_native.DT_BF16, 1024, 2048, 48) < planes(53, 2048)
+    for dtype, rows, k, groups in ((_native.DT_BF16, 65536, 512, 8), (_native.DT_F32, 8192, 256, 4)):
+        assert size(dtype, rows, k, groups) > planes(2 * groups, k)
+
+
 def test_x4t_moe_argument_errors_need_no_gpu():
     lib = _native.library()
     per_expert = 2 * 2048 * 7168 // 32 + 7168 * 2048 // 32  # w13 and w2 scale bytes
