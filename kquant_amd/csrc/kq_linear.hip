@@ -877,6 +877,16 @@ static SplitPlan plan_split(int64_t m, int64_t n, int64_t k, double step_us, int
   return p;
 }
 
+// The plan as it can run: whole tiles where its planes don't fit the
+// workspace or one launch does not cover the operands.
+static SplitPlan plan_within(SplitPlan p, int64_t plane_bytes, bool one_launch) {
+  if (p.bytes > plane_bytes || !one_launch) {
+    p.slices = 1;
+    p.bytes = 0;
+  }
+  return p;
+}
+
 static hipError_t stream_cus(hipStream_t st, int* cus) {
   int dev = 0;
   hipError_t e = st ? hipStreamGetDevice(st, &dev) : hipGetDevice(&dev);
@@ -992,20 +1002,13 @@ static hipError_t launch_linear(const uint16_t* a, int64_t lda, const uint8_t* w
   return hipGetLastError();
 }
 
-// launch_linear, split over K into `planes` (plane_bytes of workspace) where
-// that pays and fits.
+// launch_linear as planned: split over K into `planes`, or whole tiles.
 template <int FMT, int OUT>
 static hipError_t launch_linear_split(const uint16_t* a, int64_t lda, const uint8_t* wq, const uint8_t* ws, void* c,
-                                      int64_t ldc, int M, int N, int K, int KB, void* planes, int64_t plane_bytes,
+                                      int64_t ldc, int M, int N, int K, int KB, const SplitPlan& p, void* planes,
                                       hipStream_t st) {
-  int cus = 0;
-  hipError_t e = stream_cus(st, &cus);
-  if (e != hipSuccess) return e;
-  const bool dma_path = takes_dma(FMT, lda, ws, KB);
-  const SplitPlan p = plan_split(M, N, K, dma_path ? DMA_STEP_US : STAGED_STEP_US, cus);
-  if (p.slices <= 1 || p.bytes > plane_bytes || !one_range(2 * lda, FMT == 0 ? KB : KB / 2, M, N))
-    return launch_linear<FMT, OUT>(a, lda, wq, ws, c, ldc, M, N, K, KB, st);
-  e = launch_linear<FMT, 2>(a, lda, wq, ws, planes, p.ldp, M, N, K, KB, st, p.slices, p.plane);
+  if (p.slices <= 1) return launch_linear<FMT, OUT>(a, lda, wq, ws, c, ldc, M, N, K, KB, st);
+  const hipError_t e = launch_linear<FMT, 2>(a, lda, wq, ws, planes, p.ldp, M, N, K, KB, st, p.slices, p.plane);
   return e == hipSuccess ? sum_planes<OUT>(p, planes, M, N, c, ldc, st) : e;
 }
 
@@ -1052,18 +1055,21 @@ hipError_t split3_rows(const float* a, int64_t lda, int64_t m, int64_t k, uint16
 // K with its second launch ~45).  At 33 .. 64 rows the split product passes it
 // where K is long (K = 7168, N = 5000, 48 rows: 33 against 57 us) but not
 // where its two launches dominate (K = 1024: 15 against 21 us; fp32 rows, a
-// third launch, also at N <= 2048: 37 against 46 us), nor without a workspace
-// for its planes (137 us).
-static bool takes_skinny(int64_t m, int64_t n, int64_t k, bool f32_rows, const uint8_t* w_scale, bool planes_fit) {
+// third launch, also at N <= 2048: 37 against 46 us), nor unsplit (137 us).
+// p: the tiles' plan as it can run with the caller's workspace.
+static bool takes_skinny(int64_t m, int64_t n, int64_t k, bool f32_rows, const uint8_t* w_scale, const SplitPlan& p) {
   if (k % 128 == 0 && kq_misaligned(w_scale, 4)) return false;
-  return m <= 32 || (m <= 64 && (k <= 2048 || (f32_rows && n <= 2048) || !planes_fit));
+  return m <= 32 || (m <= 64 && (k <= 2048 || (f32_rows && n <= 2048) || p.slices <= 1));
 }
+
+static double step_us(bool dma) { return dma ? DMA_STEP_US : STAGED_STEP_US; }
 
 extern "C" int64_t kq_mx_linear_workspace_size(int64_t m, int64_t n, int64_t k) {
   if (m < 0 || n < 0 || k <= 0) return -1;
   const int cus = current_cus();
-  if (cus <= 0 || takes_skinny(m, n, k, false, nullptr, true)) return 0;
-  return plan_split(m, n, k, k % 128 ? STAGED_STEP_US : DMA_STEP_US, cus).bytes;
+  if (cus <= 0) return 0;
+  const SplitPlan p = plan_split(m, n, k, step_us(k % 128 == 0), cus);
+  return takes_skinny(m, n, k, false, nullptr, p) ? 0 : p.bytes;
 }
 
 extern "C" int kq_mx_linear(int w_fmt, const void* a, int64_t lda, const void* w_q,
@@ -1095,20 +1101,23 @@ extern "C" int kq_mx_linear_ws(int w_fmt, const void* a, int64_t lda, const void
   hipStream_t st = (hipStream_t)stream;
   const uint16_t* ap = (const uint16_t*)a;
   const uint8_t* wp = (const uint8_t*)w_q;
-  hipError_t e;
-  if (takes_skinny(m, n, k, false, w_scale, workspace_bytes > 0))
+  int cus = 0;
+  hipError_t e = stream_cus(st, &cus);
+  if (e != hipSuccess) return kq_check_launch(e, "kq_mx_linear");
+  const double step = step_us(takes_dma(w_fmt == KQ_FMT_MXFP8_E4M3 ? 0 : 1, lda, w_scale, k));
+  const SplitPlan p = plan_within(plan_split(m, n, k, step, cus), workspace_bytes,
+                                  one_range(2 * lda, w_fmt == KQ_FMT_MXFP8_E4M3 ? k : k / 2, m, n));
+  if (takes_skinny(m, n, k, false, w_scale, p))
     return kq_check_launch(mx_skinny_bf16(w_fmt, out_dtype == KQ_DT_F32,
                                           {a, nullptr, lda, wp, w_scale, c, ldc, (int)m, (int)n, (int)k}, st),
                            "kq_mx_linear");
-  auto split = [&](auto launch) {
-    return launch(ap, lda, wp, w_scale, c, ldc, (int)m, (int)n, (int)k, (int)k, workspace, workspace_bytes, st);
+  auto run = [&](auto launch) {
+    return launch(ap, lda, wp, w_scale, c, ldc, (int)m, (int)n, (int)k, (int)k, p, workspace, st);
   };
   if (w_fmt == KQ_FMT_MXFP8_E4M3)
-    e = out_dtype == KQ_DT_BF16 ? split(launch_linear_split<0, 0>)
-                                : split(launch_linear_split<0, 2>);
+    e = out_dtype == KQ_DT_BF16 ? run(launch_linear_split<0, 0>) : run(launch_linear_split<0, 2>);
   else
-    e = out_dtype == KQ_DT_BF16 ? split(launch_linear_split<1, 0>)
-                                : split(launch_linear_split<1, 2>);
+    e = out_dtype == KQ_DT_BF16 ? run(launch_linear_split<1, 0>) : run(launch_linear_split<1, 2>);
   return kq_check_launch(e, "kq_mx_linear");
 }
 
@@ -1123,8 +1132,9 @@ static int64_t f32_planes_offset(int64_t m, int64_t k) { return (m * 3 * k * 2 +
 extern "C" int64_t kq_mx_linear_f32_split_workspace_size(int64_t m, int64_t n, int64_t k) {
   if (m < 0 || n < 0 || k <= 0) return -1;
   const int cus = current_cus();
-  if (cus <= 0 || takes_skinny(m, n, k, true, nullptr, true)) return m * 3 * k * 2;
-  return f32_planes_offset(m, k) + plan_split(m, n, 3 * k, k % 128 ? STAGED_STEP_US : DMA_STEP_US, cus).bytes;
+  if (cus <= 0) return m * 3 * k * 2;
+  const SplitPlan p = plan_split(m, n, 3 * k, step_us(k % 128 == 0), cus);
+  return p.bytes == 0 || takes_skinny(m, n, k, true, nullptr, p) ? m * 3 * k * 2 : f32_planes_offset(m, k) + p.bytes;
 }
 
 extern "C" int kq_mx_linear_f32(int w_fmt, const float* a, int64_t lda, const void* w_q,
@@ -1148,7 +1158,12 @@ extern "C" int kq_mx_linear_f32(int w_fmt, const float* a, int64_t lda, const vo
     return kq_fail(KQ_ERR_INVALID, "kq_mx_linear_f32: a, w_q and workspace must be 16-byte aligned");
   if (m == 0 || n == 0) return KQ_OK;
   hipStream_t st = (hipStream_t)stream;
-  if (takes_skinny(m, n, k, true, w_scale, workspace_bytes > f32_planes_offset(m, k)))
+  int cus = 0;
+  if (int rc = kq_check_launch(stream_cus(st, &cus), "kq_mx_linear_f32")) return rc;
+  const int64_t off = f32_planes_offset(m, k), w_row = w_fmt == KQ_FMT_MXFP8_E4M3 ? k : k / 2;
+  const double step = step_us(takes_dma(w_fmt == KQ_FMT_MXFP8_E4M3 ? 0 : 1, 3 * k, w_scale, k));
+  const SplitPlan p = plan_within(plan_split(m, n, 3 * k, step, cus), workspace_bytes - off, one_range(6 * k, w_row, m, n));
+  if (takes_skinny(m, n, k, true, w_scale, p))
     return kq_check_launch(mx_skinny_f32(w_fmt, {a, nullptr, lda, (const uint8_t*)w_q, w_scale, c, ldc, (int)m, (int)n,
                                                  (int)k}, st),
                            "kq_mx_linear_f32");
@@ -1157,10 +1172,9 @@ extern "C" int kq_mx_linear_f32(int w_fmt, const float* a, int64_t lda, const vo
   split3_bf16_kernel<<<(unsigned)((quads + 255) / 256), 256, 0, st>>>(a, lda, m, k, a3);
   if (int rc = kq_check_launch(hipGetLastError(), "kq_mx_linear_f32")) return rc;
   const uint8_t* wp = (const uint8_t*)w_q;
-  const int64_t off = f32_planes_offset(m, k);
   auto* launch = w_fmt == KQ_FMT_MXFP8_E4M3 ? launch_linear_split<0, 2> : launch_linear_split<1, 2>;
-  const hipError_t e = launch(a3, 3 * k, wp, w_scale, c, ldc, (int)m, (int)n, (int)(3 * k), (int)k,
-                              static_cast<char*>(workspace) + off, workspace_bytes > off ? workspace_bytes - off : 0, st);
+  const hipError_t e = launch(a3, 3 * k, wp, w_scale, c, ldc, (int)m, (int)n, (int)(3 * k), (int)k, p,
+                              static_cast<char*>(workspace) + off, st);
   return kq_check_launch(e, "kq_mx_linear_f32");
 }
 
@@ -1189,8 +1203,9 @@ static int64_t mx_scale_planes(int64_t m, int64_t n, int64_t k) {
 extern "C" int64_t kq_mx_linear_mx_workspace_size(int64_t m, int64_t n, int64_t k) {
   if (m < 0 || n < 0 || k <= 0) return -1;
   const int cus = current_cus();
-  if (cus <= 0 || takes_skinny(m, n, k, false, nullptr, true)) return mx_scale_planes(m, n, k);
-  return mx_scale_planes(m, n, k) + plan_split(m, n, k, A8_STEP_US, cus).bytes;
+  if (cus <= 0) return mx_scale_planes(m, n, k);
+  const SplitPlan p = plan_split(m, n, k, A8_STEP_US, cus);
+  return mx_scale_planes(m, n, k) + (takes_skinny(m, n, k, false, nullptr, p) ? 0 : p.bytes);
 }
 
 extern "C" int kq_mx_linear_mx(int a_fmt, const void* a_q, const uint8_t* a_scale, int64_t lda, int w_fmt,
@@ -1210,15 +1225,15 @@ extern "C" int kq_mx_linear_mx(int a_fmt, const void* a_q, const uint8_t* a_scal
   hipStream_t st = (hipStream_t)stream;
   const uint8_t* ap = (const uint8_t*)a_q;
   const uint8_t* wp = (const uint8_t*)w_q;
-  if (takes_skinny(m, n, k, false, w_scale, true))
-    return kq_check_launch(mx_skinny_mx(out_dtype == KQ_DT_F32,
-                                        {a_q, a_scale, lda, wp, w_scale, c, ldc, (int)m, (int)n, (int)k}, st),
-                           fn);
   int cus = 0;
   hipError_t e = stream_cus(st, &cus);
   if (e != hipSuccess) return kq_check_launch(e, fn);
-  const SplitPlan p = plan_split(m, n, k, A8_STEP_US, cus);
-  if (p.slices > 1 && p.bytes <= workspace_bytes - need && one_range(lda, k, m, n)) {
+  const SplitPlan p = plan_within(plan_split(m, n, k, A8_STEP_US, cus), workspace_bytes - need, one_range(lda, k, m, n));
+  if (takes_skinny(m, n, k, false, w_scale, p))
+    return kq_check_launch(mx_skinny_mx(out_dtype == KQ_DT_F32,
+                                        {a_q, a_scale, lda, wp, w_scale, c, ldc, (int)m, (int)n, (int)k}, st),
+                           fn);
+  if (p.slices > 1) {
     void* planes = static_cast<char*>(workspace) + need;
     e = launch_linear_a8<2>(ap, a_scale, lda, wp, w_scale, planes, p.ldp, (int)m, (int)n, (int)k, workspace, cus, st,
                             p.slices, p.plane);

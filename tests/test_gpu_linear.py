@@ -314,3 +314,37 @@ def test_split_k(gpu, form, m, n, k):
         N.call("kq_mx_linear", N.FMT_MXFP8_E4M3 if fmt == "mxfp8" else N.FMT_MXFP4_E2M1, N.ptr(xg), k, N.ptr(qg),
                N.ptr(s), m, n, k, N.DT_F32, N.ptr(plain), n, N.stream(gpu))
         assert _max_rel(ref, plain.cpu().numpy()) <= 1e-5
+
+
+@pytest.mark.parametrize("m", [33, 48, 64])
+def test_workspace_too_small_for_the_planes(gpu, m):
+    """A workspace that does not hold the K slices' planes runs as none: the
+    same kernel, bit for bit (bf16 and fp32 rows; MXFP8 rows given the scale
+    planes alone against float64, at 5e-5 as everywhere for them)."""
+    from kquant_amd import _native as N
+
+    n, k = 2100, 2176
+    g = torch.Generator().manual_seed(m)
+    w = (torch.randn(n, k, generator=g) * 0.02).to(torch.bfloat16).to(gpu)
+    x = torch.randn(m, k, generator=g).to(gpu)
+    q, s, wd = _quantized("mxfp8", w)
+    qb, lib, st = q.view(torch.uint8), N.library(), N.stream(gpu)
+    xb = x.to(torch.bfloat16)
+    assert lib.kq_mx_linear_workspace_size(m, n, k) > 256
+    ws = torch.empty(4 * m * 3 * k * 2, dtype=torch.uint8, device=gpu)
+    out = [torch.empty(m, n, device=gpu) for _ in range(5)]
+    fmt = N.FMT_MXFP8_E4M3
+    N.call("kq_mx_linear", fmt, N.ptr(xb), k, N.ptr(qb), N.ptr(s), m, n, k, N.DT_F32, N.ptr(out[0]), n, st)
+    N.call("kq_mx_linear_ws", fmt, N.ptr(xb), k, N.ptr(qb), N.ptr(s), m, n, k, N.DT_F32, N.ptr(out[1]), n, N.ptr(ws),
+           256, st)
+    assert torch.equal(out[0], out[1])
+    need = lib.kq_mx_linear_f32_workspace_size(m, k)
+    for o, size in ((out[2], need), (out[3], (need + 255) // 256 * 256 + 256)):
+        N.call("kq_mx_linear_f32", fmt, N.ptr(x), k, N.ptr(qb), N.ptr(s), m, n, k, N.ptr(o), n, N.ptr(ws), size, st)
+    assert torch.equal(out[2], out[3])
+    xq, xs = mxfp8.mxfp8_quantize(xb)
+    planes = sum((r * (k // 32) + 255) // 256 * 256 for r in (m, n))
+    N.call("kq_mx_linear_mx", fmt, N.ptr(xq.view(torch.uint8)), N.ptr(xs), k, fmt, N.ptr(qb), N.ptr(s), m, n, k,
+           N.DT_F32, N.ptr(out[4]), n, N.ptr(ws), planes, st)
+    xv = oracle.mx_dequant("mxfp8", xq.view(torch.uint8).cpu().numpy(), xs.cpu().numpy()).astype(np.float64)
+    assert _max_rel(xv @ wd.astype(np.float64).T, out[4].cpu().numpy()) <= 5e-5
