@@ -30,7 +30,7 @@ using gemm::bf16x8_t;
 using gemm::u32x2_t;
 using gemm::u32x4_t;
 
-template <int FMT, int OUT>
+template <int FMT, int OUT, bool SPLIT>
 __global__ __launch_bounds__(512, 1) void mx_linear_kernel(
     const uint16_t* __restrict__ a, int64_t lda, const uint8_t* __restrict__ wq,
     const uint8_t* __restrict__ ws, void* __restrict__ c, int64_t ldc, int M, int N, int K, int KB, int64_t plane) {
@@ -112,9 +112,10 @@ __global__ __launch_bounds__(512, 1) void mx_linear_kernel(
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
   const int frow = lane & 31, fk = lane >> 5;  // fragment row, k half (8 elements)
-  // blockIdx.z: slice of the K steps, written to its own plane of c
-  const int steps = K / BK, slices = (int)gridDim.z, z = (int)blockIdx.z;
-  const int s_begin = (int)((int64_t)z * steps / slices), s_end = (int)((int64_t)(z + 1) * steps / slices);
+  // SPLIT: blockIdx.z is a slice of the K steps, written to its own plane of c
+  const int steps = K / BK, slices = SPLIT ? (int)gridDim.z : 1, z = SPLIT ? (int)blockIdx.z : 0;
+  const int s_begin = SPLIT ? (int)((int64_t)z * steps / slices) : 0;
+  const int s_end = SPLIT ? (int)((int64_t)(z + 1) * steps / slices) : steps;
   load(s_begin * BK);
   store(0);
   __syncthreads();
@@ -848,25 +849,29 @@ using namespace kq;
 // S slices, each writing its own fp32 plane in the workspace, and a second
 // launch adds the planes in slice order (deterministic).  S minimises the
 // rounds of (slice, tile) items times the steps of a slice, at the kernels'
-// measured time per 64-k step with one workgroup per CU, plus the sum's
-// launch and its plane traffic (written and read once, 5 TB/s).  M = 777,
-// N = 5000, K = 7168 (80 tiles, S = 3), MXFP8 x MXFP8:
-// 119 -> 66 us; M = 256, N = 2048, bf16 x E4M3: 140 -> 32 us; M = 512, N =
-// 12288 (96 tiles, S = 2): 145 -> 100 us.
+// measured time per 64-k step with one workgroup per CU, 4 us for each round of
+// slices after the first, plus the sum's launch and its plane traffic (written
+// and read once, 5 TB/s).  M = 777, N = 5000, K = 7168 (80 tiles, S = 3), MXFP8 x
+// MXFP8: 119 -> 66 us; M = 256, N = 2048, bf16 x E4M3: 140 -> 32 us; M = 512, N =
+// 12288 (96 tiles, S = 2): 145 -> 100 us.  Without the rounds' 4 us M = 1, N =
+// 49152, K = 2048 ran in four slices, 55 us against 49 in whole tiles.
 struct SplitPlan {
   int slices = 1;
   int64_t ldp = 0, plane = 0, bytes = 0;  // plane row stride and size (floats), all planes' bytes
+  int64_t tiles = 0, steps = 0;
 };
-constexpr double DMA_STEP_US = 1.25, STAGED_STEP_US = 1.6, A8_STEP_US = 0.98;
+constexpr double DMA_STEP_US = 1.25, STAGED_STEP_US = 1.6, A8_STEP_US = 0.98, ROUND_US = 4.0;
 
 static SplitPlan plan_split(int64_t m, int64_t n, int64_t k, double step_us, int cus) {
   SplitPlan p;
   p.ldp = (n + 3) / 4 * 4;
   p.plane = m * p.ldp;
-  const int64_t tiles = ((m + lin::BM - 1) / lin::BM) * ((n + lin::BN - 1) / lin::BN), steps = k / lin::BK;
-  double best = 0.97 * (double)((tiles + cus - 1) / cus) * (double)steps * step_us;
-  for (int64_t s = 2; s <= 16 && s * 4 <= steps; ++s) {
-    const double t = (double)((tiles * s + cus - 1) / cus) * (double)((steps + s - 1) / s) * step_us + 6.0 +
+  p.tiles = ((m + lin::BM - 1) / lin::BM) * ((n + lin::BN - 1) / lin::BN);
+  p.steps = k / lin::BK;
+  double best = 0.97 * (double)((p.tiles + cus - 1) / cus) * (double)p.steps * step_us;
+  for (int64_t s = 2; s <= 16 && s * 4 <= p.steps; ++s) {
+    const int64_t rounds = (p.tiles * s + cus - 1) / cus;
+    const double t = (double)rounds * (double)((p.steps + s - 1) / s) * step_us + (double)(rounds - 1) * ROUND_US + 6.0 +
                      (double)(s * p.plane * 8) / 5e6;
     if (t < best) {
       best = t;
@@ -994,7 +999,7 @@ static hipError_t launch_linear(const uint16_t* a, int64_t lda, const uint8_t* w
   if (takes_dma(FMT, lda, ws, KB))
     return launch_linear_dma<FMT, OUT>(a, lda, wq, ws, c, ldc, M, N, K, KB, st, slices, plane);
   const size_t lds = 2 * (size_t)lin::stage_bytes<FMT>();
-  auto kern = mx_linear_kernel<FMT, OUT>;
+  auto kern = OUT == 2 && slices > 1 ? mx_linear_kernel<FMT, 2, true> : mx_linear_kernel<FMT, OUT, false>;
   hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return e;
   dim3 grid((N + lin::BN - 1) / lin::BN, (M + lin::BM - 1) / lin::BM, slices);
@@ -1049,27 +1054,99 @@ hipError_t split3_rows(const float* a, int64_t lda, int64_t m, int64_t k, uint16
 
 }  // namespace kq
 
-// Which linears take the one-pass kernel of kq_skinny.hip.  Up to 32 rows
-// always: a 256 x 256 tile costs the same for 1 row as for 256 (N = 12288, K =
-// 7168 E4M3: 137 us, the one-pass kernel 24 us at 1 row, 43 at 32; split over
-// K with its second launch ~45).  At 33 .. 64 rows the split product passes it
-// where K is long (K = 7168, N = 5000, 48 rows: 33 against 57 us) but not
-// where its two launches dominate (K = 1024: 15 against 21 us; fp32 rows, a
-// third launch, also at N <= 2048: 37 against 46 us), nor unsplit (137 us).
+// Which linears of up to 64 rows take the one-pass kernel of kq_skinny.hip.
+//
+// Below 32 tiles (N < 8192): all of up to 32 rows (a 256 x 256 tile costs the
+// same for 1 row as for 256; N = 4096, K = 7168 E4M3: 134 us, split over K 27, the
+// one-pass kernel 13 us at 1 row and 21 at 32), and at 33 .. 64 rows those
+// where the split's two launches dominate (K = 1024: 15 against 21 us; fp32
+// rows, a third launch, also at N <= 2048: 37 against 46 us) or that have no
+// split.  Past that both kernels stream the weights at the chip's rate, the
+// one-pass kernel reading the rows once per 16 or 64 columns and the tiles
+// once per 256, so the shorter of two estimates is taken (with the tiles'
+// path, whose figures are the rougher ones, behind by 10 us up to N = 16384, else 3).
+// The constants are fits to times from N = 8192 to 129,280 and K = 320 to 7168, good
+// to about 15 %.  One-pass / tiles, us: MXFP8 rows, 64 x 12288 x 2048: 39 / 27,
+// 64 x 12288 x 7168: 82 / 40, 16 x 65536 x 7168: 169 / 121; bf16 rows x E4M3, 16 x 65536 x 2048: 79 / 52,
+// 16 x 32768 x 7168: 97 / 90, 1 x 65536 x 7168: 120 / 166, 64 x 65536 x 2112 (half
+// windows, no wide form): 276 / 68; fp32 rows, 32 x 65536 x 7168: 248 / 490, 64: 466 / 509.
+enum SkinnyForm { FORM_BF16_E4M3, FORM_BF16_E2M1, FORM_F32_E4M3, FORM_F32_E2M1, FORM_MX };
+static SkinnyForm skinny_form(int w_fmt, bool f32_rows) {
+  const bool e4m3 = w_fmt == KQ_FMT_MXFP8_E4M3;
+  return f32_rows ? (e4m3 ? FORM_F32_E4M3 : FORM_F32_E2M1) : e4m3 ? FORM_BF16_E4M3 : FORM_BF16_E2M1;
+}
+static bool is_f32(SkinnyForm f) { return f == FORM_F32_E4M3 || f == FORM_F32_E2M1; }
+static bool is_e2m1(SkinnyForm f) { return f == FORM_BF16_E2M1 || f == FORM_F32_E2M1; }
+
+// us of the one-pass kernel for row blocks as launch_rows (kq_skinny.hip) cuts
+// them: ns per column and 1000 k, and per column, both linear in the rows.
+static double skinny_us(SkinnyForm f, int64_t m, int64_t n, int64_t k) {
+  struct Rate { double one[2], wide[2], narrow[2]; };  // R = 1 to 16 rows, R = 4, R = 1 past 16 rows
+  static constexpr Rate rates[] = {{{0.21, 0.0077}, {0.225, 0.0023}, {0.20, 0.0088}},
+                                   {{0.13, 0.0117}, {0.155, 0.0037}, {0.20, 0.0077}},
+                                   {{0.24, 0.0225}, {0.30, 0.0045}, {0.37, 0.0166}},
+                                   {{0.215, 0.029}, {0.19, 0.0075}, {0.48, 0.0115}},
+                                   {{0.192, 0.0066}, {0.265, 0.001}, {0.23, 0.007}}};
+  const bool half = k % 128 != 0;
+  const int64_t block = m <= 16 ? 16 : m <= 32 || is_f32(f) ? 32 : 64, blocks = (m + block - 1) / block;
+  const double rows = (double)(blocks == 1 ? m : block);
+  const bool wide = n >= 8192 && !half && m > 16 && !(f == FORM_MX && m > 32);
+  const double* rate = m <= 16 ? rates[f].one : wide ? rates[f].wide : rates[f].narrow;
+  double a = rate[0] + rate[1] * rows, b;
+  if (m <= 16) b = is_f32(f) ? 0.34 + 0.0235 * rows : 0.25 + 0.0172 * rows;
+  else if (wide) b = 0.32 + 0.0072 * rows;
+  else b = is_f32(f) ? 0.75 + 0.02 * rows : 0.15 + 0.026 * rows;
+  if (f == FORM_BF16_E2M1) b *= 0.87;
+  if (half) {
+    a *= is_e2m1(f) ? 1.45 : 1.25;
+    if (is_f32(f)) b *= 1.6;
+  }
+  const double windows = (double)((k + 127) / 128);
+  const double run = (windows - 3.0) / 13.0;  // a column's own cost shows once its waves have several windows
+  const double cols = (double)(n * blocks), fill = 256.0 * (wide ? 64 : 16);
+  return 4.0 + (cols > fill ? cols : fill) / 1e3 * (a * (double)k / 1e3 + b * (run < 0.2 ? 0.2 : run > 1.0 ? 1.0 : run));
+}
+
+// us of the tiles as planned, for few rows: a step slows down as the weights
+// of more workgroups come from memory at once.
+static double tiles_us(SkinnyForm f, const SplitPlan& p, double step_us, int cus) {
+  const double lone = is_e2m1(f) ? 0.87 : 0.90, more = f == FORM_MX ? 0.07 : is_e2m1(f) ? 0.08 : is_f32(f) ? 0.27 : 0.22;
+  const int64_t items = p.tiles * p.slices, full = items / cus, rest = items % cus;
+  const double share = (double)rest / cus;
+  const double rounds = (double)full * (lone + more) + (rest ? lone + more * share * sqrt(share) : 0.0);
+  double us = 10.0 + (double)((p.steps + p.slices - 1) / p.slices) * step_us * rounds;
+  if (p.slices > 1) us += 2.0 + ROUND_US * (double)(full + (rest ? 1 : 0) - 1);
+  return us + (is_f32(f) ? 4.0 : f == FORM_MX ? 3.0 : 0.0);
+}
+
+// Calls that need no plan to tell (and no query of the device, 1 us of a small
+// call's 14): narrow ones of up to 32 rows, and wide ones of an estimate that
+// no plan of the tiles (10 us and more) comes under by that margin.
+static bool surely_skinny(SkinnyForm f, int64_t m, int64_t n, int64_t k, const uint8_t* w_scale) {
+  if (m > 64 || (k % 128 == 0 && kq_misaligned(w_scale, 4)) || (m > 32 && k > 2048)) return false;
+  return n < 8192 || skinny_us(f, m, n, k) <= (n <= 16384 ? 20.0 : 13.0);
+}
+
 // p: the tiles' plan as it can run with the caller's workspace.
-static bool takes_skinny(int64_t m, int64_t n, int64_t k, bool f32_rows, const uint8_t* w_scale, const SplitPlan& p) {
-  if (k % 128 == 0 && kq_misaligned(w_scale, 4)) return false;
-  return m <= 32 || (m <= 64 && (k <= 2048 || (f32_rows && n <= 2048) || p.slices <= 1));
+static bool takes_skinny(SkinnyForm f, int64_t m, int64_t n, int64_t k, const uint8_t* w_scale, const SplitPlan& p,
+                         double step_us, int cus) {
+  if (m > 64 || (k % 128 == 0 && kq_misaligned(w_scale, 4))) return false;
+  if (m > 32 && k > 2048 && !(is_f32(f) && n <= 2048) && p.slices > 1) return false;
+  return n < 8192 || skinny_us(f, m, n, k) <= tiles_us(f, p, step_us, cus) + (n <= 16384 ? 10.0 : 3.0);
 }
 
 static double step_us(bool dma) { return dma ? DMA_STEP_US : STAGED_STEP_US; }
 
 extern "C" int64_t kq_mx_linear_workspace_size(int64_t m, int64_t n, int64_t k) {
   if (m < 0 || n < 0 || k <= 0) return -1;
+  if (surely_skinny(FORM_BF16_E4M3, m, n, k, nullptr) && surely_skinny(FORM_BF16_E2M1, m, n, k, nullptr)) return 0;
   const int cus = current_cus();
   if (cus <= 0) return 0;
-  const SplitPlan p = plan_split(m, n, k, step_us(k % 128 == 0), cus);
-  return takes_skinny(m, n, k, false, nullptr, p) ? 0 : p.bytes;
+  const double step = step_us(k % 128 == 0);
+  const SplitPlan p = plan_split(m, n, k, step, cus);
+  return takes_skinny(FORM_BF16_E4M3, m, n, k, nullptr, p, step, cus) &&
+                 takes_skinny(FORM_BF16_E2M1, m, n, k, nullptr, p, step, cus)
+             ? 0 : p.bytes;
 }
 
 extern "C" int kq_mx_linear(int w_fmt, const void* a, int64_t lda, const void* w_q,
@@ -1101,13 +1178,19 @@ extern "C" int kq_mx_linear_ws(int w_fmt, const void* a, int64_t lda, const void
   hipStream_t st = (hipStream_t)stream;
   const uint16_t* ap = (const uint16_t*)a;
   const uint8_t* wp = (const uint8_t*)w_q;
-  int cus = 0;
-  hipError_t e = stream_cus(st, &cus);
-  if (e != hipSuccess) return kq_check_launch(e, "kq_mx_linear");
-  const double step = step_us(takes_dma(w_fmt == KQ_FMT_MXFP8_E4M3 ? 0 : 1, lda, w_scale, k));
-  const SplitPlan p = plan_within(plan_split(m, n, k, step, cus), workspace_bytes,
-                                  one_range(2 * lda, w_fmt == KQ_FMT_MXFP8_E4M3 ? k : k / 2, m, n));
-  if (takes_skinny(m, n, k, false, w_scale, p))
+  const SkinnyForm form = skinny_form(w_fmt, false);
+  bool skinny = surely_skinny(form, m, n, k, w_scale);
+  hipError_t e;
+  SplitPlan p;
+  if (!skinny) {
+    int cus = 0;
+    if ((e = stream_cus(st, &cus)) != hipSuccess) return kq_check_launch(e, "kq_mx_linear");
+    const double step = step_us(takes_dma(w_fmt == KQ_FMT_MXFP8_E4M3 ? 0 : 1, lda, w_scale, k));
+    p = plan_within(plan_split(m, n, k, step, cus), workspace_bytes,
+                    one_range(2 * lda, w_fmt == KQ_FMT_MXFP8_E4M3 ? k : k / 2, m, n));
+    skinny = takes_skinny(form, m, n, k, w_scale, p, step, cus);
+  }
+  if (skinny)
     return kq_check_launch(mx_skinny_bf16(w_fmt, out_dtype == KQ_DT_F32,
                                           {a, nullptr, lda, wp, w_scale, c, ldc, (int)m, (int)n, (int)k}, st),
                            "kq_mx_linear");
@@ -1131,10 +1214,14 @@ static int64_t f32_planes_offset(int64_t m, int64_t k) { return (m * 3 * k * 2 +
 
 extern "C" int64_t kq_mx_linear_f32_split_workspace_size(int64_t m, int64_t n, int64_t k) {
   if (m < 0 || n < 0 || k <= 0) return -1;
+  if (surely_skinny(FORM_F32_E4M3, m, n, k, nullptr) && surely_skinny(FORM_F32_E2M1, m, n, k, nullptr)) return m * 3 * k * 2;
   const int cus = current_cus();
   if (cus <= 0) return m * 3 * k * 2;
-  const SplitPlan p = plan_split(m, n, 3 * k, step_us(k % 128 == 0), cus);
-  return p.bytes == 0 || takes_skinny(m, n, k, true, nullptr, p) ? m * 3 * k * 2 : f32_planes_offset(m, k) + p.bytes;
+  const double step = step_us(k % 128 == 0);
+  const SplitPlan p = plan_split(m, n, 3 * k, step, cus);
+  return p.bytes == 0 || (takes_skinny(FORM_F32_E4M3, m, n, k, nullptr, p, step, cus) &&
+                          takes_skinny(FORM_F32_E2M1, m, n, k, nullptr, p, step, cus))
+             ? m * 3 * k * 2 : f32_planes_offset(m, k) + p.bytes;
 }
 
 extern "C" int kq_mx_linear_f32(int w_fmt, const float* a, int64_t lda, const void* w_q,
@@ -1158,12 +1245,18 @@ extern "C" int kq_mx_linear_f32(int w_fmt, const float* a, int64_t lda, const vo
     return kq_fail(KQ_ERR_INVALID, "kq_mx_linear_f32: a, w_q and workspace must be 16-byte aligned");
   if (m == 0 || n == 0) return KQ_OK;
   hipStream_t st = (hipStream_t)stream;
-  int cus = 0;
-  if (int rc = kq_check_launch(stream_cus(st, &cus), "kq_mx_linear_f32")) return rc;
   const int64_t off = f32_planes_offset(m, k), w_row = w_fmt == KQ_FMT_MXFP8_E4M3 ? k : k / 2;
-  const double step = step_us(takes_dma(w_fmt == KQ_FMT_MXFP8_E4M3 ? 0 : 1, 3 * k, w_scale, k));
-  const SplitPlan p = plan_within(plan_split(m, n, 3 * k, step, cus), workspace_bytes - off, one_range(6 * k, w_row, m, n));
-  if (takes_skinny(m, n, k, true, w_scale, p))
+  const SkinnyForm form = skinny_form(w_fmt, true);
+  bool skinny = surely_skinny(form, m, n, k, w_scale);
+  SplitPlan p;
+  if (!skinny) {
+    int cus = 0;
+    if (int rc = kq_check_launch(stream_cus(st, &cus), "kq_mx_linear_f32")) return rc;
+    const double step = step_us(takes_dma(w_fmt == KQ_FMT_MXFP8_E4M3 ? 0 : 1, 3 * k, w_scale, k));
+    p = plan_within(plan_split(m, n, 3 * k, step, cus), workspace_bytes - off, one_range(6 * k, w_row, m, n));
+    skinny = takes_skinny(form, m, n, k, w_scale, p, step, cus);
+  }
+  if (skinny)
     return kq_check_launch(mx_skinny_f32(w_fmt, {a, nullptr, lda, (const uint8_t*)w_q, w_scale, c, ldc, (int)m, (int)n,
                                                  (int)k}, st),
                            "kq_mx_linear_f32");
@@ -1202,10 +1295,11 @@ static int64_t mx_scale_planes(int64_t m, int64_t n, int64_t k) {
 
 extern "C" int64_t kq_mx_linear_mx_workspace_size(int64_t m, int64_t n, int64_t k) {
   if (m < 0 || n < 0 || k <= 0) return -1;
+  if (surely_skinny(FORM_MX, m, n, k, nullptr)) return mx_scale_planes(m, n, k);
   const int cus = current_cus();
   if (cus <= 0) return mx_scale_planes(m, n, k);
   const SplitPlan p = plan_split(m, n, k, A8_STEP_US, cus);
-  return mx_scale_planes(m, n, k) + (takes_skinny(m, n, k, false, nullptr, p) ? 0 : p.bytes);
+  return mx_scale_planes(m, n, k) + (takes_skinny(FORM_MX, m, n, k, nullptr, p, A8_STEP_US, cus) ? 0 : p.bytes);
 }
 
 extern "C" int kq_mx_linear_mx(int a_fmt, const void* a_q, const uint8_t* a_scale, int64_t lda, int w_fmt,
@@ -1226,10 +1320,15 @@ extern "C" int kq_mx_linear_mx(int a_fmt, const void* a_q, const uint8_t* a_scal
   const uint8_t* ap = (const uint8_t*)a_q;
   const uint8_t* wp = (const uint8_t*)w_q;
   int cus = 0;
-  hipError_t e = stream_cus(st, &cus);
-  if (e != hipSuccess) return kq_check_launch(e, fn);
-  const SplitPlan p = plan_within(plan_split(m, n, k, A8_STEP_US, cus), workspace_bytes - need, one_range(lda, k, m, n));
-  if (takes_skinny(m, n, k, false, w_scale, p))
+  hipError_t e;
+  bool skinny = surely_skinny(FORM_MX, m, n, k, w_scale);
+  SplitPlan p;
+  if (!skinny) {
+    if ((e = stream_cus(st, &cus)) != hipSuccess) return kq_check_launch(e, fn);
+    p = plan_within(plan_split(m, n, k, A8_STEP_US, cus), workspace_bytes - need, one_range(lda, k, m, n));
+    skinny = takes_skinny(FORM_MX, m, n, k, w_scale, p, A8_STEP_US, cus);
+  }
+  if (skinny)
     return kq_check_launch(mx_skinny_mx(out_dtype == KQ_DT_F32,
                                         {a_q, a_scale, lda, wp, w_scale, c, ldc, (int)m, (int)n, (int)k}, st),
                            fn);

@@ -22,6 +22,7 @@ import oracle
 from kquant_amd import linear, workloads
 from kquant_amd import mxfp4 as kq_mxfp4
 from kquant_amd import mxfp8
+from kquant_amd.io import mxfp4 as io_mxfp4
 
 pytestmark = pytest.mark.gpu
 
@@ -348,3 +349,33 @@ def test_workspace_too_small_for_the_planes(gpu, m):
            N.DT_F32, N.ptr(out[4]), n, N.ptr(ws), planes, st)
     xv = oracle.mx_dequant("mxfp8", xq.view(torch.uint8).cpu().numpy(), xs.cpu().numpy()).astype(np.float64)
     assert _max_rel(xv @ wd.astype(np.float64).T, out[4].cpu().numpy()) <= 5e-5
+
+
+@pytest.mark.parametrize("form,m,n,k", [("bf16-mxfp8", 16, 65600, 576), ("bf16-mxfp4", 33, 65537, 320),
+                                        ("bf16-mxfp8", 64, 49153, 512), ("f32-mxfp8", 33, 65540, 320),
+                                        ("mx-mxfp8", 64, 12288, 2048), ("mx-mxfp8", 32, 40001, 1024)])
+def test_few_rows_of_wide_weights(gpu, form, m, n, k):
+    """Few rows of weights wide enough for the 256 x 256 tiles to win: fp32
+    output within 1e-5 of float64 (MXFP8 rows on the matrix cores 5e-5), and
+    the MXFP8 rows' workspace has the split's planes."""
+    from kquant_amd import _native as N
+
+    dtype, fmt = form.split("-")
+    print(f"case wide {form} {m} {n} {k}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    w = (torch.randn(n, k, generator=g, device=gpu) * 0.02).to(torch.bfloat16)
+    x = torch.randn(m, k, generator=g, device=gpu).to(torch.float32 if dtype == "f32" else torch.bfloat16)
+    quantize = mxfp8.mxfp8_quantize if fmt == "mxfp8" else kq_mxfp4.mxfp4_quantize
+    q, s = quantize(w)
+    dequant = mxfp8.mxfp8_dequantize if fmt == "mxfp8" else io_mxfp4.dequant
+    if dtype == "mx":
+        xq, xs = mxfp8.mxfp8_quantize(x)
+        c = linear.mxfp8_linear_mx(xq, xs, q, s, out_dtype=torch.float32)
+        x = mxfp8.mxfp8_dequantize(xq, xs, dtype=torch.float32)
+        planes = sum((r * (k // 32) + 255) // 256 * 256 for r in (m, n))
+        if n == 12288:
+            assert N.library().kq_mx_linear_mx_workspace_size(m, n, k) > planes
+    else:
+        c = (linear.mxfp8_linear if fmt == "mxfp8" else linear.mxfp4_linear)(x, q, s, out_dtype=torch.float32)
+    ref = x.double() @ dequant(q, s, dtype=torch.float32).double().T
+    assert float((c.double() - ref).abs().max() / ref.abs().max()) <= (5e-5 if dtype == "mx" else 1e-5)
