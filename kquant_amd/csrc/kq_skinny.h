@@ -130,7 +130,7 @@ __global__ __launch_bounds__(512) void mx_skinny_kernel(
         for (int t = 0; t < 4; ++t) {
           const int koff = FMT == 0 ? 64 * (t >> 1) + 8 * (t & 1) : 8 * t;
           const bool gone = cut && (FMT == 1 || t >= 2);
-          const uint8_t* p = arow[i] + (k0 + (gone ? (FMT == 0 ? koff - 64 : koff - 64) : koff)) * ES;
+          const uint8_t* p = arow[i] + (k0 + (gone ? koff - 64 : koff)) * ES;
 #pragma unroll
           for (int e = 0; e < PER; ++e) {
             v.a[i][PER * t + e] = load16(p + 16 * e);
@@ -147,37 +147,22 @@ __global__ __launch_bounds__(512) void mx_skinny_kernel(
 #pragma unroll
     for (int j = 0; j < R; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
+  // MXFP8 rows: E4M3 x 2^(s - 127) is a normal bf16 for 10 <= s <= 246; a
+  // window with another scale byte (any lane's) is left for after the loop
+  auto odd_scales = [&](const Win& v) -> bool {
+    bool odd = false;
+#pragma unroll
+    for (int j = 0; j < R; ++j) odd |= (v.s[j] >> (8 * g) & 0xffu) - 10u > 236u;
+#pragma unroll
+    for (int i = 0; i < MB; ++i) odd |= (v.as[i] >> (8 * g) & 0xffu) - 10u > 236u;
+    return __any(odd);
+  };
+  bool left = false;
+
   auto compute = [&](const Win& v) {
     if constexpr (AT == A_MXFP8) {
-      // E4M3 x 2^(s - 127) is a normal bf16 for 10 <= s <= 246; a window with
-      // another scale byte multiplies in fp32 (element e of every lane is one
-      // k of a 16x16x4 MFMA)
-      bool odd = false;
-#pragma unroll
-      for (int j = 0; j < R; ++j) odd |= (v.s[j] >> (8 * g) & 0xffu) - 10u > 236u;
-#pragma unroll
-      for (int i = 0; i < MB; ++i) odd |= (v.as[i] >> (8 * g) & 0xffu) - 10u > 236u;
-      if (__any(odd)) {
-#pragma unroll
-        for (int e = 0; e < 32; e += 2) {
-          const int h = e >> 4, d = (e >> 2) & 3, sh = 16 * h + 8 * (g >> 1);
-          const bool hi = e & 2;
-          auto expand = [&](uint32_t word, uint32_t scales) -> float2_t {
-            const float sc = __uint_as_float((scales >> sh & 0xffu) << 23);
-            return hi ? __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(word, sc, true)
-                      : __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(word, sc, false);
-          };
-#pragma unroll
-          for (int j = 0; j < R; ++j) {
-            const float2_t b = expand(v.w[j][h][d], v.s[j]);
-#pragma unroll
-            for (int i = 0; i < MB; ++i) {
-              const float2_t x = expand(v.a[i][h][d], v.as[i]);
-              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[0], b[0], acc[i][j], 0, 0, 0);
-              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[1], b[1], acc[i][j], 0, 0, 0);
-            }
-          }
-        }
+      if (odd_scales(v)) {
+        left = true;
         return;
       }
     }
@@ -241,6 +226,47 @@ __global__ __launch_bounds__(512) void mx_skinny_kernel(
 #pragma unroll
     for (int p = 0; p < P - 1; ++p)
       if (w + p < w_end) compute(v[p]);
+  }
+
+  if constexpr (AT == A_MXFP8) {
+    // The windows left: the codes themselves multiply in fp32, each 32-k block
+    // on its own (lane groups 2 blk and 2 blk + 1 of its chunk; element e of
+    // every lane is one k of a 16x16x4 MFMA), and both scales apply to the
+    // block's sum as one exponent, so an operand may leave fp32's range where
+    // the product does not.  Scale byte 255 is NaN.
+    for (int w = w_begin; left && w < w_end; ++w) {
+      Win v;
+      load(w, v);
+      if (!odd_scales(v)) continue;
+#pragma nounroll
+      for (int blk = 0; blk < 4; ++blk) {
+        const bool mine = (g >> 1) == (blk & 1);
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+          for (int j = 0; j < R; ++j) {
+            f32x4_t dot = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int e = 0; e < 16; e += 2) {
+              const uint32_t aw = blk & 2 ? v.a[i][1][e >> 2] : v.a[i][0][e >> 2];
+              const uint32_t ww = !mine ? 0u : blk & 2 ? v.w[j][1][e >> 2] : v.w[j][0][e >> 2];
+              const float2_t x = e & 2 ? __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(aw, 1.0f, true)
+                                       : __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(aw, 1.0f, false);
+              const float2_t b = e & 2 ? __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(ww, 1.0f, true)
+                                       : __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(ww, 1.0f, false);
+              dot = __builtin_amdgcn_mfma_f32_16x16x4f32(x[0], b[0], dot, 0, 0, 0);
+              dot = __builtin_amdgcn_mfma_f32_16x16x4f32(x[1], b[1], dot, 0, 0, 0);
+            }
+            const int sw = (int)(v.s[j] >> (8 * blk) & 0xffu);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {  // row 4 g + q: lane 4 g + q has its scales
+              const int sa = (int)((uint32_t)__shfl((int)v.as[i], 4 * g + q) >> (8 * blk) & 0xffu);
+              const float term = __builtin_amdgcn_ldexpf(dot[q], sa + sw - 254);
+              acc[i][j][q] += sa == 255 || sw == 255 ? __builtin_nanf("") : term;
+            }
+          }
+      }
+    }
   }
 
   // D (16x16): lane holds column lane % 16, rows 4 (lane / 16) + j

@@ -379,3 +379,47 @@ def test_few_rows_of_wide_weights(gpu, form, m, n, k):
         c = (linear.mxfp8_linear if fmt == "mxfp8" else linear.mxfp4_linear)(x, q, s, out_dtype=torch.float32)
     ref = x.double() @ dequant(q, s, dtype=torch.float32).double().T
     assert float((c.double() - ref).abs().max() / ref.abs().max()) <= (5e-5 if dtype == "mx" else 1e-5)
+
+
+def _mx_values(q, s):
+    v = q.view(torch.float8_e4m3fn).double().reshape(q.shape[0], -1, 32)
+    return (v * torch.exp2(s.double() - 127)[..., None]).reshape(q.shape)
+
+
+@pytest.mark.parametrize("m,n,k", [(3, 40, 512), (16, 16, 128), (31, 8200, 256), (64, 70, 384)])
+@pytest.mark.parametrize("a_byte", [247, 254, 0, 120, -1])
+def test_few_rows_scales_past_fp32(gpu, m, n, k, a_byte):
+    """Operands that leave fp32's range by their own scale while the product
+    does not (448 x 2^127 against 2^-127; -1: another scale for every block,
+    its counterpart on the other side), in every row-block form.  Codes of one
+    sign, products and the 32-k sums in fp32: k 2^-24 <= 3e-5 of float64."""
+    g = torch.Generator().manual_seed(m + a_byte)
+    aq = torch.randint(1, 127, (m, k), generator=g, dtype=torch.uint8)
+    wq = torch.randint(1, 127, (n, k), generator=g, dtype=torch.uint8)
+    base = torch.randint(0, 255, (k // 32,), generator=g) if a_byte < 0 else torch.full((k // 32,), a_byte)
+    a_s = (base + torch.randint(-3, 4, (m, k // 32), generator=g)).clamp(0, 254).to(torch.uint8)
+    w_s = (254 - base + torch.randint(-3, 4, (n, k // 32), generator=g)).clamp(0, 254).to(torch.uint8)
+    c = linear.mxfp8_linear_mx(aq.to(gpu).view(torch.float8_e4m3fn), a_s.to(gpu), wq.to(gpu), w_s.to(gpu),
+                               out_dtype=torch.float32)
+    assert _max_rel((_mx_values(aq, a_s) @ _mx_values(wq, w_s).T).numpy(), c.cpu().numpy()) <= 3e-5
+
+
+def test_few_rows_scale_and_code_nans(gpu):
+    """A NaN code or scale byte 255 makes its own row (column) NaN and no
+    other, beside a block whose scales need the fp32 products."""
+    g = torch.Generator().manual_seed(9)
+    m, n, k = 20, 50, 256
+    aq = torch.randint(1, 127, (m, k), generator=g, dtype=torch.uint8)
+    wq = torch.randint(1, 127, (n, k), generator=g, dtype=torch.uint8)
+    a_s = torch.full((m, k // 32), 127, dtype=torch.uint8)
+    w_s = torch.full((n, k // 32), 127, dtype=torch.uint8)
+    a_s[:, 1], w_s[:, 1] = 250, 4
+    aq[3, 70], aq[5, 200], w_s[7, 1], a_s[11, 6], wq[13, 33] = 127, 255, 255, 255, 127
+    nan = torch.zeros(m, n, dtype=torch.bool)
+    nan[[3, 5, 11]] = True
+    nan[:, [7, 13]] = True
+    c = linear.mxfp8_linear_mx(aq.to(gpu).view(torch.float8_e4m3fn), a_s.to(gpu), wq.to(gpu), w_s.to(gpu),
+                               out_dtype=torch.float32).cpu()
+    assert torch.equal(torch.isnan(c), nan)
+    ref = (_mx_values(aq, a_s) @ _mx_values(wq, w_s).T)
+    assert float(((c.double() - ref)[~nan] / ref[~nan]).abs().max()) <= 3e-5
