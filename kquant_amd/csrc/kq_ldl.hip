@@ -203,6 +203,12 @@ __device__ __forceinline__ int factor64_wg(float (*a)[LD], float (*xi)[LD]) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(m[e], v[e], acc, 0, 0, 0);
   };
+  // between LDS stores of a wave's lanes and its other lanes' loads (the
+  // hardware completes one wave's accesses in order; this orders the compiler's)
+  auto lanes_exchange = [&]() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
   // tb[j] = sum over k = j .. i - 1 of L[i][k] X[k][j] (X = inv(L), 16 x 16 blocks)
   auto inv_sum = [&](int i, int j) {
     f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
@@ -210,13 +216,15 @@ __device__ __forceinline__ int factor64_wg(float (*a)[LD], float (*xi)[LD]) {
       mul(acc, a, PB * i, PB * k, [&](int kk) { return xi[PB * k + kk][PB * j + li]; });
 #pragma unroll
     for (int q = 0; q < 4; ++q) tb[j][4 * lk + q][li] = acc[q];
+    lanes_exchange();
   };
-  // X[i][j] = -X[i][i] tb[j] (one wave's LDS accesses complete in order)
+  // X[i][j] = -X[i][i] tb[j]
   auto inv_block = [&](int i, int j) {
     f32x4_t x = {0.f, 0.f, 0.f, 0.f};
     mul(x, xi, PB * i, PB * i, [&](int kk) { return tb[j][kk][li]; });
 #pragma unroll
     for (int q = 0; q < 4; ++q) xi[PB * i + 4 * lk + q][PB * j + li] = -x[q];
+    lanes_exchange();
   };
   if (tid == 0) s_bad = 0;
   // the diagonal blocks symmetric, zeros in the blocks above them (and of inv(L))
@@ -285,6 +293,7 @@ __device__ __forceinline__ int factor64_wg(float (*a)[LD], float (*xi)[LD]) {
       const int r0 = c0 + PB * (1 + wave);
       f32x4_t l21 = {0.f, 0.f, 0.f, 0.f};
       mul(l21, a, r0, c0, [&](int kk) { return xi[c0 + li][c0 + kk]; });
+      lanes_exchange();  // every lane has read the rows
 #pragma unroll
       for (int j = 0; j < 4; ++j) a[r0 + 4 * lk + j][c0 + li] = l21[j];
     }

@@ -259,11 +259,12 @@ def test_hadamard_ragged_rows_and_row_strides(gpu, ld):
     assert np.array_equal(got[:, cols:], buf[:, cols:])
 
 
-@pytest.mark.parametrize("batch,n,b", [(2, 1024, 16), (11, 1216, 4), (9, 1296, 16), (36, 1376, 32), (1, 4160, 64)])
+@pytest.mark.parametrize("batch,n,b", [(2, 1024, 16), (5, 720, 16), (11, 1216, 4), (9, 1296, 16), (36, 1280, 16),
+                                       (36, 1376, 32), (1, 4160, 64)])
 def test_super_panel_widths_and_ldl_tiles(gpu, batch, n, b):
-    """Super-panels of two, four and eight panels, whole and ragged 64-column
-    tiles (direct loads or not) and every block size class of the LDL tiles,
-    from a separate source: the factor of the first and last matrix against
+    """Super-panels of two, four and eight panels, each with whole and ragged
+    64-column tiles (direct loads or not), and every block size class of the
+    LDL tiles, from a separate source: the factor of the first and last matrix against
     numpy's float64 one.  Bound as test_cholesky_*: 2e-5 (fp32 rounding
     through well-conditioned blocks); the source is left as it was."""
     base = [_spd(n, 70 + e) for e in range(2)]
@@ -273,6 +274,8 @@ def test_super_panel_widths_and_ldl_tiles(gpu, batch, n, b):
     assert torch.equal(a, keep) and not info.any()
     for e, ref in ((0, base[0]), (batch - 1, base[min(1, batch - 1)])):
         want = ldl.block_ldl(ref, b)
-        assert _rel(want, lower[e].cpu().numpy()) <= 1e-4
+        rel = _rel(want, lower[e].cpu().numpy())
+        print(f"block ldl {batch} x {n} b={b}: {rel:.2e}", flush=True)
+        assert rel <= 2e-5
     if batch > 2:
         assert torch.equal(lower[1], lower[batch - 1])
