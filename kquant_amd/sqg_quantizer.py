@@ -30,8 +30,6 @@ import torch
 from . import _native as N
 from .sqg_e4m3 import sqg_e4m3_bytes
 
-_WORKSPACES: dict[tuple[torch.device, int, int], torch.Tensor] = {}
-
 
 def _workgroups(device: torch.device) -> int:
     return 2 * torch.cuda.get_device_properties(device).multi_processor_count  # two tiles per CU
@@ -58,21 +56,19 @@ def quantize_tiles_sqg(tiles: torch.Tensor, lut: torch.Tensor, bits: int,
     table = N.aligned(lut.to(device=device).contiguous(), 16)
     out = torch.empty_like(x)
     states = torch.empty(x.shape, dtype=torch.int16, device=device)
-    ws = _workspace(device, bits)
+    workgroups, ws = _workspace(device, bits, x.shape[0])
     N.call("kq_sqg_quantize_tiles", N.ptr(x), x.shape[0], N.ptr(table), bits, int(tailbite_context), N.ptr(out),
-           N.ptr(states), N.ptr(ws), ws.numel(), _workgroups(device), N.stream(device))
+           N.ptr(states), N.ptr(ws), ws.numel(), workgroups, N.stream(device))
     return out, states
 
 
-def _workspace(device: torch.device, bits: int) -> torch.Tensor:
-    """Decision workspace, one per (device, stream, rate)."""
-    need = int(N.library().kq_sqg_quantize_workspace_size(bits, _workgroups(device)))
-    key = (device, N.stream_handle(device), bits)
-    ws = _WORKSPACES.get(key)
-    if ws is None or ws.numel() < need:
-        ws = torch.empty(need, dtype=torch.uint8, device=device)
-        _WORKSPACES[key] = ws
-    return ws
+def _workspace(device: torch.device, bits: int, tiles: int) -> tuple[int, torch.Tensor]:
+    """Workgroups of a call and their decisions (1 MiB each at K2 and K3, half
+    at K4), the call's own: none holds more than its tiles need, and nothing is
+    shared between streams or captured graphs."""
+    workgroups = max(1, min(tiles, _workgroups(device)))
+    need = int(N.library().kq_sqg_quantize_workspace_size(bits, workgroups))
+    return workgroups, torch.empty(need, dtype=torch.uint8, device=device)
 
 
 def quantize_tiles_procedural(tiles: torch.Tensor, bits: int, codebook: int,
@@ -96,9 +92,9 @@ def quantize_tiles_procedural(tiles: torch.Tensor, bits: int, codebook: int,
     x = N.aligned(tiles.contiguous(), 4)
     out = torch.empty_like(x)
     states = torch.empty(x.shape, dtype=torch.int16, device=device)
-    ws = _workspace(device, bits)
+    workgroups, ws = _workspace(device, bits, x.shape[0])
     N.call("kq_sqg_quantize_tiles_procedural", N.ptr(x), x.shape[0], bits, codebook, int(tailbite_context),
-           N.ptr(out), N.ptr(states), N.ptr(ws), ws.numel(), _workgroups(device), N.stream(device))
+           N.ptr(out), N.ptr(states), N.ptr(ws), ws.numel(), workgroups, N.stream(device))
     return out, states
 
 

@@ -121,3 +121,15 @@ def test_two_tiles_per_cu(gpu, bits, ctx):
         vals, states = sqg_quantizer.quantize_tiles_sqg(torch.from_numpy(x).to(gpu).repeat(copies, 1), lut, bits, ctx)
         assert np.array_equal(states.cpu().numpy(), np.tile(want_states, (copies, 1)))
         assert np.array_equal(vals.cpu().numpy(), np.tile(want_vals, (copies, 1)))
+
+
+def test_workspace_is_the_calls_own(gpu):
+    """A call of few tiles holds the decisions of its own workgroups only (six
+    of 1 MiB at K2) and none of them after it."""
+    x = torch.from_numpy(_tiles(2, 3)).to(gpu)
+    lut = sqg_xor_cheb_t12_bytes(2, device=gpu)
+    before = torch.cuda.memory_allocated(gpu)
+    torch.cuda.reset_peak_memory_stats(gpu)
+    out = sqg_quantizer.quantize_tiles_sqg(x, lut, 2, 16)
+    assert torch.cuda.max_memory_allocated(gpu) - before <= 8 << 20
+    assert torch.cuda.memory_allocated(gpu) - before <= 4096 + sum(o.numel() * o.element_size() for o in out)
