@@ -66,6 +66,19 @@ template <int K> constexpr int edges() { return 65536 >> K; }
 // decision bytes per step: K bits a node (3 take the room of 4)
 template <int K> constexpr int row_bytes() { return K == 2 ? edges<K>() / 4 : edges<K>() / 2; }
 
+// Global accesses of the table and the decisions, which a caller may hand over
+// at any address (one instruction all the same).
+template <typename T>
+__device__ __forceinline__ T load_bytes(const uint8_t* p) {
+  T v;
+  __builtin_memcpy(&v, p, sizeof(T));
+  return v;
+}
+template <typename T>
+__device__ __forceinline__ void store_bytes(uint8_t* p, T v) {
+  __builtin_memcpy(p, &v, sizeof(T));
+}
+
 // E4M3 (fn) byte -> fp16, exact (labels are finite).
 __device__ __forceinline__ _Float16 e4m3_to_f16(uint32_t b) {
   const uint32_t s = (b >> 7) & 1, e = (b >> 3) & 15, m = b & 7;
@@ -194,7 +207,7 @@ __global__ __launch_bounds__(T, 4) void sqg_viterbi_kernel(const float* __restri
 #pragma unroll
     for (int k = 0; k < Q; ++k) {
       const uint32_t s = (uint32_t)(k << KR | o);
-      if constexpr (CB == 0) label[j][k] = pair_labels(*reinterpret_cast<const uint16_t*>(lut + s));
+      if constexpr (CB == 0) label[j][k] = pair_labels(load_bytes<uint16_t>(lut + s));
       else label[j][k] = procedural_pair<CB>(s * CM, s * CM + CM);
     }
   }
@@ -263,9 +276,9 @@ __global__ __launch_bounds__(T, 4) void sqg_viterbi_kernel(const float* __restri
     }
     if constexpr (keep) {
       uint8_t* at = dec + ri * RB + BYTES * tid;
-      if constexpr (NW == 2) *reinterpret_cast<u32x2_t*>(at) = u32x2_t{word[0], word[1]};
-      else if constexpr (BYTES == 4) *reinterpret_cast<uint32_t*>(at) = word[0];
-      else *reinterpret_cast<uint16_t*>(at) = (uint16_t)((word[0] >> 8 & 0xffu) | (word[0] >> 16 & 0xff00u));
+      if constexpr (NW == 2) store_bytes(at, u32x2_t{word[0], word[1]});
+      else if constexpr (BYTES == 4) store_bytes(at, word[0]);
+      else store_bytes(at, (uint16_t)((word[0] >> 8 & 0xffu) | (word[0] >> 16 & 0xff00u)));
     }
     __syncthreads();
   };
@@ -276,7 +289,7 @@ __global__ __launch_bounds__(T, 4) void sqg_viterbi_kernel(const float* __restri
     uint32_t half[NW];  // the halves of this parity, at bits 15 .. 0
 #pragma unroll
     for (int v = 0; v < NW; ++v)
-      half[v] = BYTES == 2 ? (uint32_t)at[h] << 8 : *reinterpret_cast<const uint16_t*>(at + 4 * v + 2 * h);
+      half[v] = BYTES == 2 ? (uint32_t)at[h] << 8 : load_bytes<uint16_t>(at + 4 * v + 2 * h);
     uint32_t k = 0;
 #pragma unroll
     for (int b = 0; b < K; ++b) k |= (half[NP * b / 16] >> (15 - NP * b % 16 - j) & 1u) << b;

@@ -14,6 +14,7 @@ import pytest
 import torch
 
 import oracle
+from kquant_amd import _native as N
 from kquant_amd import sqg_quantizer
 from kquant_amd.sqg_e4m3 import sqg_xor_cheb_t12_bytes
 
@@ -133,3 +134,22 @@ def test_workspace_is_the_calls_own(gpu):
     out = sqg_quantizer.quantize_tiles_sqg(x, lut, 2, 16)
     assert torch.cuda.max_memory_allocated(gpu) - before <= 8 << 20
     assert torch.cuda.memory_allocated(gpu) - before <= 4096 + sum(o.numel() * o.element_size() for o in out)
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4])
+def test_table_and_workspace_at_odd_addresses(gpu, bits):
+    """The C entry takes the table and the decisions at any address."""
+    x = _tiles(bits, 7)
+    lut_np = oracle.sqg_xor_cheb_t12_bytes(bits)
+    want_vals, want_states = oracle.sqg_quantize_tiles(x, lut_np, bits, 16)
+    t = torch.from_numpy(x).to(gpu)
+    lut = torch.empty(65537, dtype=torch.uint8, device=gpu)[1:]
+    lut.copy_(torch.from_numpy(lut_np))
+    need = int(N.library().kq_sqg_quantize_workspace_size(bits, len(x)))
+    ws = torch.empty(need + 1, dtype=torch.uint8, device=gpu)[1:]
+    assert lut.data_ptr() % 2 and ws.data_ptr() % 2
+    out, states = torch.empty_like(t), torch.empty(t.shape, dtype=torch.int16, device=gpu)
+    N.call("kq_sqg_quantize_tiles", N.ptr(t), len(x), N.ptr(lut), bits, 16, N.ptr(out), N.ptr(states), N.ptr(ws), need,
+           len(x), N.stream(gpu))
+    assert np.array_equal(states.cpu().numpy(), want_states)
+    assert np.array_equal(out.cpu().numpy(), want_vals)
