@@ -281,7 +281,9 @@ int kq_mx_linear_mm(int w_fmt, const void* a, int a_dtype, int64_t lda, const vo
  * the 128x128 upper tiles, which is what kq_syrk_finalize reads.  With
  * KQ_SYRK_OVERWRITE the tiles are written instead of accumulated (acc need
  * not be initialised).  bf16 rows use bf16 MFMA with exact products; fp16 /
- * fp32 rows and weights use a two-term bf16 split (16 significant bits). */
+ * fp32 rows and weights use a two-term bf16 split (16 significant bits).  A
+ * non-finite feature of a row makes its entries non-finite, Inf or NaN as the
+ * launch taken sums them, and no others. */
 int kq_syrk_accumulate(int in_dtype, const void* x, int64_t ld, int64_t n, int64_t k,
                        const float* weights, float* acc, int64_t ld_acc, uint32_t flags,
                        void* stream);

@@ -344,7 +344,7 @@ def test_split_launch_matches_plain_launch(gpu, n, k):
     lib = N.library()
     need = int(lib.kq_syrk_accumulate_workspace_size(N.DT_BF16, n, k, 0))
     assert need > 0, "the split launch should pay for this shape"
-    assert lib.kq_syrk_accumulate_workspace_size(N.DT_BF16, n, k, 1) == 0  # weighted rows: plain launch
+    assert lib.kq_syrk_accumulate_workspace_size(N.DT_BF16, n, k, 1) == 0  # weighted rows: no tail; sliced in a workspace of kq_syrk_sliced_workspace_size
     x = workloads.student_t4(n, k, seed=n + 3 * k, dtype=torch.bfloat16).to(gpu)
     ws = torch.empty(need, dtype=torch.uint8, device=gpu).fill_(0xFF)  # slots need no initialisation
     st = N.stream(gpu)
@@ -505,3 +505,80 @@ def test_short_groups(gpu, k, groups, most, dtype):
             ref = _f64_covariance(x[a:b], w[a:b])
             assert float((h[e].double() - ref).norm() / ref.norm()) <= TOL, e
             assert float(den[e]) == pytest.approx(float(w[a:b].double().sum()), rel=1e-12)
+
+
+@pytest.mark.parametrize("n,k,ld_acc", [(6000, 200, 264), (3000, 520, 520)])
+@pytest.mark.parametrize("dtype,weighted", [(torch.bfloat16, True), (torch.float16, True), (torch.float16, False),
+                                            (torch.float32, True), (torch.float32, False)])
+def test_sliced_rows_accumulate(gpu, n, k, ld_acc, dtype, weighted):
+    """kq_syrk_accumulate_ws in row slices without KQ_SYRK_OVERWRITE: onto a
+    prefilled accumulator of a wider stride, nothing written past column k or
+    below the upper tiles (256 wide for bf16 rows, else 128)."""
+    print(f"case sliced accumulate n={n} k={k} {dtype} weighted={weighted}", flush=True)
+    code = N.DTYPE_CODES[dtype]
+    need = int(N.library().kq_syrk_sliced_workspace_size(code, n, k, int(weighted)))
+    assert need > 0
+    x = workloads.student_t4(n, k, seed=n, dtype=dtype).to(gpu)
+    g = torch.Generator(device=gpu).manual_seed(k)
+    w = torch.rand(n, generator=g, device=gpu) + 0.1 if weighted else None
+    acc0 = torch.randn(k, ld_acc, generator=g, device=gpu) * 100.0
+    acc = acc0.clone()
+    ws = torch.empty(need, dtype=torch.uint8, device=gpu).fill_(0xFF)
+    N.call("kq_syrk_accumulate_ws", code, N.ptr(x), k, n, k, N.ptr(w), N.ptr(acc), ld_acc, 0, N.ptr(ws), need,
+           N.stream(gpu))
+    t = torch.arange(k, device=gpu) // (256 if dtype == torch.bfloat16 else 128)
+    upper = t[:, None] <= t[None, :]
+    xd = x.double()
+    want = acc0[:, :k].double() + xd.T @ (xd if w is None else xd * w.double()[:, None])
+    diff = (acc[:, :k].double() - want)[upper]
+    assert float(diff.norm() / want[upper].norm()) <= TOL
+    assert torch.equal(acc[:, :k][~upper], acc0[:, :k][~upper]) and torch.equal(acc[:, k:], acc0[:, k:])
+
+
+def test_grouped_covariance_stays_in_a_too_small_plan(gpu):
+    """A row bound below the list's length: more slices are asked for than
+    there are slots, and nothing past the workspace (or the outputs) is
+    written; the denominators come from the offsets alone."""
+    k, sizes, bound = 256, [3000, 2000, 10], 2000
+    n, groups, guard = sum(sizes), len(sizes), 4096
+    need = int(N.library().kq_grouped_covariance_workspace_size(N.DT_BF16, bound, k, groups))
+    assert need > groups * k * k * 4  # a sliced plan
+    x = workloads.student_t4(n, k, seed=3).to(gpu)
+    w = (torch.rand(n, generator=torch.Generator().manual_seed(3)) + 0.1).to(gpu)
+    offsets = torch.tensor([0, 3000, 5000, 5010], device=gpu)
+    ws = torch.full((need + guard,), 0x5A, dtype=torch.uint8, device=gpu)
+    out = torch.full((groups * k * k + 1024,), -7.0, device=gpu)
+    den = torch.empty(groups, dtype=torch.float64, device=gpu)
+    N.call("kq_grouped_covariance", N.DT_BF16, N.ptr(x), k, N.ptr(offsets), groups, None, N.ptr(w), bound, k,
+           N.ptr(out), N.ptr(den), 0, N.ptr(ws), need, N.stream(gpu))
+    assert bool((ws[need:] == 0x5A).all()) and bool((out[groups * k * k:] == -7.0).all())
+    want = torch.stack([w[a:b].double().sum() for a, b in ((0, 3000), (3000, 5000), (5000, 5010))])
+    assert torch.allclose(den, want, rtol=1e-12)
+
+
+@pytest.mark.parametrize("n", [19, 3001])
+def test_non_finite_rows_stay_in_their_features(gpu, n):
+    """Weighted bf16 rows with an Inf in the last row (the one that the direct
+    loads repeat past the end) and a NaN in another: the entries of those two
+    features are non-finite and all others those of the finite rest, in one
+    launch, in slices and as a group."""
+    k = 64
+    x = workloads.student_t4(n, k, seed=n, dtype=torch.bfloat16).to(gpu)
+    w = (torch.rand(n, generator=torch.Generator().manual_seed(n)) + 0.1).to(gpu)
+    ref = x.double().T @ (x.double() * w.double()[:, None])
+    x[-1, 5], x[10, 9] = float("inf"), float("nan")
+    hit = torch.zeros(k, dtype=torch.bool, device=gpu)
+    hit[[5, 9]] = True
+    hit = hit[:, None] | hit[None, :]
+    st = N.stream(gpu)
+    need = int(N.library().kq_syrk_sliced_workspace_size(N.DT_BF16, n, k, 1))
+    ws = torch.empty(max(need, 256), dtype=torch.uint8, device=gpu)
+    offsets = torch.tensor([0, n], device=gpu)
+    accs = [torch.zeros(k, k, device=gpu) for _ in range(3)]
+    N.call("kq_syrk_accumulate", N.DT_BF16, N.ptr(x), k, n, k, N.ptr(w), N.ptr(accs[0]), k, N.SYRK_OVERWRITE, st)
+    N.call("kq_syrk_accumulate_ws", N.DT_BF16, N.ptr(x), k, n, k, N.ptr(w), N.ptr(accs[1]), k, N.SYRK_OVERWRITE,
+           N.ptr(ws), need, st)
+    N.call("kq_syrk_grouped", N.DT_BF16, N.ptr(x), k, N.ptr(offsets), 1, None, N.ptr(w), k, N.ptr(accs[2]), 0, st)
+    for acc in accs:
+        assert not torch.isfinite(acc[hit]).any() and torch.isfinite(acc[~hit]).all()
+        assert float((acc.double() - ref)[~hit].norm() / ref[~hit].norm()) <= TOL

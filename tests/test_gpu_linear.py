@@ -423,3 +423,24 @@ def test_few_rows_scale_and_code_nans(gpu):
     assert torch.equal(torch.isnan(c), nan)
     ref = (_mx_values(aq, a_s) @ _mx_values(wq, w_s).T)
     assert float(((c.double() - ref)[~nan] / ref[~nan]).abs().max()) <= 3e-5
+
+
+@pytest.mark.parametrize("k", [128, 192, 320])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("fmt", ["mxfp8", "mxfp4"])
+def test_few_rows_non_finite(gpu, fmt, dtype, k):
+    """Inf and NaN stay in their rows: the last row (read again for the block's
+    missing ones) and the columns a half window reads twice included."""
+    g = torch.Generator().manual_seed(k)
+    m, n = 21, 70
+    w = (torch.randn(n, k, generator=g) * 0.02).to(torch.bfloat16).to(gpu)
+    x = torch.randn(m, k, generator=g).to(dtype)
+    q, s, wd = _quantized(fmt, w)
+    ref = x.double().numpy() @ wd.astype(np.float64).T
+    x[2, 64], x[9, k - 1], x[-1, 3] = float("nan"), float("inf"), float("-inf")
+    hit = np.zeros(m, dtype=bool)
+    hit[[2, 9, m - 1]] = True
+    fn = linear.mxfp8_linear if fmt == "mxfp8" else linear.mxfp4_linear
+    c = fn(x.to(gpu), q, s, out_dtype=torch.float32).cpu().numpy()
+    assert not np.isfinite(c[hit]).any() and np.isfinite(c[~hit]).all()
+    assert _max_rel(ref[~hit], c[~hit]) <= 1e-5
