@@ -248,8 +248,11 @@ int kq_mx_linear_ws(int w_fmt, const void* a, int64_t lda, const void* w_q, cons
  * 256-byte aligned, uninitialised) takes both scale planes transposed to
  * [k/128][rows] dwords, the layout the kernel loads a 128-k stage's scales
  * from, and the planes of a split over K as in kq_mx_linear_ws (the scale
- * planes alone are enough: it then runs unsplit).  The matrix cores sum the 64 products of a step with a few fp32 ulps
- * of error (measured ~1e-5 relative). */
+ * planes alone are enough: it then runs unsplit).  The matrix cores sum the
+ * 64 products of a step with a few fp32 ulps of error (measured ~1e-5
+ * relative); few rows multiply in one pass over the weights instead, exact
+ * products summed in fp32, the scales added as exponents where an operand
+ * would leave fp32's range. */
 int64_t kq_mx_linear_mx_workspace_size(int64_t m, int64_t n, int64_t k);
 int kq_mx_linear_mx(int a_fmt, const void* a_q, const uint8_t* a_scale, int64_t lda, int w_fmt,
                     const void* w_q, const uint8_t* w_scale, int64_t m, int64_t n, int64_t k,

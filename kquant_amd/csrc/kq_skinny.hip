@@ -27,7 +27,10 @@ static hipError_t launch(const SkinnyArgs& s, hipStream_t st) {
 // K = 7168 E4M3, one row, cold: 24 us; R = 2 / 4: 27 / 30); with 17 rows and
 // more the activations outweigh the weights unless four blocks share a read
 // of them (32 rows: 42.6 us against 52; 64 rows: 57 against 95), which pays
-// while N / 64 workgroups still cover half the CUs.
+// while N / 64 workgroups still cover half the CUs.  Half windows keep R = 1
+// past 16 rows: fp32 rows, N = 12288, K = 2112, 17 / 32 rows 44 / 58 us with E4M3 weights
+// (171 / 172 in whole tiles), 53 at 17 with E2M1 (16 registers spill; 160), and
+// the tiles' split, 46, at 32.
 template <int FMT, int AT, int OUT, bool HALF>
 static hipError_t launch_rows(const SkinnyArgs& s, hipStream_t st) {
   const bool wide = s.n >= 64 * 128;
